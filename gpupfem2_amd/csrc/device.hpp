@@ -8,10 +8,34 @@ namespace pfem {
 constexpr int kBlock = 256;          // 4 wavefronts of 64 lanes
 constexpr int kWaves = kBlock / 64;
 
+// The value of lane i + OFF in lane i < OFF, for the steps of a tree sum whose result is lane 0's: halves and
+// rows of 16 are swapped, and within a row the shift is part of the move (DPP), all in registers. A
+// shuffle through LDS (ds_bpermute) waits about 120 cycles per step.
+template <int OFF>
+__device__ __forceinline__ unsigned lane_down(unsigned v)
+{
+    if constexpr (OFF == 32) return __builtin_amdgcn_permlane32_swap(v, v, false, false)[1];
+    else if constexpr (OFF == 16) return __builtin_amdgcn_permlane16_swap(v, v, false, false)[1];
+    else return __builtin_amdgcn_update_dpp(0, v, 0x100 + OFF, 0xF, 0xF, true);   // row_shl:OFF
+}
+
+template <int OFF>
+__device__ __forceinline__ double lane_down(double v)
+{
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned hi = lane_down<OFF>((unsigned)(u >> 32)), lo = lane_down<OFF>((unsigned)u);
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
+// Sum over the wave, valid in lane 0: lanes i and i + 32 first, then i + 16, 8, 4, 2, 1
 __device__ __forceinline__ double wave_sum(double v)
 {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+    v += lane_down<32>(v);
+    v += lane_down<16>(v);
+    v += lane_down<8>(v);
+    v += lane_down<4>(v);
+    v += lane_down<2>(v);
+    v += lane_down<1>(v);
     return v;
 }
 

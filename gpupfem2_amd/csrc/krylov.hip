@@ -13,6 +13,7 @@
 
 #include "device.hpp"
 #include "internal.hpp"
+#include "resident.hpp"
 #include "solver.hpp"
 #include "spmv.hpp"
 #include "sync.hpp"
@@ -620,6 +621,7 @@ __global__ void k_perm_scatter(int n, const int* __restrict__ perm, const double
 // ------------------------------------------------------------------ host drivers
 template <typename T>
 struct KArgs {
+    std::shared_ptr<Pattern> pat;   // P's owner (plans that outlive a solve keep it)
     const Pattern* P;
     const T* val;
     const T* invd;       // Jacobi diagonal (null otherwise)
@@ -641,6 +643,29 @@ static void papply(Context* c, const KArgs<T>& A, T* z, const T* r)
     precond_apply_t<T>(c, A.pc, z, r, A.pc_fp32, ApplyOpts<T>{nullptr, 0, A.factor_order});
 }
 
+// The whole solve as one launch (resident.hip), with the bits of the launch-per-kernel iterations below.
+// Systems of up to 262144 rows whose matrix rows hold at most 16 entries fit (2D meshes), and it is the
+// quicker one at every size that fits: us per iteration, launch-per-kernel and here, at 1k, 4k, 17k, 40k,
+// 131k and 251k rows: 12.6, 14.5, 14.6, 14.5, 16.2, 19.3 against 1.8, 3.7, 4.4, 5.5, 6.0, 9.0.
+template <typename T>
+static bool cg_resident(Context* c, pfem_solver_t* s, const KArgs<T>& A, CgState* hst)
+{
+    if (!s->resident) s->resident.reset(new ResidentWork());
+    ResidentWork& w = *s->resident;
+    if (!w.plan(c, A.pat, {0, A.P->n}, true)) return false;
+    if (!w.solve<T>(c, A.val, A.invd, A.b, A.x, A.x_zero, A.tol, A.tol_mode, A.maxit, 0.0,
+                    A.pc ? A.pc->spin_limit : 1 << 16))
+        return false;
+    const ResOut& o = w.h_out[0];
+    *hst = CgState{};
+    hst->it = o.it;
+    hst->converged = o.converged;
+    hst->nan = o.nan;
+    hst->res = o.res;
+    hst->done = 1;
+    return true;
+}
+
 template <typename T>
 static void cg_run(Context* c, pfem_solver_t* s, const KArgs<T>& A, CgState* st, CgState* hst)
 {
@@ -648,6 +673,7 @@ static void cg_run(Context* c, pfem_solver_t* s, const KArgs<T>& A, CgState* st,
     const int n = P.n;
     const unsigned g = vec_grid(n);
     const bool jac = A.kind == PFEM_PRECOND_JACOBI, none = A.kind == PFEM_PRECOND_NONE;
+    if ((jac || none) && cg_resident<T>(c, s, A, hst)) return;
     // x/r update fused into the forward sweep: multicolour IC0/ILU0, single-pass sweeps, factor ordering
     // (a blocked factor has the fused forms in their tagged form only)
     const bool fused = A.factor_order && A.pc && A.pc->sweep &&
@@ -1056,6 +1082,7 @@ static KArgs<double> args64(pfem_solver_t* s, pfem_csr_t* a, double* x, const do
     KArgs<double> A{};
     A.pc_fp32 = s->precision == PFEM_PRECISION_MIXED_PRECOND && s->pc &&
                 (s->pc->kind == PFEM_PRECOND_IC0 || s->pc->kind == PFEM_PRECOND_ILU0);
+    A.pat = a->pat;
     A.P = a->pat.get();
     A.val = a->val.p;
     A.kind = s->pc ? s->pc->kind : PFEM_PRECOND_NONE;
@@ -1093,6 +1120,7 @@ static KArgs<double> args_factor_order(Context* c, pfem_solver_t* s, double* x, 
                        (const double*)x, s->xp.p);
     PFEM_HIP(hipGetLastError());
     KArgs<double> A{};
+    A.pat = pc->fpat;
     A.P = pc->fpat.get();
     A.val = pc->aval.p;
     A.kind = pc->kind;
@@ -1186,6 +1214,7 @@ struct MixedSys {
         init.first = 1;
         PFEM_HIP(hipMemcpyAsync(ist, &init, sizeof(IrState), hipMemcpyHostToDevice, c->stream));
         const int kind = s->pc ? s->pc->kind : PFEM_PRECOND_NONE;
+        A.pat = a->pat;
         A.P = &P;
         A.val = a->val32.p;
         A.kind = kind;

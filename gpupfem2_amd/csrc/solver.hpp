@@ -66,6 +66,10 @@ struct BatchWork;   // batched-systems PCG work space (batched.hip)
 struct BatchWorkDeleter {
     void operator()(BatchWork* w) const;
 };
+struct ResidentWork;   // single-launch PCG work space (resident.hip)
+struct ResidentWorkDeleter {
+    void operator()(ResidentWork* w) const;
+};
 
 constexpr int kMaxRestart = 1024;   // largest GMRES cycle (the reference's maxIterations default is 1000)
 constexpr int kVecGrid = 1024;      // grid of the vector kernels (grid-stride loops)
@@ -275,6 +279,7 @@ struct pfem_solver_t {
     hipEvent_t ev[2] = {nullptr, nullptr};   // pipelined polls of the device state
     std::unique_ptr<pfem::MultiWork, pfem::MultiWorkDeleter> multi;   // pfem_solver_solve_multi
     std::unique_ptr<pfem::BatchWork, pfem::BatchWorkDeleter> batch;   // pfem_solver_solve_batched
+    std::unique_ptr<pfem::ResidentWork, pfem::ResidentWorkDeleter> resident;   // single-launch Jacobi PCG
     std::vector<int> batch_tiling;   // {row bound, tile rows, tile non-zeros} per size bucket (empty: defaults)
     pfem::DevArray<pfem::CgState> cg;
     pfem::DevArray<pfem::GmState> gm;

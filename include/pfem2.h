@@ -212,7 +212,9 @@ int pfem_precond_download(pfem_precond pc, double* factor, int* n_levels, int* p
 int pfem_precond_set_sweep(pfem_precond pc, int single_pass);
 /* Polls a single-pass wait makes before it is declared failed (no counterpart in the reference; default
  * 65536, about 0.1 s). A failed wait does not hang or fault: the launch completes, and the solve or apply
- * reports PFEM_ENUMERIC and re-arms the sweep buffers. 0 fails every wait that is not satisfied at once. */
+ * reports PFEM_ENUMERIC and re-arms the sweep buffers. 0 fails every wait that is not satisfied at once. With a
+ * Jacobi preconditioner or none it scales the waits of the single-launch PCG, which falls back to one
+ * launch per kernel, with the same results, when a wait fails. */
 int pfem_precond_set_spin_limit(pfem_precond pc, int polls);
 /* Storage of the reduced-precision factor copy that PFEM_PRECISION_MIXED_PRECOND applies to FP64 vectors
  * (no counterpart in the reference, whose factor is FP64): 32 (default) or 16 bits per value (IEEE half;
@@ -301,7 +303,8 @@ int pfem_solver_set_batch_tiles(pfem_solver s, int nbuckets, const int* max_rows
  * [h_sys_rows[k], h_sys_rows[k+1]) (h_sys_rows: nsys + 1 host ints from 0 to n; checked). Each system runs
  * the solver's PCG recurrence and stopping test with its own scalars and stops on its own; all systems
  * share every launch. Jacobi preconditioner or none; PFEM_PRECISION_FP64 or PFEM_PRECISION_MIXED (reliable
- * updates per system, as pfem_solver_solve_multi). d_x is the initial guess (FP64 path) and the solution.
+ * updates per system, as pfem_solver_solve_multi; systems that a single launch holds in registers iterate in
+ * FP64 there as well, which costs them no bandwidth). d_x is the initial guess (FP64 path) and the solution.
  * stats: nsys entries (or NULL); h_time_ms (or NULL): per-system time to solution on the device clock,
  * from the start of the call's first Krylov or refinement pass to the pass where the system stopped. */
 int pfem_solver_solve_batched(pfem_solver s, pfem_csr a, int nsys, const int* h_sys_rows, double* d_x,

@@ -1,0 +1,94 @@
+"""GPU: the single-launch (resident) PCG against the launch-per-kernel PCG, which a zero spin limit forces
+(every wait that is not satisfied at once fails, and the solve falls back): the same bits of the solution and the
+same iteration count, since both add the same partials in the same order."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def poisson(ctx, nx, ny, seed, jitter=0.2):
+    from gpupfem2_amd import capi, meshgen
+    xy, tri = meshgen.rectangle(0.0, 2.0, 0.0, 1.0, nx, ny, jitter=jitter, seed=seed)
+    m = capi.Mesh2D(ctx, xy, tri, fill_neighbors=False)
+    a = capi.CSR(ctx, mesh=m)
+    n = xy.shape[0]
+    scratch = ctx.zeros(n)
+    capi.assemble_poisson2d(m, a, scratch, coeff=1.0, rhs_kind=2, rhs_param=0.0)
+    left = np.nonzero(xy[:, 0] < 1e-9)[0].astype(np.int32)
+    capi.Dirichlet(ctx, n, left, np.zeros(left.size)).apply(a, scratch)
+    b = np.random.default_rng(seed).standard_normal(n)
+    b[left] = 0.0
+    return m, a, b
+
+
+# rows: one workgroup, 1024 and one more (a second workgroup with one row), one tile short of and past a
+# workgroup, many workgroups, more than 256 tiles (several slots per lane)
+@pytest.mark.parametrize("nx,ny", [(1, 1), (15, 15), (31, 31), (40, 24), (63, 19), (100, 50), (400, 100), (361, 361)])
+@pytest.mark.parametrize("kind,precision", [(1, 0), (0, 0), (1, 1)])
+def test_resident_same_bits(ctx, nx, ny, kind, precision):
+    from gpupfem2_amd import capi
+    print("resident", nx, ny, kind, precision, flush=True)
+    m, a, b = poisson(ctx, nx, ny, seed=nx + ny)
+    n = a.n
+    start = np.random.default_rng(5).standard_normal(n) * 1e-3
+    out = []
+    for limit in (1 << 16, 0):
+        pc = capi.Preconditioner(a, kind)
+        pc.set_spin_limit(limit)
+        s = capi.Solver(a, capi.SOLVER_CG, 1e-11, 8000, 0, capi.TOL_RELATIVE, pc)
+        if precision:
+            s.set_precision(precision, 1e-5, 30)
+        x = ctx.to_device(start)
+        d = ctx.to_device(b)
+        st = s.solve(a, x, d)
+        assert st.converged and not st.nan_detected
+        out.append((x.download(), st.iterations, st.final_residual, st.refinements))
+    assert out[0][1:] == out[1][1:]
+    assert np.array_equal(out[0][0], out[1][0])
+
+
+def test_resident_iteration_limit_and_zero(ctx):
+    """stopped by the iteration limit: the iterate of that many steps; a zero right-hand side stops at once"""
+    from gpupfem2_amd import capi
+    m, a, b = poisson(ctx, 60, 60, seed=2)
+    out = []
+    for limit in (1 << 16, 0):
+        pc = capi.Preconditioner(a, 1)
+        pc.set_spin_limit(limit)
+        s = capi.Solver(a, capi.SOLVER_CG, 1e-11, 17, 0, capi.TOL_RELATIVE, pc)
+        x = ctx.zeros(a.n)
+        st = s.solve(a, x, ctx.to_device(b))
+        assert not st.converged and st.iterations == 17
+        out.append(x.download())
+        st = s.solve(a, ctx.zeros(a.n), ctx.zeros(a.n))
+        assert st.iterations <= 17
+    assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_resident_batch(ctx, precision):
+    """systems of one row tile to many workgroups: in FP64 the bits of the launch-per-kernel path; in mixed
+    precision both solve to the tolerance with the true residual in the stopping test"""
+    from gpupfem2_amd import capi, cases
+    case = cases.batched_poisson_case(nmesh=14, tmin=60, tmax=30000, seed=8)
+    mesh, a, b = cases.build_batched_poisson(ctx, case)
+    rows, n = case["sys_rows"], case["sys_rows"][-1]
+    out = []
+    for limit in (1 << 16, 0):
+        pc = capi.Preconditioner(a, 1)
+        pc.set_spin_limit(limit)
+        s = capi.Solver(a, capi.SOLVER_CG, 1e-11, 20000, 0, capi.TOL_RELATIVE, pc)
+        if precision:
+            s.set_precision(precision, 1e-5, 30)
+        x = ctx.zeros(n)
+        st, ms = s.solve_batched(a, rows, x, b)
+        assert all(q.converged and not q.nan_detected for q in st)
+        assert (ms > 0).all()
+        out.append((x.download(), [q.iterations for q in st], [q.refinements for q in st]))
+    if precision:
+        assert all(r >= 1 for r in out[0][2])
+        assert np.linalg.norm(out[0][0] - out[1][0]) < 1e-8 * np.linalg.norm(out[1][0])
+    else:
+        assert out[0][1] == out[1][1]
+        assert np.array_equal(out[0][0], out[1][0])
