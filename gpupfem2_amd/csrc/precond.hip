@@ -1461,6 +1461,7 @@ static void build_factor_structure(Context* c, pfem_precond_t* pc)
         }
         slice(ftiles, 2, pc->sl_all, pc->asl_val);
     }
+    if (pc->ordering == PFEM_ORDER_NATURAL) pc->band = band_build(c, F, lev, ulev, pc->nlevels);
     pc->fac.alloc(F.nnz);
     pc->tmp.alloc(n);
     pc->sy.alloc(n);
@@ -1536,6 +1537,7 @@ void precond_initialize(Context* c, pfem_precond_t* pc, pfem_csr_t* a)
                                pc->sell_u.p);
         }
     }
+    if (pc->band) band_refresh(c, *pc->band, F, pc->fac.p, pc->fac32.p);
     if (pc->split16.p) {
         // the scale from the largest factor entry, then c L in 16 bits
         const long nl = (long)pc->sell_l.n, nu = (long)pc->sell_u.n;
@@ -1757,6 +1759,9 @@ static void sweeps(Context* c, pfem_precond_t* pc, const TV* src, TV* out, const
             else hipLaunchKernelGGL((k_sweep_lower<TV, TS, TF, true, kRange, false>), gl, bl, 0, c->stream, lo);
         }
         hipLaunchKernelGGL((k_sweep_upper<TV, TS, TF, kRange>), gu, bl, 0, c->stream, up);
+    } else if (pc->band) {
+        if constexpr (sizeof(TS) != 2)
+            band_sweeps<TV, TS, TF>(c, *pc->band, F.n, !ic, src, out, sy, sw, part, o.done, pc->sweep_err.p, pc->spin_limit);
     } else {
         PFEM_REQUIRE(!o.tagged, "tagged sweeps need the sliced layout");
         lo.rows = pc->lrows.p;
@@ -1815,7 +1820,9 @@ int precond_apply_t(Context* c, pfem_precond_t* pc, TV* z, const TV* r, bool fp3
     }
     PFEM_HIP(hipGetLastError());
     // partials written: one per backward launch workgroup
-    const int nbw = (pc->contiguous && pc->sell) || (pc->blocked && opt.tagged) ? pc->nuslices : pc->nuchunks;
+    const int nbw = (pc->contiguous && pc->sell) || (pc->blocked && opt.tagged) ? pc->nuslices
+                    : pc->band                                                  ? pc->band->bands
+                                                                                : pc->nuchunks;
     return part && (pc->kind == PFEM_PRECOND_IC0 || pc->kind == PFEM_PRECOND_ILU0) ? nbw : 0;
 }
 

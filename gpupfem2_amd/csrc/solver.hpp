@@ -4,6 +4,7 @@
 #include <cmath>
 #include <cstddef>
 
+#include "band.hpp"
 #include "internal.hpp"
 
 namespace pfem {
@@ -248,6 +249,8 @@ struct pfem_precond_t {
     // take the dependencies outside the block, a dense triangle per block the ones inside); the per-level
     // tables (lrows, lchunks, ...) hold the longest-path levels of the same factor
     bool blocked = false;
+    // natural ordering with many small levels: the sweeps' other form (band.hip)
+    std::unique_ptr<pfem::BandSweeps> band;
 };
 
 struct pfem_solver_t {
