@@ -133,6 +133,7 @@ struct pfem_mesh2d_t {
     std::vector<int> h_tri;        // host cells (all parsed cells)
     std::vector<int> h_edge_ids;
     pfem::DevArray<double> xy, area, invJ;
+    pfem::DevArray<double2> v3;    // third vertex of every cell (the origin of its local coordinates)
     pfem::DevArray<int> tri, edge_ids, nbr_off, nbr_idx;
     long n_nbr = 0;
     std::shared_ptr<pfem::Pattern> pat;

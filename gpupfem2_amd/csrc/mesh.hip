@@ -192,7 +192,7 @@ static void build_incidence(Context* ctx, int nv, int nt, int nper, const std::v
 // kCalculateCellArea (src/mesh_2d.cu:10-19) and kCalculateInvJacobi (:21-34) with
 // Matrix2x2::inverse (src/common/cuda_math.cuh:124-141); invJ row-major.
 __global__ void k_geometry2d(int nt, const double* __restrict__ xy, const int* __restrict__ tri,
-                             double* __restrict__ area, double* __restrict__ invJ)
+                             double* __restrict__ area, double* __restrict__ invJ, double2* __restrict__ v3)
 {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= nt) return;
@@ -210,6 +210,7 @@ __global__ void k_geometry2d(int nt, const double* __restrict__ xy, const int* _
     o.z = -j10 * inv;
     o.w = j00 * inv;
     reinterpret_cast<double4*>(invJ)[c] = o;
+    v3[c] = make_double2(dx, dy);
 }
 
 // kCalculateCellVolume / kCalculateInvJacobi (src/mesh_3d.cu:12-35), GenericMatrix3x3::inverse
@@ -382,9 +383,10 @@ static pfem_mesh2d_t* mesh2d_build(Context* c, int nv, std::vector<double>&& xy,
     upload(c, m->edge_ids, m->h_edge_ids);
     m->area.alloc(m->nt);
     m->invJ.alloc(4 * (size_t)m->nt);
+    m->v3.alloc(m->nt);
     if (m->nt > 0)
         hipLaunchKernelGGL(k_geometry2d, dim3(blocks_for(m->nt)), dim3(kBlock), 0, c->stream, m->nt, m->xy.p,
-                           m->tri.p, m->area.p, m->invJ.p);
+                           m->tri.p, m->area.p, m->invJ.p, m->v3.p);
     PFEM_HIP(hipGetLastError());
     if (fill_neighbors) {
         std::vector<int> off, idx;
