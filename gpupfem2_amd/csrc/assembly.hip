@@ -8,6 +8,13 @@
 // precomputed slot map. Every row is written by exactly one lane, so there are no races, the result
 // is deterministic, and each entry sums its element contributions in ascending element order -- the
 // order of a sequential element loop.
+//
+// The chain of loads per incidence bounds these kernels. So a workgroup sums its 256 rows' entries in LDS and
+// writes them once, coalesced (adding them in memory waits for a load of the entry at every incidence); the
+// cell of the next incidence is loaded during the current one; a row's places are one byte each; the matrix
+// kernels with a three-point rule have its loops unrolled and its one weight folded; and neighbouring tiles run
+// on one XCD. 1.01M rows, 2.0M triangles: prediction 535 -> 169 us, pressure 332 -> 97, correction 337 -> 104
+// (without the XCD bands 174, 98 and 118; prediction at two wavefronts a SIMD 187, at four 213, at three 169).
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -15,6 +22,7 @@
 
 #include "device.hpp"
 #include "internal.hpp"
+#include "spmv.hpp"
 #include "solver.hpp"
 
 namespace pfem {
@@ -174,70 +182,173 @@ struct Pfem2Prm {
     double nrm[8][2];
 };
 
+// x_i of three values, i per lane
+__device__ __forceinline__ double pick(int i, double x0, double x1, double x2) { return i == 0 ? x0 : (i == 1 ? x1 : x2); }
+
+// The rows of a workgroup and the entries they sum, NM matrices on one pattern: in LDS, or (more than CAP
+// entries in the 256 rows) in the matrices themselves.
+template <int NM, int CAP>
+struct RowTile {
+    double (&acc)[NM][CAP];
+    double* const (&val)[NM];
+    int r, k0, nk, row;   // this lane's row and its first entry
+    bool on, lds;
+
+    __device__ __forceinline__ RowTile(double (&a)[NM][CAP], double* const (&v)[NM], int nv, const int* __restrict__ rowptr)
+        : acc(a), val(v)
+    {
+        const int r0 = xcd_band_tile() * kBlock;   // neighbouring tiles on one XCD: they share vertices and cells
+        r = r0 + (int)threadIdx.x;
+        on = r < nv;
+        k0 = rowptr[r0];
+        nk = rowptr[min(r0 + kBlock, nv)] - k0;
+        row = on ? rowptr[r] : 0;
+        lds = nk <= CAP;
+        for (int k = threadIdx.x; k < nk; k += kBlock)
+#pragma unroll
+            for (int m = 0; m < NM; ++m) (lds ? acc[m][k] : val[m][k0 + k]) = 0.0;
+        __syncthreads();
+    }
+    __device__ __forceinline__ void add(int m, int at, double x)
+    {
+        if (lds) acc[m][at - k0] += x;
+        else val[m][at] += x;
+    }
+    __device__ __forceinline__ void finish()
+    {
+        __syncthreads();
+        if (!lds) return;
+        for (int k = threadIdx.x; k < nk; k += kBlock)
+#pragma unroll
+            for (int m = 0; m < NM; ++m) val[m][k0 + k] = acc[m][k];
+    }
+};
+constexpr int kTile2d = 2048, kTile3d = 4096;
+
+// A lane's incidences in order, the cell of the next one loaded during the current one
+struct Incidences {
+    const int *code_, *tri_;
+    int e, end;   // of the current incidence
+    int code, v[3], code1, v1[3], code2;
+    __device__ __forceinline__ Incidences(bool on, int r, const int* __restrict__ off, const int* __restrict__ code0,
+                                          const int* __restrict__ tri)
+        : code_(code0), tri_(tri)
+    {
+        e = (on ? off[r] : 0) - 1;
+        end = on ? off[r + 1] : 0;
+        if (e + 1 < end) {
+            code1 = code_[e + 1];
+            code2 = code_[min(e + 2, end - 1)];
+            cell(code1, v1);
+        }
+    }
+    __device__ __forceinline__ void cell(int c, int (&w)[3])
+    {
+        const int* t = tri_ + 3 * (size_t)(c >> 2);
+        w[0] = t[0]; w[1] = t[1]; w[2] = t[2];
+    }
+    __device__ __forceinline__ bool next()
+    {
+        if (++e >= end) return false;
+        code = code1;
+        v[0] = v1[0]; v[1] = v1[1]; v[2] = v1[2];
+        code1 = code2;
+        cell(code1, v1);
+        code2 = code_[min(e + 2, end - 1)];
+        return true;
+    }
+};
+
+// The CSR slot of (row, vertex j of the incidence's cell)
+struct SlotMap {
+    const uint32_t* rel;
+    const int* slots;
+};
+template <int N>
+__device__ __forceinline__ void incidence_slots(const SlotMap& m, int e, int row, int (&at)[N])
+{
+    if (m.rel) {
+        const uint32_t x = m.rel[e];
+#pragma unroll
+        for (int j = 0; j < N; ++j) at[j] = row + (int)((x >> (8 * j)) & 255u);
+    } else {
+#pragma unroll
+        for (int j = 0; j < N; ++j) at[j] = m.slots[N * (size_t)e + j];
+    }
+}
+
 // ------------------------------------------------------------------ Poisson 2D (cases/Poisson2D/main.cu:28-68)
+template <int NQ>
 __global__ __launch_bounds__(kBlock) void k_asm_poisson2d(int nv, const int* __restrict__ inc_off,
-                                                          const int* __restrict__ inc_code,
-                                                          const int* __restrict__ inc_slots,
+                                                          const int* __restrict__ inc_code, SlotMap map,
                                                           const double* __restrict__ xy, const int* __restrict__ tri,
                                                           const double* __restrict__ area,
                                                           const double4* __restrict__ invJ,
-                                                          const int* __restrict__ rowptr, double* __restrict__ val,
+                                                          const int* __restrict__ rowptr, double* val,
                                                           double* __restrict__ rhs, double coeff, int rhs_kind,
                                                           double rhs_param, Quad2 q)
 {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nv) return;
-    for (int k = rowptr[r]; k < rowptr[r + 1]; ++k) val[k] = 0.0;
+    __shared__ double acc[1][kTile2d];
+    double* const vals[1] = {val};
+    RowTile<1, kTile2d> T(acc, vals, nv, rowptr);
+    const int nq = NQ ? NQ : q.n;
     const double PI = 3.14159265358979323846;
     double rr = 0.0;
-    for (int e = inc_off[r]; e < inc_off[r + 1]; ++e) {
-        const int code = inc_code[e];
-        const int c = code >> 2, li = code & 3;
-        const int v0 = tri[3 * c], v1 = tri[3 * c + 1], v2 = tri[3 * c + 2];
+    Incidences in(T.on, T.r, inc_off, inc_code, tri);
+    while (in.next()) {
+        const int c = in.code >> 2, li = in.code & 3;
+        const int v0 = in.v[0], v1 = in.v[1], v2 = in.v[2];
         const double4 J = invJ[c];
+        const double ar = area[c];
+        int s[3];
+        incidence_slots<3>(map, in.e, T.row, s);
+        const double x0 = xy[2 * v0], x1 = xy[2 * v1], x2 = xy[2 * v2];
+        const double y0 = xy[2 * v0 + 1], y1 = xy[2 * v1 + 1], y2 = xy[2 * v2 + 1];
         double M[3] = {0.0, 0.0, 0.0};
         double R = 0.0;
-        for (int k = 0; k < q.n; ++k) {
+#pragma unroll NQ ? NQ : 1
+        for (int k = 0; k < nq; ++k) {
             const double L0 = q.l[k][0], L1 = q.l[k][1], L2 = q.l[k][2];
-            const double qx = L0 * xy[2 * v0] + L1 * xy[2 * v1] + L2 * xy[2 * v2];
-            const double qy = L0 * xy[2 * v0 + 1] + L1 * xy[2 * v1 + 1] + L2 * xy[2 * v2 + 1];
+            const double qx = L0 * x0 + L1 * x1 + L2 * x2;
+            const double qy = L0 * y0 + L1 * y1 + L2 * y2;
+#pragma unroll
             for (int j = 0; j < 3; ++j) {
                 const int a = li < j ? li : j, b = li < j ? j : li;   // SymmetricMatrix3x3 visits (min, max)
                 const double2 ga = grad2(J, a), gb = grad2(J, b);
-                const double aux = coeff * (ga.x * gb.x + ga.y * gb.y) * q.w[k];
+                const double aux = coeff * (ga.x * gb.x + ga.y * gb.y) * q.w[NQ ? 0 : k];
                 M[j] += aux;
             }
             double f;
             if (rhs_kind == 0) f = exp(-(qx * qx + 10 * qy * qy));
             else if (rhs_kind == 1) f = rhs_param * sin(PI * qx) * sin(PI * qy);
             else f = rhs_param;
-            R += f * q.l[k][li] * q.w[k];
+            R += f * pick(li, L0, L1, L2) * q.w[NQ ? 0 : k];
         }
-        const double ar = area[c];
-        const int* s = inc_slots + 3 * (size_t)e;
-        for (int j = 0; j < 3; ++j) val[s[j]] += M[j] * ar;
+#pragma unroll
+        for (int j = 0; j < 3; ++j) T.add(0, s[j], M[j] * ar);
         rr += R * ar;
     }
-    rhs[r] = rr;
+    if (T.on) rhs[T.r] = rr;
+    T.finish();
 }
 
 // ------------------------------------------------------------------ Poisson 3D (cases/Poisson3D/main.cu:26-67)
 __global__ __launch_bounds__(kBlock) void k_asm_poisson3d(int nv, const int* __restrict__ inc_off,
-                                                          const int* __restrict__ inc_code,
-                                                          const int* __restrict__ inc_slots,
+                                                          const int* __restrict__ inc_code, SlotMap map,
                                                           const double* __restrict__ p, const int* __restrict__ tet,
                                                           const double* __restrict__ vol, const double* __restrict__ invJ,
-                                                          const int* __restrict__ rowptr, double* __restrict__ val,
+                                                          const int* __restrict__ rowptr, double* val,
                                                           double* __restrict__ rhs, double coeff, int rhs_kind,
                                                           double rhs_param, Quad3 q)
 {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nv) return;
-    for (int k = rowptr[r]; k < rowptr[r + 1]; ++k) val[k] = 0.0;
+    __shared__ double acc[1][kTile3d];
+    double* const vals[1] = {val};
+    RowTile<1, kTile3d> T(acc, vals, nv, rowptr);
     const double PI = 3.14159265358979323846;
     const double g3[4][3] = {{1, 0, 0}, {0, 1, 0}, {0, 0, 1}, {-1, -1, -1}};
     double rr = 0.0;
-    for (int e = inc_off[r]; e < inc_off[r + 1]; ++e) {
+    const int e1 = T.on ? inc_off[T.r + 1] : 0;
+    for (int e = T.on ? inc_off[T.r] : 0; e < e1; ++e) {
         const int code = inc_code[e];
         const int c = code >> 2, li = code & 3;
         int v[4];
@@ -265,62 +376,81 @@ __global__ __launch_bounds__(kBlock) void k_asm_poisson3d(int nv, const int* __r
             R += f * q.l[k][li] * w;
         }
         const double vc = vol[c];
-        const int* s = inc_slots + 4 * (size_t)e;
-        for (int j = 0; j < 4; ++j) val[s[j]] += M[j] * vc;
+        int s[4];
+        incidence_slots<4>(map, e, T.row, s);
+        for (int j = 0; j < 4; ++j) T.add(0, s[j], M[j] * vc);
         rr += R * vc;
     }
-    rhs[r] = rr;
+    if (T.on) rhs[T.r] = rr;
+    T.finish();
 }
 
 // ------------------------------------------------------------------ PFEM-2 velocity prediction
 // cases/Cylinder2D/main.cu:72-167 (and PoiseuilleFlow2D/main.cu:81-176 for the boundary term on every ID)
-__global__ __launch_bounds__(kBlock) void k_asm_prediction(
-    int nv, const int* __restrict__ inc_off, const int* __restrict__ inc_code, const int* __restrict__ inc_slots,
+template <int NQ>
+__global__ __launch_bounds__(kBlock, 3) void k_asm_prediction(
+    int nv, const int* __restrict__ inc_off, const int* __restrict__ inc_code, SlotMap map,
     const double* __restrict__ xy, const int* __restrict__ tri, const double* __restrict__ area,
     const double4* __restrict__ invJ, const int* __restrict__ edge_ids, const int* __restrict__ rowptr,
-    double* __restrict__ val0, double* __restrict__ val1, double* __restrict__ rhs0, double* __restrict__ rhs1,
+    double* val0, double* val1, double* __restrict__ rhs0, double* __restrict__ rhs1,
     const double* __restrict__ u0, const double* __restrict__ u1, const double* __restrict__ uo0,
     const double* __restrict__ uo1, const double* __restrict__ p_old, Pfem2Prm prm, Quad2 q, Quad1 qe)
 {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nv) return;
-    for (int k = rowptr[r]; k < rowptr[r + 1]; ++k) { val0[k] = 0.0; val1[k] = 0.0; }
+    __shared__ double acc[2][kTile2d];
+    double* const vals[2] = {val0, val1};
+    RowTile<2, kTile2d> T(acc, vals, nv, rowptr);
+    const int nq = NQ ? NQ : q.n;
     const double rho = prm.rho, mu = prm.mu, dt = prm.dt;
     double rr0 = 0.0, rr1 = 0.0;
-    for (int e = inc_off[r]; e < inc_off[r + 1]; ++e) {
-        const int code = inc_code[e];
-        const int c = code >> 2, i = code & 3;
-        int v[3];
-        v[0] = tri[3 * c]; v[1] = tri[3 * c + 1]; v[2] = tri[3 * c + 2];
+    Incidences in(T.on, T.r, inc_off, inc_code, tri);
+    while (in.next()) {
+        const int c = in.code >> 2, i = in.code & 3;
+        const int (&v)[3] = in.v;
         const double4 J = invJ[c];
+        const double ar = area[c];
+        const int ids[3] = {edge_ids[3 * c], edge_ids[3 * c + 1], edge_ids[3 * c + 2]};
+        int s[3];
+        incidence_slots<3>(map, in.e, T.row, s);
+        double U0[3], U1[3], O0[3], O1[3], PO[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            U0[j] = u0[v[j]];
+            U1[j] = u1[v[j]];
+            O0[j] = uo0[v[j]];
+            O1[j] = uo1[v[j]];
+            PO[j] = p_old ? p_old[v[j]] : 0.0;
+        }
         double M0[3] = {0, 0, 0}, M1[3] = {0, 0, 0};
         double R0 = 0.0, R1 = 0.0;
         const double2 gI = grad2(J, i);
-        for (int qp = 0; qp < q.n; ++qp) {
-            const double w = q.w[qp];
-            const double Ni = q.l[qp][i];
+#pragma unroll NQ ? NQ : 1
+        for (int qp = 0; qp < nq; ++qp) {
+            const double w = q.w[NQ ? 0 : qp];
+            const double Ni = pick(i, q.l[qp][0], q.l[qp][1], q.l[qp][2]);
+#pragma unroll
             for (int j = 0; j < 3; ++j) {
                 const double2 gJ = grad2(J, j);
                 const double Nj = q.l[qp][j];
                 double aux = rho * Ni * Nj * w;
                 M0[j] += aux;
-                R0 += aux * uo0[v[j]];
+                R0 += aux * O0[j];
                 M1[j] += aux;
-                R1 += aux * uo1[v[j]];
+                R1 += aux * O1[j];
                 aux = mu * dt * w;
                 M0[j] += aux * (gI.y * gJ.y + 4.0 / 3.0 * gI.x * gJ.x);
                 M1[j] += aux * (gI.x * gJ.x + 4.0 / 3.0 * gI.y * gJ.y);
-                R0 -= aux * (gI.y * gJ.x - 2.0 / 3.0 * gI.x * gJ.y) * u1[v[j]];
-                R1 -= aux * (gI.x * gJ.y - 2.0 / 3.0 * gI.y * gJ.x) * u0[v[j]];
+                R0 -= aux * (gI.y * gJ.x - 2.0 / 3.0 * gI.x * gJ.y) * U1[j];
+                R1 -= aux * (gI.x * gJ.y - 2.0 / 3.0 * gI.y * gJ.x) * U0[j];
                 if (p_old) {
-                    aux = Ni * p_old[v[j]] * dt * w;
+                    aux = Ni * PO[j] * dt * w;
                     R0 -= aux * gJ.x;
                     R1 -= aux * gJ.y;
                 }
             }
         }
+#pragma unroll
         for (int ed = 0; ed < 3; ++ed) {
-            const int id = edge_ids[3 * c + ed];
+            const int id = ids[ed];
             if (id < 0 || id > 7 || !((prm.traction_mask >> id) & 1)) continue;
             const double nx = prm.nrm[id][0], ny = prm.nrm[id][1];
             const int a = v[ed], b = v[(ed + 1) % 3];
@@ -337,113 +467,143 @@ __global__ __launch_bounds__(kBlock) void k_asm_prediction(
                 L[1] = J.y * dx + J.w * dy;
                 L[2] = 1.0 - L[0] - L[1];
                 const double aux = mu * dt * qe.w[qp] * halfLength;
-                const double Ni = L[i];
+                const double Ni = pick(i, L[0], L[1], L[2]);
                 for (int j = 0; j < 3; ++j) {
                     const double2 gJ = grad2(J, j);
                     M0[j] -= aux * Ni * ((4.0 / 3.0) * gJ.x * nx + gJ.y * ny);
                     M1[j] -= aux * Ni * (gJ.x * nx + (4.0 / 3.0) * gJ.y * ny);
-                    R0 += aux * Ni * u1[v[j]] * ((-2.0 / 3.0) * gJ.y * nx + gJ.x * ny);
-                    R1 += aux * Ni * u0[v[j]] * (gJ.y * nx + (-2.0 / 3.0) * gJ.x * ny);
+                    R0 += aux * Ni * U1[j] * ((-2.0 / 3.0) * gJ.y * nx + gJ.x * ny);
+                    R1 += aux * Ni * U0[j] * (gJ.y * nx + (-2.0 / 3.0) * gJ.x * ny);
                 }
             }
         }
-        const double ar = area[c];
-        const int* s = inc_slots + 3 * (size_t)e;
+#pragma unroll
         for (int j = 0; j < 3; ++j) {
-            val0[s[j]] += M0[j] * ar;
-            val1[s[j]] += M1[j] * ar;
+            T.add(0, s[j], M0[j] * ar);
+            T.add(1, s[j], M1[j] * ar);
         }
         rr0 += R0 * ar;
         rr1 += R1 * ar;
     }
-    rhs0[r] = rr0;
-    rhs1[r] = rr1;
+    if (T.on) {
+        rhs0[T.r] = rr0;
+        rhs1[T.r] = rr1;
+    }
+    T.finish();
 }
 
 // ------------------------------------------------------------------ PFEM-2 pressure (Cylinder2D/main.cu:169-211)
+template <int NQ>
 __global__ __launch_bounds__(kBlock) void k_asm_pressure(
-    int nv, const int* __restrict__ inc_off, const int* __restrict__ inc_code, const int* __restrict__ inc_slots,
+    int nv, const int* __restrict__ inc_off, const int* __restrict__ inc_code, SlotMap map,
     const int* __restrict__ tri, const double* __restrict__ area, const double4* __restrict__ invJ,
-    const int* __restrict__ rowptr, double* __restrict__ val, double* __restrict__ rhs, const double* __restrict__ vp0,
+    const int* __restrict__ rowptr, double* val, double* __restrict__ rhs, const double* __restrict__ vp0,
     const double* __restrict__ vp1, const double* __restrict__ p_old, Pfem2Prm prm, Quad2 q)
 {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nv) return;
-    for (int k = rowptr[r]; k < rowptr[r + 1]; ++k) val[k] = 0.0;
+    __shared__ double acc[1][kTile2d];
+    double* const vals[1] = {val};
+    RowTile<1, kTile2d> T(acc, vals, nv, rowptr);
+    const int nq = NQ ? NQ : q.n;
     double rr = 0.0;
-    for (int e = inc_off[r]; e < inc_off[r + 1]; ++e) {
-        const int code = inc_code[e];
-        const int c = code >> 2, i = code & 3;
-        int v[3];
-        v[0] = tri[3 * c]; v[1] = tri[3 * c + 1]; v[2] = tri[3 * c + 2];
+    Incidences in(T.on, T.r, inc_off, inc_code, tri);
+    while (in.next()) {
+        const int c = in.code >> 2, i = in.code & 3;
+        const int (&v)[3] = in.v;
         const double4 J = invJ[c];
+        const double ar = area[c];
+        int s[3];
+        incidence_slots<3>(map, in.e, T.row, s);
+        double V0[3], V1[3], PO[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            V0[j] = vp0[v[j]];
+            V1[j] = vp1[v[j]];
+            PO[j] = p_old ? p_old[v[j]] : 0.0;
+        }
         double M[3] = {0, 0, 0};
         double R = 0.0;
         const double2 gI = grad2(J, i);
-        for (int qp = 0; qp < q.n; ++qp) {
-            const double w = q.w[qp];
-            const double Ni = q.l[qp][i];
+#pragma unroll NQ ? NQ : 1
+        for (int qp = 0; qp < nq; ++qp) {
+            const double w = q.w[NQ ? 0 : qp];
+            const double Ni = pick(i, q.l[qp][0], q.l[qp][1], q.l[qp][2]);
             const double aux = -prm.rho / prm.dt * Ni * w;
+#pragma unroll
             for (int j = 0; j < 3; ++j) {
                 const double2 gJ = grad2(J, j);
-                const double vx = vp0[v[j]], vy = vp1[v[j]];
+                const double vx = V0[j], vy = V1[j];
                 const double aux2 = (gI.x * gJ.x + gI.y * gJ.y) * w;
                 M[j] += aux2;
-                if (p_old) R += aux2 * p_old[v[j]];
+                if (p_old) R += aux2 * PO[j];
                 R += aux * (gJ.x * vx + gJ.y * vy);
             }
         }
-        const double ar = area[c];
-        const int* s = inc_slots + 3 * (size_t)e;
-        for (int j = 0; j < 3; ++j) val[s[j]] += M[j] * ar;
+#pragma unroll
+        for (int j = 0; j < 3; ++j) T.add(0, s[j], M[j] * ar);
         rr += R * ar;
     }
-    rhs[r] = rr;
+    if (T.on) rhs[T.r] = rr;
+    T.finish();
 }
 
 // ------------------------------------------------------------------ PFEM-2 correction (Cylinder2D/main.cu:213-259)
+template <int NQ>
 __global__ __launch_bounds__(kBlock) void k_asm_correction(
-    int nv, const int* __restrict__ inc_off, const int* __restrict__ inc_code, const int* __restrict__ inc_slots,
+    int nv, const int* __restrict__ inc_off, const int* __restrict__ inc_code, SlotMap map,
     const int* __restrict__ tri, const double* __restrict__ area, const double4* __restrict__ invJ,
-    const int* __restrict__ rowptr, double* __restrict__ val, double* __restrict__ rhs0, double* __restrict__ rhs1,
+    const int* __restrict__ rowptr, double* val, double* __restrict__ rhs0, double* __restrict__ rhs1,
     const double* __restrict__ vp0, const double* __restrict__ vp1, const double* __restrict__ p,
     const double* __restrict__ p_old, Pfem2Prm prm, Quad2 q)
 {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nv) return;
-    for (int k = rowptr[r]; k < rowptr[r + 1]; ++k) val[k] = 0.0;
+    __shared__ double acc[1][kTile2d];
+    double* const vals[1] = {val};
+    RowTile<1, kTile2d> T(acc, vals, nv, rowptr);
+    const int nq = NQ ? NQ : q.n;
     double rr0 = 0.0, rr1 = 0.0;
-    for (int e = inc_off[r]; e < inc_off[r + 1]; ++e) {
-        const int code = inc_code[e];
-        const int c = code >> 2, i = code & 3;
-        int v[3];
-        v[0] = tri[3 * c]; v[1] = tri[3 * c + 1]; v[2] = tri[3 * c + 2];
+    Incidences in(T.on, T.r, inc_off, inc_code, tri);
+    while (in.next()) {
+        const int c = in.code >> 2, i = in.code & 3;
+        const int (&v)[3] = in.v;
         const double4 J = invJ[c];
+        const double ar = area[c];
+        int s[3];
+        incidence_slots<3>(map, in.e, T.row, s);
+        double V0[3], V1[3], PV[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            V0[j] = vp0[v[j]];
+            V1[j] = vp1[v[j]];
+            PV[j] = p[v[j]];
+            if (p_old) PV[j] -= p_old[v[j]];
+        }
         double M[3] = {0, 0, 0};
         double R0 = 0.0, R1 = 0.0;
-        for (int qp = 0; qp < q.n; ++qp) {
-            const double w = q.w[qp];
-            const double Ni = q.l[qp][i];
+#pragma unroll NQ ? NQ : 1
+        for (int qp = 0; qp < nq; ++qp) {
+            const double w = q.w[NQ ? 0 : qp];
+            const double Ni = pick(i, q.l[qp][0], q.l[qp][1], q.l[qp][2]);
             const double aux2 = prm.dt * Ni * w;
+#pragma unroll
             for (int j = 0; j < 3; ++j) {
                 const double2 gJ = grad2(J, j);
                 const double Nj = q.l[qp][j];
                 const double aux = prm.rho * Ni * Nj * w;
-                double pv = p[v[j]];
-                if (p_old) pv -= p_old[v[j]];
+                const double pv = PV[j];
                 M[j] += aux;
-                R0 += aux * vp0[v[j]] - aux2 * gJ.x * pv;
-                R1 += aux * vp1[v[j]] - aux2 * gJ.y * pv;
+                R0 += aux * V0[j] - aux2 * gJ.x * pv;
+                R1 += aux * V1[j] - aux2 * gJ.y * pv;
             }
         }
-        const double ar = area[c];
-        const int* s = inc_slots + 3 * (size_t)e;
-        for (int j = 0; j < 3; ++j) val[s[j]] += M[j] * ar;
+#pragma unroll
+        for (int j = 0; j < 3; ++j) T.add(0, s[j], M[j] * ar);
         rr0 += R0 * ar;
         rr1 += R1 * ar;
     }
-    rhs0[r] = rr0;
-    rhs1[r] = rr1;
+    if (T.on) {
+        rhs0[T.r] = rr0;
+        rhs1[T.r] = rr1;
+    }
+    T.finish();
 }
 
 // ------------------------------------------------------------------ prediction BC values
@@ -544,6 +704,11 @@ __global__ void k_body_sum(int ne, const double* __restrict__ loads, double* __r
     for (int d = 0; d < 4; ++d) out[d] = t[d];
 }
 
+static SlotMap slot_map(const Incidence& inc) { return SlotMap{inc.rel.p, inc.slots.p}; }
+
+// The three-point rules have one weight; terms without a barycentric coordinate are then the same at every point.
+static bool equal_weights3(const Quad2& q) { return q.n == 3 && q.w[0] == q.w[1] && q.w[1] == q.w[2]; }
+
 static Pfem2Prm to_prm(const pfem_pfem2_params* p)
 {
     Pfem2Prm o{};
@@ -570,8 +735,8 @@ void assemble_prediction(pfem_mesh2d m, pfem_csr a0, pfem_csr a1, double* rhs0, 
     const Quad2 q = face_rule(prm->face_quad);
     const Quad1 qe = edge_rule(prm->edge_quad);
     Context* c = C(m->ctx);
-    hipLaunchKernelGGL(k_asm_prediction, dim3(blocks_for(m->nv)), dim3(kBlock), 0, c->stream, m->nv, m->inc.off.p,
-                       m->inc.code.p, m->inc.slots.p, m->xy.p, m->tri.p, m->area.p, (const double4*)m->invJ.p,
+    hipLaunchKernelGGL(equal_weights3(q) ? k_asm_prediction<3> : k_asm_prediction<0>, dim3(blocks_for(m->nv)), dim3(kBlock), 0, c->stream, m->nv, m->inc.off.p,
+                       m->inc.code.p, slot_map(m->inc), m->xy.p, m->tri.p, m->area.p, (const double4*)m->invJ.p,
                        m->edge_ids.p, m->pat->rowptr.p, a0->val.p, a1->val.p, rhs0, rhs1, u0, u1, uo0, uo1, p_old,
                        to_prm(prm), q, qe);
     PFEM_HIP(hipGetLastError());
@@ -583,8 +748,8 @@ void assemble_pressure(pfem_mesh2d m, pfem_csr a, double* rhs, const double* vp0
     check_pattern(m, a);
     const Quad2 q = face_rule(prm->face_quad);
     Context* c = C(m->ctx);
-    hipLaunchKernelGGL(k_asm_pressure, dim3(blocks_for(m->nv)), dim3(kBlock), 0, c->stream, m->nv, m->inc.off.p,
-                       m->inc.code.p, m->inc.slots.p, m->tri.p, m->area.p, (const double4*)m->invJ.p,
+    hipLaunchKernelGGL(equal_weights3(q) ? k_asm_pressure<3> : k_asm_pressure<0>, dim3(blocks_for(m->nv)), dim3(kBlock), 0, c->stream, m->nv, m->inc.off.p,
+                       m->inc.code.p, slot_map(m->inc), m->tri.p, m->area.p, (const double4*)m->invJ.p,
                        m->pat->rowptr.p, a->val.p, rhs, vp0, vp1, p_old, to_prm(prm), q);
     PFEM_HIP(hipGetLastError());
 }
@@ -595,8 +760,8 @@ void assemble_correction(pfem_mesh2d m, pfem_csr a, double* rhs0, double* rhs1, 
     check_pattern(m, a);
     const Quad2 q = face_rule(prm->face_quad);
     Context* c = C(m->ctx);
-    hipLaunchKernelGGL(k_asm_correction, dim3(blocks_for(m->nv)), dim3(kBlock), 0, c->stream, m->nv, m->inc.off.p,
-                       m->inc.code.p, m->inc.slots.p, m->tri.p, m->area.p, (const double4*)m->invJ.p,
+    hipLaunchKernelGGL(equal_weights3(q) ? k_asm_correction<3> : k_asm_correction<0>, dim3(blocks_for(m->nv)), dim3(kBlock), 0, c->stream, m->nv, m->inc.off.p,
+                       m->inc.code.p, slot_map(m->inc), m->tri.p, m->area.p, (const double4*)m->invJ.p,
                        m->pat->rowptr.p, a->val.p, rhs0, rhs1, vp0, vp1, p, p_old, to_prm(prm), q);
     PFEM_HIP(hipGetLastError());
 }
@@ -787,8 +952,8 @@ int pfem_assemble_poisson2d(pfem_mesh2d m, pfem_csr a, double* d_rhs, double coe
         check_pattern(m, a);
         const Quad2 q = face_rule(quad_index);
         Context* c = C(m->ctx);
-        hipLaunchKernelGGL(k_asm_poisson2d, dim3(blocks_for(m->nv)), dim3(kBlock), 0, c->stream, m->nv,
-                           m->inc.off.p, m->inc.code.p, m->inc.slots.p, m->xy.p, m->tri.p, m->area.p,
+        hipLaunchKernelGGL(equal_weights3(q) ? k_asm_poisson2d<3> : k_asm_poisson2d<0>, dim3(blocks_for(m->nv)), dim3(kBlock), 0, c->stream, m->nv,
+                           m->inc.off.p, m->inc.code.p, slot_map(m->inc), m->xy.p, m->tri.p, m->area.p,
                            (const double4*)m->invJ.p, m->pat->rowptr.p, a->val.p, d_rhs, coeff, rhs_kind, rhs_param, q);
         PFEM_HIP(hipGetLastError());
     });
@@ -803,7 +968,7 @@ int pfem_assemble_poisson3d(pfem_mesh3d m, pfem_csr a, double* d_rhs, double coe
         const Quad3 q = cell_rule(quad_index);
         Context* c = C(m->ctx);
         hipLaunchKernelGGL(k_asm_poisson3d, dim3(blocks_for(m->nv)), dim3(kBlock), 0, c->stream, m->nv,
-                           m->inc.off.p, m->inc.code.p, m->inc.slots.p, m->xyz.p, m->tet.p, m->vol.p, m->invJ.p,
+                           m->inc.off.p, m->inc.code.p, slot_map(m->inc), m->xyz.p, m->tet.p, m->vol.p, m->invJ.p,
                            m->pat->rowptr.p, a->val.p, d_rhs, coeff, rhs_kind, rhs_param, q);
         PFEM_HIP(hipGetLastError());
     });

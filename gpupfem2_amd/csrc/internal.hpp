@@ -122,7 +122,10 @@ struct Incidence {
     int nper = 3;
     pfem::DevArray<int> off;    // nv + 1
     pfem::DevArray<int> code;   // cell * 4 + local
-    pfem::DevArray<int> slots;  // nper per incidence
+    // where (node, vertex j) lies in the node's CSR row: one byte per j, or, if a row holds more than 256
+    // entries, the CSR slots themselves (nper per incidence)
+    pfem::DevArray<uint32_t> rel;
+    pfem::DevArray<int> slots;
     std::vector<int> h_off, h_code;
 };
 

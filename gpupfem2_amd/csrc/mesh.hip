@@ -167,7 +167,11 @@ static void build_incidence(Context* ctx, int nv, int nt, int nper, const std::v
     for (int v = 0; v < nv; ++v) inc.h_off[v + 1] += inc.h_off[v];
     const size_t ninc = inc.h_off[nv];
     inc.h_code.assign(ninc, 0);
-    std::vector<int> slots(ninc * nper);
+    int longest = 0;
+    for (int v = 0; v < nv; ++v) longest = std::max(longest, P.h_rowptr[v + 1] - P.h_rowptr[v]);
+    const bool bytes = longest <= 256;
+    std::vector<int> slots(bytes ? 0 : ninc * nper);
+    std::vector<uint32_t> rel(bytes ? ninc : 0, 0u);
     std::vector<int> fill(inc.h_off.begin(), inc.h_off.end() - 1);
     for (int c = 0; c < nt; ++c)
         for (int a = 0; a < nper; ++a) {
@@ -180,11 +184,13 @@ static void build_incidence(Context* ctx, int nv, int nt, int nper, const std::v
                 const int* e = P.h_col.data() + P.h_rowptr[v + 1];
                 const int* it = std::lower_bound(b, e, w);
                 if (it == e || *it != w) throw Error(PFEM_EINVAL, "mesh cell vertex missing from CSR row");
-                slots[(size_t)k * nper + j] = (int)(it - P.h_col.data());
+                if (bytes) rel[k] |= (uint32_t)(it - b) << (8 * j);
+                else slots[(size_t)k * nper + j] = (int)(it - P.h_col.data());
             }
         }
     upload(ctx, inc.off, inc.h_off);
     upload(ctx, inc.code, inc.h_code);
+    upload(ctx, inc.rel, rel);
     upload(ctx, inc.slots, slots);
 }
 
