@@ -23,6 +23,7 @@
 #include <cmath>
 #include <cstddef>
 #include <cstring>
+#include <memory>
 #include <vector>
 
 #include "device.hpp"
@@ -32,325 +33,416 @@
 namespace pfem {
 
 constexpr int kMaxRhs = 8;
-constexpr int kMGrid = 2048;   // grid of the multi-RHS kernels (grid-stride over row groups)
-static_assert(kMGrid % kBlock == 0, "partial series are read in whole blocks");
+constexpr int kMBlock = 512;              // workgroup of the multi-RHS kernels: one wave per column when it adds up partials
+constexpr int kMWaves = kMBlock / 64;
+constexpr int kMGrid = 768;               // most workgroups of a kernel that leaves partial sums
+constexpr int kMStream = 512;             // workgroups of the vector kernels
+static_assert(kMGrid % 64 == 0 && kMStream <= kMGrid, "a wave adds up a series in whole rounds");
 
-struct MState {
-    double tol;
-    int tol_mode, maxit, ncol, all_done;
-    double gam[2][kMaxRhs], alpha[kMaxRhs], beta[kMaxRhs], thr[kMaxRhs], res[kMaxRhs];
-    int it[kMaxRhs], done[kMaxRhs], converged[kMaxRhs], nan[kMaxRhs];
-    // reliable updates: gamma of the current residual, gamma at the last replacement, the slot state
-    // (0 iterating, 1 replacement due, 2 direction update after a replacement) and the replacements made
-    double rz[kMaxRhs], rzmax[kMaxRhs], drop;
-    int mode[kMaxRhs], nrep[kMaxRhs];
+// One column's scalars. gam: gamma of the current residual; rzmax: gamma at the last replacement (mixed); mode:
+// 0 iterating, 1 replacement due, 2 direction update after a replacement (mixed).
+struct MCol {
+    double gam, thr, res, alpha, beta, rzmax;
+    int it, done, converged, nan, mode, nrep;
 };
 
+// Two of these take turns within an iteration: the kernel after the product reads the first and leaves the
+// second, the direction update reads the second and leaves the first, so that no workgroup reads what
+// another of its launch writes.
+struct MState {
+    double tol, drop;
+    int tol_mode, maxit, ncol, all_done;
+    MCol col[kMaxRhs];
+};
 
-// Per-column block sums of NV values: lane l holds column l % G. Reduced over the wave with shuffles that
-// keep the column (offsets 32 .. G), then over the four waves in order; part[(i * G + j) * gridDim.x +
+// N consecutive columns of a row, loaded and stored at once
+template <typename T, int N>
+struct Columns {
+    typedef T type __attribute__((ext_vector_type(N)));
+};
+
+// Columns that one lane of a product takes
+template <int G>
+constexpr int kCols = G < 2 ? G : 2;
+
+// Per-column block sums of NV values: lane l holds the NC columns from (l % (G / NC)) * NC on. Reduced over the
+// wave with shuffles that keep the columns, then over the waves in order; part[(i * G + j) * gridDim.x +
 // blockIdx.x] = value i of column j.
-template <int G, int NV>
-__device__ __forceinline__ void group_partials(double (&v)[NV], double* __restrict__ part)
+template <int G, int NV, int NC>
+__device__ __forceinline__ void group_partials(double (&v)[NV][NC], double* __restrict__ part)
 {
-    __shared__ double sh[NV][kWaves][G];
+    __shared__ double sh[NV][kMWaves][G];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
+    for (int i = 0; i < NV; ++i)
 #pragma unroll
-        for (int off = 32; off >= G; off >>= 1) v[i] += __shfl_down(v[i], off, 64);
-        if (lane < G) sh[i][wid][lane] = v[i];
-    }
+        for (int c = 0; c < NC; ++c) {
+#pragma unroll
+            for (int off = 32; off >= G / NC; off >>= 1) v[i][c] += __shfl_down(v[i][c], off, 64);
+            if (lane < G / NC) sh[i][wid][lane * NC + c] = v[i][c];
+        }
     __syncthreads();
     if (threadIdx.x < G) {
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
             double s = sh[i][0][threadIdx.x];
-            for (int w = 1; w < kWaves; ++w) s += sh[i][w][threadIdx.x];
+            for (int w = 1; w < kMWaves; ++w) s += sh[i][w][threadIdx.x];
             part[((size_t)i * G + threadIdx.x) * gridDim.x + blockIdx.x] = s;
         }
     }
 }
 
-// Totals of NJ partial series of nb <= kMGrid terms each (series j at part + j * nb: the grid of the
-// kernel that wrote them), valid in thread 0. Every load of a lane is issued before the first addition
-// (one memory round trip); lane t adds terms t, t + 256, ... of each series in order, then block_sum.
-template <int NJ>
-__device__ __forceinline__ void series_totals(const double* __restrict__ part, int nb, double (&tot)[NJ])
+// Total of a partial series of nb <= kMGrid terms, valid in lane 0 of the wave. Every load is issued before
+// the first addition (one memory round trip); lane t adds terms t, t + 64, ... in order, then wave_sum.
+__device__ __forceinline__ double series_total(const double* __restrict__ part, int nb)
 {
-    constexpr int kPer = kMGrid / kBlock;
-    double t[NJ][kPer];
+    constexpr int kPer = kMGrid / 64;
+    const int lane = threadIdx.x & 63;
+    double t[kPer];
 #pragma unroll
-    for (int j = 0; j < NJ; ++j)
-#pragma unroll
-        for (int u = 0; u < kPer; ++u) {
-            const int k = threadIdx.x + u * kBlock;
-            t[j][u] = k < nb ? part[(size_t)j * nb + k] : 0.0;
-        }
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-        double s = 0.0;
-#pragma unroll
-        for (int u = 0; u < kPer; ++u) s += t[j][u];
-        tot[j] = s;
+    for (int u = 0; u < kPer; ++u) {
+        const int k = lane + u * 64;
+        t[u] = k < nb ? part[k] : 0.0;
     }
-    block_sum<NJ>(tot);
+    double s = 0.0;
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) s += t[u];
+    return wave_sum(s);
 }
 
-// ---- FP64 / FP32 multi-RHS CG kernels (T = vector type, VT = matrix value type)
-constexpr int kMTileNnz = 1024;   // non-zeros of a row tile staged in LDS
-constexpr int kMRows = 2;         // rows per lane in a row tile
+// The scalar step between two kernels, at the head of the second one: wave j adds up column j's partials and
+// moves the column's scalars on with f(column, total); every workgroup does so for itself (a few loads from
+// L2, where a launch of one workgroup between the kernels took 8.5 to 12 us of a 78 us iteration of 8 columns
+// x 0.27M rows), and workgroup 0 leaves the result in `out`. False if nothing is left to do.
+template <int G, typename F>
+__device__ __forceinline__ bool scalar_step(const MState* __restrict__ in, MState* __restrict__ out,
+                                            const double* __restrict__ part, int nb, MCol (&sc)[G], F f)
+{
+    static_assert(G <= kMWaves, "one wave per column");
+    const bool live = !in->all_done;
+    const int wid = threadIdx.x >> 6;
+    if (wid < G) {
+        const double tot = live ? series_total(part + (size_t)wid * nb, nb) : 0.0;
+        if ((threadIdx.x & 63) == 0) {
+            MCol c = in->col[wid];
+            if (live && !c.done) f(c, tot);
+            sc[wid] = c;
+        }
+    }
+    __syncthreads();
+    if (blockIdx.x == 0) {
+        if (threadIdx.x < G) out->col[threadIdx.x] = sc[threadIdx.x];
+        if (threadIdx.x == 0) {
+            int all = 1;
+            for (int j = 0; j < G; ++j) all &= sc[j].done;
+            out->all_done = all;
+        }
+    }
+    return live;
+}
 
-// Row tiles of the multi-RHS products: tile t = rows [tiles[2t], tiles[2t+1]), at most kMRows * kBlock / G
-// rows and at most kMTileNnz non-zeros unless a single row is longer. Lane (q, j) of a workgroup takes
-// column j of rows q and q + kBlock / G of the tile. Workgroup b takes a contiguous range of tiles; the
+// Elements o = i * G + j of the interleaved vectors in grid strides (a lane keeps its column), kMU at a time
+constexpr int kMU = 4;
+template <int G, typename F>
+__device__ __forceinline__ void for_elements(int n, F f)
+{
+    const long m = (long)n * G, stride = (long)gridDim.x * kMBlock;
+    for (long o = (long)blockIdx.x * kMBlock + threadIdx.x; o < m; o += kMU * stride) f(o, stride, m);
+}
+
+constexpr int kMTileNnz = 2048;   // non-zeros of a row tile staged in LDS
+template <int G>
+constexpr int tile_rows = kMBlock / G * kCols<G>;
+
+// Row tiles of the multi-RHS products: tile t = rows [tiles[2t], tiles[2t+1]), at most tile_rows<G>
+// rows and at most kMTileNnz non-zeros unless a single row is longer. A lane takes kCols columns of a row. Workgroup b takes a contiguous range of tiles; the
 // ranges of XCD x (workgroups b = x mod 8) form the x-th band of rows, so neighbouring rows share their
-// gathered vector entries in one L2. A tile's values, column indices and row offsets are staged in LDS
-// with unit-stride loads while the next tile's bounds are fetched; each lane then adds val * x[col * G + j]
-// over its rows left to right (the sequential order), with up to 8 gathers per row in flight, and hands
-// each sum to f(row, j, s). The G lanes of a row gather G contiguous values.
+// gathered vector entries in one L2. A tile's values, column indices and row offsets pass through registers into
+// LDS with unit-stride loads that are in flight while the tile before is computed; each lane then adds
+// val * x[col * G + j] over its rows left to right (the sequential order), with up to kU gathers per row in
+// flight, and hands each sum to f(row, j, s). The lanes of a row gather G contiguous values.
+// The gathers bound it (33M of them through L1 and L2, 8 columns x 0.27M rows): two columns to a lane halve the
+// gather and LDS instructions, and six wavefronts a SIMD with four gathers in flight each hide more than four
+// with eight or sixteen. 29.0 us before, with one column to a lane; now 22.2 (with eight in flight 24.5 at four
+// wavefronts, 31.9 at six with spills; two in flight 24.3).
 template <int G, typename T, typename VT, typename F>
 __device__ __forceinline__ void for_tile_rows(int ntiles, const int* __restrict__ tiles, const int* __restrict__ rowptr,
                                               const int* __restrict__ col, const VT* __restrict__ val,
                                               const T* __restrict__ x, F f)
 {
-    constexpr int kLanesRows = kBlock / G;
-    constexpr int kTileRows = kMRows * kLanesRows;
-    constexpr int kU = 8;
+    constexpr int NC = kCols<G>, kLanes = G / NC;   // lanes per row
+    constexpr int kTileRows = tile_rows<G>;
+    using V = typename Columns<T, NC>::type;
+    constexpr int kU = 4;
+    constexpr int kStage = kMTileNnz / kMBlock;
+    constexpr int kRp = (kTileRows + 1 + kMBlock - 1) / kMBlock;
     __shared__ VT sval[kMTileNnz];
     __shared__ int scol[kMTileNnz];
     __shared__ int rp[kTileRows + 1];
     const int nb = gridDim.x, b = blockIdx.x;
     const int rb = (b % 8) * (nb / 8) + b / 8;
     const int t0 = (int)((long)ntiles * rb / nb), t1 = (int)((long)ntiles * (rb + 1) / nb);
-    const int j = threadIdx.x % G, q = threadIdx.x / G;
-    int r0 = 0, r1 = 0, k0 = 0, k1 = 0;
-    if (t0 < t1) {
-        r0 = tiles[2 * t0];
-        r1 = tiles[2 * t0 + 1];
-        k0 = rowptr[r0];
-        k1 = rowptr[r1];
+    const int j = threadIdx.x % kLanes * NC, q = threadIdx.x / kLanes;
+    if (t0 >= t1) return;
+    // bounds of tile t (current), of t + 1 (being staged) and of t + 2
+    int r0 = tiles[2 * t0], r1 = tiles[2 * t0 + 1];
+    int k0 = rowptr[r0], k1 = rowptr[r1];
+    VT nv[kStage];
+    int nc[kStage], nr[kRp];
+    auto fetch = [&](int a, int z, int ka, int kz) {
+#pragma unroll
+        for (int u = 0; u < kRp; ++u) {
+            const int i = threadIdx.x + u * kMBlock;
+            nr[u] = i <= z - a ? rowptr[a + i] - ka : 0;
+        }
+        if (kz - ka <= kMTileNnz)
+#pragma unroll
+            for (int u = 0; u < kStage; ++u) {
+                const int k = ka + (int)threadIdx.x + u * kMBlock;
+                if (k < kz) {
+                    nv[u] = val[k];
+                    nc[u] = col[k];
+                }
+            }
+    };
+    fetch(r0, r1, k0, k1);
+    int n0 = 0, n1 = 0, m0 = 0, m1 = 0;
+    if (t0 + 1 < t1) {
+        n0 = tiles[2 * t0 + 2];
+        n1 = tiles[2 * t0 + 3];
+        m0 = rowptr[n0];
+        m1 = rowptr[n1];
     }
     for (int t = t0; t < t1; ++t) {
-        const int nk = k1 - k0;
-        const bool staged = nk <= kMTileNnz;
+        const bool staged = k1 - k0 <= kMTileNnz;
         __syncthreads();   // the previous tile's readers are done with the LDS arrays
-        for (int i = threadIdx.x; i <= r1 - r0; i += kBlock) rp[i] = rowptr[r0 + i] - k0;
+#pragma unroll
+        for (int u = 0; u < kRp; ++u) {
+            const int i = threadIdx.x + u * kMBlock;
+            if (i <= r1 - r0) rp[i] = nr[u];
+        }
         if (staged)
-            for (int k = threadIdx.x; k < nk; k += kBlock) {
-                sval[k] = val[k0 + k];
-                scol[k] = col[k0 + k];
+#pragma unroll
+            for (int u = 0; u < kStage; ++u) {
+                const int k = threadIdx.x + u * kMBlock;
+                if (k < k1 - k0) {
+                    sval[k] = nv[u];
+                    scol[k] = nc[u];
+                }
             }
-        // the next tile's bounds, fetched while this one is computed
-        int n0 = 0, n1 = 0, m0 = 0, m1 = 0;
-        if (t + 1 < t1) {
-            n0 = tiles[2 * t + 2];
-            n1 = tiles[2 * t + 3];
-            m0 = rowptr[n0];
-            m1 = rowptr[n1];
+        // the next tile is fetched while this one is computed
+        if (t + 1 < t1) fetch(n0, n1, m0, m1);
+        int p0 = 0, p1 = 0, l0 = 0, l1 = 0;
+        if (t + 2 < t1) {
+            p0 = tiles[2 * t + 4];
+            p1 = tiles[2 * t + 5];
+            l0 = rowptr[p0];
+            l1 = rowptr[p1];
         }
         __syncthreads();
-        T s[kMRows];
-#pragma unroll
-        for (int u = 0; u < kMRows; ++u) s[u] = 0;
-        if (staged) {
-            int ka[kMRows], ke[kMRows];
-#pragma unroll
-            for (int u = 0; u < kMRows; ++u) {
-                const int lr = q + u * kLanesRows;
-                ka[u] = lr < r1 - r0 ? rp[lr] : 0;
-                ke[u] = lr < r1 - r0 ? rp[lr + 1] : 0;
-            }
-            int len = 0;
-#pragma unroll
-            for (int u = 0; u < kMRows; ++u) len = max(len, ke[u] - ka[u]);
-            for (int d = 0; d < len; d += kU) {
-                T xv[kMRows][kU], vv[kMRows][kU];
-#pragma unroll
-                for (int u = 0; u < kMRows; ++u)
-#pragma unroll
-                    for (int w = 0; w < kU; ++w) {
-                        const int k = ka[u] + d + w;
-                        if (k < ke[u]) {
-                            vv[u][w] = (T)sval[k];
-                            xv[u][w] = x[(size_t)scol[k] * G + j];
-                        }
-                    }
-#pragma unroll
-                for (int u = 0; u < kMRows; ++u)
+        const int row = r0 + q;
+        if (row < r1) {
+            V s = (V)(T)0;
+            if (staged) {
+                const int ka = rp[q], ke = rp[q + 1];
+                for (int d = ka; d < ke; d += kU) {
+                    V xv[kU];
+                    T vv[kU];
 #pragma unroll
                     for (int w = 0; w < kU; ++w)
-                        if (ka[u] + d + w < ke[u]) s[u] += vv[u][w] * xv[u][w];
-            }
-        } else {
+                        if (d + w < ke) {
+                            vv[w] = (T)sval[d + w];
+                            xv[w] = *reinterpret_cast<const V*>(x + (size_t)scol[d + w] * G + j);
+                        }
 #pragma unroll
-            for (int u = 0; u < kMRows; ++u) {
-                const int row = r0 + q + u * kLanesRows;
-                if (row < r1)
-                    for (int k = rowptr[row]; k < rowptr[row + 1]; ++k) s[u] += (T)val[k] * x[(size_t)col[k] * G + j];
+                    for (int w = 0; w < kU; ++w)
+                        if (d + w < ke) s += vv[w] * xv[w];
+                }
+            } else {
+                for (int k = rowptr[row]; k < rowptr[row + 1]; ++k)
+                    s += (T)val[k] * *reinterpret_cast<const V*>(x + (size_t)col[k] * G + j);
             }
+            f(row, j, s);
         }
-#pragma unroll
-        for (int u = 0; u < kMRows; ++u) {
-            const int row = r0 + q + u * kLanesRows;
-            if (row < r1) f(row, j, s[u]);
-        }
-        r0 = n0;
-        r1 = n1;
-        k0 = m0;
-        k1 = m1;
+        r0 = n0; r1 = n1; k0 = m0; k1 = m1;
+        n0 = p0; n1 = p1; m0 = l0; m1 = l1;
     }
 }
 
-// r = b - A x (or b when x = 0), p = z = M^-1 r; partials (r, z) and (b, M^-1 b) per column
-template <int G, typename T, typename VT, bool JAC>
-__global__ __launch_bounds__(kBlock) void k_m_init(int n, int ntiles, const int* __restrict__ tiles,
-                                                   const int* __restrict__ rowptr, const int* __restrict__ col,
-                                                   const VT* __restrict__ val, const T* __restrict__ x,
-                                                   const T* __restrict__ b, const T* __restrict__ invd, T* __restrict__ r,
-                                                   T* __restrict__ p, double* __restrict__ part, int x_zero)
+// ---- FP64 multi-RHS CG kernels
+// r = b - A x, p = z = M^-1 r; partials (r, z) and (b, M^-1 b) per column
+template <int G, bool JAC>
+__global__ __launch_bounds__(kMBlock, 6) void k_m_init(int ntiles, const int* __restrict__ tiles,
+                                                       const int* __restrict__ rowptr, const int* __restrict__ col,
+                                                       const double* __restrict__ val, const double* __restrict__ x,
+                                                       const double* __restrict__ b, const double* __restrict__ invd,
+                                                       double* __restrict__ r, double* __restrict__ p, double* __restrict__ part)
 {
-    double v[2] = {0.0, 0.0};
-    auto row_init = [&](int i, int j, T ax) {
+    constexpr int NC = kCols<G>;
+    using V = typename Columns<double, NC>::type;
+    double v[2][NC] = {};
+    for_tile_rows<G, double, double>(ntiles, tiles, rowptr, col, val, x, [&](int i, int j, V ax) {
         const size_t o = (size_t)i * G + j;
-        const T bb = b[o];
-        const T rr = bb - ax;
-        const T zz = JAC ? rr * invd[i] : rr;
-        const T mb = JAC ? bb * invd[i] : bb;
-        r[o] = rr;
-        p[o] = zz;
-        v[0] += (double)(rr * zz);
-        v[1] += (double)(bb * mb);
-    };
-    if (x_zero) {
-        const int j = threadIdx.x % G;
-        for (int i = blockIdx.x * (kBlock / G) + threadIdx.x / G; i < n; i += gridDim.x * (kBlock / G))
-            row_init(i, j, (T)0);
-    } else {
-        for_tile_rows<G, T, VT>(ntiles, tiles, rowptr, col, val, x, row_init);
-    }
-    group_partials<G, 2>(v, part);
+        const V bb = *reinterpret_cast<const V*>(b + o);
+        const double d = JAC ? invd[i] : 1.0;
+        const V rr = bb - ax;
+        const V zz = JAC ? rr * d : rr;
+        const V mb = JAC ? bb * d : bb;
+        *reinterpret_cast<V*>(r + o) = rr;
+        *reinterpret_cast<V*>(p + o) = zz;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            v[0][c] += rr[c] * zz[c];
+            v[1][c] += bb[c] * mb[c];
+        }
+    });
+    group_partials<G>(v, part);
 }
 
 // gamma_0, the per-column thresholds (linear_solver.cu:360; relative to (b, M^-1 b) on request, absolute
 // for a zero column) and the columns already converged; one block
 template <int G>
-__global__ void k_m_begin(MState* st, const double* __restrict__ part, int nb)
+__global__ __launch_bounds__(kMBlock) void k_m_begin(MState* st, const double* __restrict__ part, int nb)
 {
-    double tot[2 * G];
-    series_totals<2 * G>(part, nb, tot);
-    if (threadIdx.x != 0) return;
-    int all = 1;
-    for (int j = 0; j < G; ++j) {
-        const double rz = tot[j], bmb = tot[G + j];
-        st->gam[0][j] = rz;
-        st->thr[j] = st->tol_mode == PFEM_TOL_RELATIVE && bmb > 0.0 ? st->tol * st->tol * bmb : st->tol * st->tol;
-        st->it[j] = 0;
-        st->nan[j] = rz != rz;
-        st->converged[j] = rz < st->thr[j] ? 1 : 0;
-        st->done[j] = j >= st->ncol || st->converged[j] || st->nan[j];
-        st->res[j] = sqrt(fabs(rz));
-        all &= st->done[j];
+    __shared__ int done[G];
+    const int j = threadIdx.x >> 6;
+    if (j < G) {
+        const double rz = series_total(part + (size_t)j * nb, nb), bmb = series_total(part + (size_t)(G + j) * nb, nb);
+        if ((threadIdx.x & 63) == 0) {
+            MCol c{};
+            c.gam = c.rzmax = rz;
+            c.thr = st->tol_mode == PFEM_TOL_RELATIVE && bmb > 0.0 ? st->tol * st->tol * bmb : st->tol * st->tol;
+            c.nan = rz != rz;
+            c.converged = rz < c.thr ? 1 : 0;
+            c.done = j >= st->ncol || c.converged || c.nan;
+            c.res = sqrt(fabs(rz));
+            st->col[j] = c;
+            done[j] = c.done;
+        }
     }
-    st->all_done = all;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int all = 1;
+        for (int k = 0; k < G; ++k) all &= done[k];
+        st->all_done = all;
+    }
 }
 
 // q = A p; partials (p, q) per column
-template <int G, typename T, typename VT>
-__global__ __launch_bounds__(kBlock) void k_m_spmv(int ntiles, const int* __restrict__ tiles, const int* __restrict__ rowptr,
-                                                   const int* __restrict__ col, const VT* __restrict__ val,
-                                                   const T* __restrict__ p, T* __restrict__ q, const MState* st,
-                                                   double* __restrict__ part)
+template <int G>
+__global__ __launch_bounds__(kMBlock, 6) void k_m_spmv(int ntiles, const int* __restrict__ tiles,
+                                                       const int* __restrict__ rowptr, const int* __restrict__ col,
+                                                       const double* __restrict__ val, const double* __restrict__ p,
+                                                       double* __restrict__ q, const MState* __restrict__ st,
+                                                       double* __restrict__ part)
 {
     if (st->all_done) return;
-    double v[1] = {0.0};
-    for_tile_rows<G, T, VT>(ntiles, tiles, rowptr, col, val, p, [&](int i, int j, T ap) {
+    constexpr int NC = kCols<G>;
+    using V = typename Columns<double, NC>::type;
+    double v[1][NC] = {};
+    for_tile_rows<G, double, double>(ntiles, tiles, rowptr, col, val, p, [&](int i, int j, V ap) {
         const size_t o = (size_t)i * G + j;
-        q[o] = ap;
-        v[0] += (double)(p[o] * ap);
+        *reinterpret_cast<V*>(q + o) = ap;
+        const V pp = *reinterpret_cast<const V*>(p + o);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) v[0][c] += pp[c] * ap[c];
     });
-    group_partials<G, 1>(v, part);
+    group_partials<G>(v, part);
 }
 
-// alpha_j = gamma_j / (p_j, q_j) for the active columns; one block
-template <int G>
-__global__ void k_m_alpha(MState* st, const double* __restrict__ part, int nb, int k)
+// alpha = gamma / (p, q); r -= alpha q (updateXR, linear_solver.cu:68-77) for the active columns; partials
+// (r, M^-1 r). x += alpha p is left to k_m_p, which reads p anyway: 8 vectors pass per iteration instead of 9.
+template <int G, bool JAC>
+__global__ __launch_bounds__(kMBlock) void k_m_update(int n, double* __restrict__ r, const double* __restrict__ q,
+                                                      const double* __restrict__ invd, const MState* __restrict__ st,
+                                                      MState* __restrict__ out, const double* __restrict__ pa, int na,
+                                                      double* __restrict__ part)
 {
-    if (st->all_done) return;
-    double tot[G];
-    series_totals<G>(part, nb, tot);
-    if (threadIdx.x != 0) return;
-    for (int j = 0; j < G; ++j) st->alpha[j] = st->done[j] ? 0.0 : st->gam[k & 1][j] / tot[j];
-}
-
-// x += alpha p, r -= alpha q (updateXR, linear_solver.cu:68-77) for the active columns; partials (r, M^-1 r)
-template <int G, typename T, bool JAC>
-__global__ void k_m_update(int n, T* __restrict__ x, T* __restrict__ r, const T* __restrict__ p, const T* __restrict__ q,
-                           const T* __restrict__ invd, const MState* st, double* __restrict__ part)
-{
-    if (st->all_done) return;
+    __shared__ MCol sc[G];
+    const bool live = scalar_step<G>(st, out, pa, na, sc, [](MCol& c, double tot) { c.alpha = c.gam / tot; });
+    if (!live) return;
     const int j = threadIdx.x % G;
-    const bool active = !st->done[j];
-    const T alpha = (T)st->alpha[j];
-    double v[1] = {0.0};
-    for (int i = blockIdx.x * (kBlock / G) + threadIdx.x / G; i < n; i += gridDim.x * (kBlock / G)) {
-        if (!active) continue;
-        const size_t o = (size_t)i * G + j;
-        x[o] += alpha * p[o];
-        const T rr = r[o] - alpha * q[o];
-        r[o] = rr;
-        const T zz = JAC ? rr * invd[i] : rr;
-        v[0] += (double)(rr * zz);
-    }
-    group_partials<G, 1>(v, part);
-}
-
-// gamma_{k+1}, beta and the stopping test per active column; one block
-template <int G>
-__global__ void k_m_beta(MState* st, const double* __restrict__ part, int nb, int k)
-{
-    if (st->all_done) return;
-    double tot[G];
-    series_totals<G>(part, nb, tot);
-    if (threadIdx.x != 0) return;
-    int all = 1;
-    for (int j = 0; j < G; ++j) {
-        if (!st->done[j]) {
-            const double gnew = tot[j];
-            st->beta[j] = gnew / st->gam[k & 1][j];
-            st->gam[(k + 1) & 1][j] = gnew;
-            st->it[j] = k + 1;
-            st->res[j] = sqrt(fabs(gnew));
-            if (gnew != gnew) {
-                st->nan[j] = 1;
-                st->done[j] = 1;
-            } else if (gnew < st->thr[j]) {
-                st->converged[j] = 1;
-                st->done[j] = 1;
-            } else if (k + 1 >= st->maxit) {
-                st->done[j] = 1;
+    double v[1][1] = {};
+    if (!sc[j].done) {
+        const double alpha = sc[j].alpha;
+        for_elements<G>(n, [&](long o, long stride, long m) {
+            double rv[kMU], qv[kMU], dv[kMU];
+#pragma unroll
+            for (int u = 0; u < kMU; ++u) {
+                const long k = o + u * stride;
+                if (k < m) {
+                    rv[u] = r[k];
+                    qv[u] = q[k];
+                    dv[u] = JAC ? invd[k / G] : 1.0;
+                }
             }
-            // a column that stops here keeps its p: it is not used again
-            if (st->done[j]) st->beta[j] = 0.0;
-        }
-        all &= st->done[j];
+#pragma unroll
+            for (int u = 0; u < kMU; ++u) {
+                const long k = o + u * stride;
+                if (k < m) {
+                    const double rr = rv[u] - alpha * qv[u];
+                    r[k] = rr;
+                    v[0][0] += rr * (JAC ? rr * dv[u] : rr);
+                }
+            }
+        });
     }
-    st->all_done = all;
+    group_partials<G>(v, part);
 }
 
-// p = M^-1 r + beta p (updateP, linear_solver.cu:79-87) for the columns still active
-template <int G, typename T, bool JAC>
-__global__ void k_m_p(int n, T* __restrict__ p, const T* __restrict__ r, const T* __restrict__ invd, const MState* st)
+// gamma_{k+1}, beta and the stopping test per active column; x += alpha p; p = M^-1 r + beta p (updateP,
+// linear_solver.cu:79-87) for the columns still active
+template <int G, bool JAC>
+__global__ __launch_bounds__(kMBlock) void k_m_p(int n, double* __restrict__ x, double* __restrict__ p,
+                                                 const double* __restrict__ r, const double* __restrict__ invd,
+                                                 const MState* __restrict__ st, MState* __restrict__ out,
+                                                 const double* __restrict__ pb, int nb)
 {
-    if (st->all_done) return;
+    __shared__ MCol sc[G];
+    __shared__ int was[G];
+    const int maxit = st->maxit;
+    if (threadIdx.x < G) was[threadIdx.x] = st->col[threadIdx.x].done;
+    const bool live = scalar_step<G>(st, out, pb, nb, sc, [maxit](MCol& c, double gnew) {
+        c.beta = gnew / c.gam;
+        c.gam = gnew;
+        c.it += 1;
+        c.res = sqrt(fabs(gnew));
+        if (gnew != gnew) {
+            c.nan = 1;
+            c.done = 1;
+        } else if (gnew < c.thr) {
+            c.converged = 1;
+            c.done = 1;
+        } else if (c.it >= maxit) {
+            c.done = 1;
+        }
+    });
+    if (!live) return;
     const int j = threadIdx.x % G;
-    if (st->done[j]) return;
-    const T beta = (T)st->beta[j];
-    for (int i = blockIdx.x * (kBlock / G) + threadIdx.x / G; i < n; i += gridDim.x * (kBlock / G)) {
-        const size_t o = (size_t)i * G + j;
-        const T zz = JAC ? r[o] * invd[i] : r[o];
-        p[o] = zz + beta * p[o];
-    }
+    if (was[j]) return;
+    const bool on = !sc[j].done;   // a column that stops here keeps its p: it is not used again
+    const double alpha = sc[j].alpha, beta = sc[j].beta;
+    for_elements<G>(n, [&](long o, long stride, long m) {
+        double xv[kMU], pv[kMU], rv[kMU], dv[kMU];
+#pragma unroll
+        for (int u = 0; u < kMU; ++u) {
+            const long k = o + u * stride;
+            if (k < m) {
+                xv[u] = x[k];
+                pv[u] = p[k];
+                rv[u] = r[k];
+                dv[u] = JAC ? invd[k / G] : 1.0;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kMU; ++u) {
+            const long k = o + u * stride;
+            if (k < m) {
+                x[k] = xv[u] + alpha * pv[u];
+                if (on) p[k] = (JAC ? rv[u] * dv[u] : rv[u]) + beta * pv[u];
+            }
+        }
+    });
 }
 
 // ---- layout changes and refinement kernels
@@ -376,234 +468,204 @@ __global__ void k_m_unpack(int n, int ncol, const double* __restrict__ s, double
 // ---- reliable-update PCG (PFEM_PRECISION_MIXED)
 // r = b - A x (FP64), r_s = (float) r, p_s = D_s r_s, x_s = 0; partials (r, D r) and (b, D b) in FP64
 template <int G, bool JAC>
-__global__ __launch_bounds__(kBlock) void k_mr_init(int ntiles, const int* __restrict__ tiles, const int* __restrict__ rowptr,
+__global__ __launch_bounds__(kMBlock, 6) void k_mr_init(int ntiles, const int* __restrict__ tiles, const int* __restrict__ rowptr,
                                                     const int* __restrict__ col, const double* __restrict__ val,
                                                     const double* __restrict__ x, const double* __restrict__ b,
                                                     const double* __restrict__ invd, const float* __restrict__ invd32,
                                                     float* __restrict__ rs, float* __restrict__ ps, float* __restrict__ xs,
                                                     double* __restrict__ part)
 {
-    double v[2] = {0.0, 0.0};
-    for_tile_rows<G, double, double>(ntiles, tiles, rowptr, col, val, x, [&](int i, int j, double ax) {
+    constexpr int NC = kCols<G>;
+    using V = typename Columns<double, NC>::type;
+    using S = typename Columns<float, NC>::type;
+    double v[2][NC] = {};
+    for_tile_rows<G, double, double>(ntiles, tiles, rowptr, col, val, x, [&](int i, int j, V ax) {
         const size_t o = (size_t)i * G + j;
-        const double bb = b[o];
-        const double rr = bb - ax;
-        const float r32 = (float)rr;
-        rs[o] = r32;
-        ps[o] = JAC ? r32 * invd32[i] : r32;
-        xs[o] = 0.0f;
+        const V bb = *reinterpret_cast<const V*>(b + o);
+        const V rr = bb - ax;
         const double d = JAC ? invd[i] : 1.0;
-        v[0] += rr * (rr * d);
-        v[1] += bb * (bb * d);
+        const float d32 = JAC ? invd32[i] : 1.0f;
+        S r32;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            r32[c] = (float)rr[c];
+            v[0][c] += rr[c] * (rr[c] * d);
+            v[1][c] += bb[c] * (bb[c] * d);
+        }
+        *reinterpret_cast<S*>(rs + o) = r32;
+        *reinterpret_cast<S*>(ps + o) = JAC ? r32 * d32 : r32;
+        *reinterpret_cast<S*>(xs + o) = (S)0.0f;
     });
-    group_partials<G, 2>(v, part);
-}
-
-template <int G>
-__global__ void k_mr_begin(MState* st, const double* __restrict__ part, int nb)
-{
-    double tot[2 * G];
-    series_totals<2 * G>(part, nb, tot);
-    if (threadIdx.x != 0) return;
-    int all = 1;
-    for (int j = 0; j < G; ++j) {
-        const double rz = tot[j], bmb = tot[G + j];
-        st->thr[j] = st->tol_mode == PFEM_TOL_RELATIVE && bmb > 0.0 ? st->tol * st->tol * bmb : st->tol * st->tol;
-        st->rz[j] = st->rzmax[j] = rz;
-        st->res[j] = sqrt(fabs(rz));
-        st->it[j] = 0;
-        st->mode[j] = 0;
-        st->nrep[j] = 0;
-        st->nan[j] = rz != rz;
-        st->converged[j] = rz < st->thr[j] ? 1 : 0;
-        st->done[j] = j >= st->ncol || st->converged[j] || st->nan[j];
-        all &= st->done[j];
-    }
-    st->all_done = all;
+    group_partials<G>(v, part);
 }
 
 // Iterating columns: q_s = A_s p_s, partial (p_s, q_s). Columns due a replacement: r = b - A x with the
-// FP64 matrix, r_s = (float) r, partial (r, D r). The tile stages FP64 values only while some column is
-// being replaced ((float) of the FP64 value is the FP32 copy's value, so the FP32 products do not change).
+// FP64 matrix, r_s = (float) r, partial (r, D r). While some columns iterate and others are replaced both
+// products pass over the rows, each keeping its own columns.
 template <int G, bool JAC>
-__global__ __launch_bounds__(kBlock) void k_mr_spmv(int ntiles, const int* __restrict__ tiles, const int* __restrict__ rowptr,
+__global__ __launch_bounds__(kMBlock, 6) void k_mr_spmv(int ntiles, const int* __restrict__ tiles, const int* __restrict__ rowptr,
                                                     const int* __restrict__ col, const float* __restrict__ val32,
                                                     const double* __restrict__ val, const float* __restrict__ ps,
                                                     float* __restrict__ qs, const double* __restrict__ x,
                                                     const double* __restrict__ b, const double* __restrict__ invd,
-                                                    float* __restrict__ rs, const MState* st, double* __restrict__ part)
+                                                    float* __restrict__ rs, const MState* __restrict__ st,
+                                                    double* __restrict__ part)
 {
     if (st->all_done) return;
-    int anyrep = 0;
-    for (int c = 0; c < G; ++c) anyrep |= st->mode[c] == 1 && !st->done[c];
-    double v[1] = {0.0};
-    if (!anyrep) {
-        for_tile_rows<G, float, float>(ntiles, tiles, rowptr, col, val32, ps, [&](int i, int j, float ap) {
+    constexpr int NC = kCols<G>;
+    using V = typename Columns<double, NC>::type;
+    using S = typename Columns<float, NC>::type;
+    int rep = 0, iter = 0;   // columns, a bit each
+    for (int c = 0; c < G; ++c)
+        if (!st->col[c].done) (st->col[c].mode == 1 ? rep : iter) |= 1 << c;
+    double v[1][NC] = {};
+    if (iter)
+        for_tile_rows<G, float, float>(ntiles, tiles, rowptr, col, val32, ps, [&](int i, int j, S ap) {
             const size_t o = (size_t)i * G + j;
-            qs[o] = ap;
-            v[0] += (double)(ps[o] * ap);
+            *reinterpret_cast<S*>(qs + o) = ap;
+            const S pp = *reinterpret_cast<const S*>(ps + o);
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+                if (!((rep >> (j + c)) & 1)) v[0][c] += (double)(pp[c] * ap[c]);
         });
-    } else {
-        const int j = threadIdx.x % G;
-        const bool rep = st->mode[j] == 1;
-        __shared__ double sval[kMTileNnz];
-        __shared__ int scol[kMTileNnz];
-        const int nb = gridDim.x, bk = blockIdx.x;
-        const int rb = (bk % 8) * (nb / 8) + bk / 8;
-        const int t0 = (int)((long)ntiles * rb / nb), t1 = (int)((long)ntiles * (rb + 1) / nb);
-        for (int t = t0; t < t1; ++t) {
-            const int r0 = tiles[2 * t], r1 = tiles[2 * t + 1];
-            const int k0 = rowptr[r0], nk = rowptr[r1] - k0;
-            const bool staged = nk <= kMTileNnz;
-            if (staged) {
-                __syncthreads();
-                for (int k = threadIdx.x; k < nk; k += kBlock) {
-                    sval[k] = val[k0 + k];
-                    scol[k] = col[k0 + k];
+    if (rep)
+        for_tile_rows<G, double, double>(ntiles, tiles, rowptr, col, val, x, [&](int i, int j, V ax) {
+            const size_t o = (size_t)i * G + j;
+            const V bb = *reinterpret_cast<const V*>(b + o);
+            const double d = JAC ? invd[i] : 1.0;
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+                if ((rep >> (j + c)) & 1) {
+                    const double rr = bb[c] - ax[c];
+                    rs[o + c] = (float)rr;
+                    v[0][c] += rr * (rr * d);
                 }
-                __syncthreads();
-            }
-            for (int u = 0; u < kMRows; ++u) {
-                const int row = r0 + (int)threadIdx.x / G + u * (kBlock / G);
-                if (row >= r1) continue;
-                const size_t o = (size_t)row * G + j;
-                const int ka = rowptr[row], ke = rowptr[row + 1];
-                if (rep) {
-                    double ax = 0.0;
-                    for (int k = ka; k < ke; ++k) {
-                        const double a = staged ? sval[k - k0] : val[k];
-                        const int cc = staged ? scol[k - k0] : col[k];
-                        ax += a * x[(size_t)cc * G + j];
-                    }
-                    const double rr = b[o] - ax;
-                    rs[o] = (float)rr;
-                    v[0] += rr * (rr * (JAC ? invd[row] : 1.0));
-                } else {
-                    float ap = 0.0f;
-                    for (int k = ka; k < ke; ++k) {
-                        const float a = staged ? (float)sval[k - k0] : val32[k];
-                        const int cc = staged ? scol[k - k0] : col[k];
-                        ap += a * ps[(size_t)cc * G + j];
-                    }
-                    qs[o] = ap;
-                    v[0] += (double)(ps[o] * ap);
-                }
-            }
-        }
-    }
-    group_partials<G, 1>(v, part);
+        });
+    group_partials<G>(v, part);
 }
 
-// alpha = gamma / (p_s, q_s) for iterating columns; for a replaced column the true gamma: the stopping
-// test, then beta for the direction update; one block
-template <int G>
-__global__ void k_mr_alpha(MState* st, const double* __restrict__ part, int nb)
-{
-    if (st->all_done) return;
-    double tot[G];
-    series_totals<G>(part, nb, tot);
-    if (threadIdx.x != 0) return;
-    int all = 1;
-    for (int j = 0; j < G; ++j) {
-        if (!st->done[j]) {
-            if (st->mode[j] == 1) {
-                const double g = tot[j];
-                st->nrep[j] += 1;
-                st->res[j] = sqrt(fabs(g));
-                if (g != g) {
-                    st->nan[j] = 1;
-                    st->done[j] = 1;
-                } else if (g < st->thr[j]) {
-                    st->converged[j] = 1;
-                    st->done[j] = 1;
-                } else {
-                    st->beta[j] = g / st->rz[j];
-                    st->rz[j] = st->rzmax[j] = g;
-                    st->mode[j] = 2;
-                }
-            } else {
-                st->mode[j] = 0;
-                st->alpha[j] = st->rz[j] / tot[j];
-            }
-        }
-        all &= st->done[j];
-    }
-    st->all_done = all;
-}
-
-// x_s += alpha p_s, r_s -= alpha q_s for iterating columns (FP32); partial (r_s, D_s r_s)
+// Iterating columns: alpha = gamma / (p_s, q_s); r_s -= alpha q_s (FP32), partial (r_s, D_s r_s). A replaced
+// column has its true gamma: the stopping test, then beta for the direction update.
 template <int G, bool JAC>
-__global__ void k_mr_update(int n, float* __restrict__ xs, float* __restrict__ rs, const float* __restrict__ ps,
-                            const float* __restrict__ qs, const float* __restrict__ invd32, const MState* st,
-                            double* __restrict__ part)
+__global__ __launch_bounds__(kMBlock) void k_mr_update(int n, float* __restrict__ rs, const float* __restrict__ qs,
+                                                       const float* __restrict__ invd32, const MState* __restrict__ st,
+                                                       MState* __restrict__ out, const double* __restrict__ pa, int na,
+                                                       double* __restrict__ part)
 {
-    if (st->all_done) return;
+    __shared__ MCol sc[G];
+    const bool live = scalar_step<G>(st, out, pa, na, sc, [](MCol& c, double tot) {
+        if (c.mode == 1) {
+            c.nrep += 1;
+            c.res = sqrt(fabs(tot));
+            if (tot != tot) {
+                c.nan = 1;
+                c.done = 1;
+            } else if (tot < c.thr) {
+                c.converged = 1;
+                c.done = 1;
+            } else {
+                c.beta = tot / c.gam;
+                c.gam = c.rzmax = tot;
+                c.mode = 2;
+            }
+        } else {
+            c.mode = 0;
+            c.alpha = c.gam / tot;
+        }
+    });
+    if (!live) return;
     const int j = threadIdx.x % G;
-    const bool active = !st->done[j] && st->mode[j] == 0;
-    const float alpha = (float)st->alpha[j];
-    double v[1] = {0.0};
-    for (int i = blockIdx.x * (kBlock / G) + threadIdx.x / G; i < n && active; i += gridDim.x * (kBlock / G)) {
-        const size_t o = (size_t)i * G + j;
-        xs[o] += alpha * ps[o];
-        const float rr = rs[o] - alpha * qs[o];
-        rs[o] = rr;
-        v[0] += (double)(rr * (JAC ? rr * invd32[i] : rr));
+    double v[1][1] = {};
+    if (!sc[j].done && sc[j].mode == 0) {
+        const float alpha = (float)sc[j].alpha;
+        for_elements<G>(n, [&](long o, long stride, long m) {
+            float rv[kMU], qv[kMU], dv[kMU];
+#pragma unroll
+            for (int u = 0; u < kMU; ++u) {
+                const long k = o + u * stride;
+                if (k < m) {
+                    rv[u] = rs[k];
+                    qv[u] = qs[k];
+                    dv[u] = JAC ? invd32[k / G] : 1.0f;
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < kMU; ++u) {
+                const long k = o + u * stride;
+                if (k < m) {
+                    const float rr = rv[u] - alpha * qv[u];
+                    rs[k] = rr;
+                    v[0][0] += (double)(rr * (JAC ? rr * dv[u] : rr));
+                }
+            }
+        });
     }
-    group_partials<G, 1>(v, part);
+    group_partials<G>(v, part);
 }
 
 // gamma of the recursive residual: the iteration count, then either beta or a replacement (after a 10x
-// drop since the last one, or when the recursive residual passes the stopping test); one block
-template <int G>
-__global__ void k_mr_beta(MState* st, const double* __restrict__ part, int nb)
+// drop since the last one, or when the recursive residual passes the stopping test). x_s += alpha p_s and
+// p_s = D_s r_s + beta p_s (iterating columns; after a replacement the direction alone); a column due a
+// replacement moves its correction into the FP64 solution: x += x_s, x_s = 0.
+template <int G, bool JAC>
+__global__ __launch_bounds__(kMBlock) void k_mr_p(int n, float* __restrict__ ps, const float* __restrict__ rs,
+                                                  const float* __restrict__ invd32, double* __restrict__ x,
+                                                  float* __restrict__ xs, const MState* __restrict__ st,
+                                                  MState* __restrict__ out, const double* __restrict__ pb, int nb)
 {
-    if (st->all_done) return;
-    double tot[G];
-    series_totals<G>(part, nb, tot);
-    if (threadIdx.x != 0) return;
-    int all = 1;
-    for (int j = 0; j < G; ++j) {
-        if (!st->done[j] && st->mode[j] == 0) {
-            const double g = tot[j];
-            st->it[j] += 1;
-            if (g != g) {
-                st->nan[j] = 1;
-                st->done[j] = 1;
-            } else if (st->it[j] >= st->maxit) {
-                st->done[j] = 1;
-            } else if (g < st->thr[j] || g < st->drop * st->rzmax[j]) {
-                st->mode[j] = 1;
-            } else {
-                st->beta[j] = g / st->rz[j];
-                st->rz[j] = g;
+    __shared__ MCol sc[G];
+    __shared__ int was[G];
+    const int maxit = st->maxit;
+    const double drop = st->drop;
+    if (threadIdx.x < G) was[threadIdx.x] = st->col[threadIdx.x].done ? 2 : st->col[threadIdx.x].mode == 0;
+    const bool live = scalar_step<G>(st, out, pb, nb, sc, [maxit, drop](MCol& c, double g) {
+        if (c.mode != 0) return;
+        c.it += 1;
+        if (g != g) {
+            c.nan = 1;
+            c.done = 1;
+        } else if (c.it >= maxit) {
+            c.done = 1;
+        } else if (g < c.thr || g < drop * c.rzmax) {
+            c.mode = 1;
+        } else {
+            c.beta = g / c.gam;
+            c.gam = g;
+        }
+    });
+    if (!live) return;
+    const int j = threadIdx.x % G;
+    if (was[j] == 2) return;
+    const bool step = was[j] == 1;                        // x_s moves
+    const bool done = sc[j].done != 0, fold = !done && sc[j].mode == 1;
+    const float alpha = (float)sc[j].alpha, beta = (float)sc[j].beta;
+    for_elements<G>(n, [&](long o, long stride, long m) {
+        float xv[kMU], pv[kMU], rv[kMU], dv[kMU];
+#pragma unroll
+        for (int u = 0; u < kMU; ++u) {
+            const long k = o + u * stride;
+            if (k < m) {
+                xv[u] = step ? xs[k] : 0.0f;
+                pv[u] = ps[k];
+                rv[u] = rs[k];
+                dv[u] = JAC ? invd32[k / G] : 1.0f;
             }
         }
-        all &= st->done[j];
-    }
-    st->all_done = all;
-}
-
-// p_s = D_s r_s + beta p_s (iterating columns and after a replacement); a column due a replacement
-// first moves its correction into the FP64 solution: x += x_s, x_s = 0
-template <int G, bool JAC>
-__global__ void k_mr_p(int n, float* __restrict__ ps, const float* __restrict__ rs, const float* __restrict__ invd32,
-                       double* __restrict__ x, float* __restrict__ xs, const MState* st)
-{
-    if (st->all_done) return;
-    const int j = threadIdx.x % G;
-    if (st->done[j]) return;
-    const int mode = st->mode[j];
-    const float beta = (float)st->beta[j];
-    for (int i = blockIdx.x * (kBlock / G) + threadIdx.x / G; i < n; i += gridDim.x * (kBlock / G)) {
-        const size_t o = (size_t)i * G + j;
-        if (mode == 1) {
-            x[o] += (double)xs[o];
-            xs[o] = 0.0f;
-        } else {
-            const float zz = JAC ? rs[o] * invd32[i] : rs[o];
-            ps[o] = zz + beta * ps[o];
+#pragma unroll
+        for (int u = 0; u < kMU; ++u) {
+            const long k = o + u * stride;
+            if (k < m) {
+                const float xn = step ? xv[u] + alpha * pv[u] : 0.0f;
+                if (fold) {
+                    x[k] += (double)xn;
+                    xs[k] = 0.0f;
+                } else {
+                    if (step) xs[k] = xn;
+                    if (!done) ps[k] = (JAC ? rv[u] * dv[u] : rv[u]) + beta * pv[u];
+                }
+            }
         }
-    }
+    });
 }
 
 // x += x_s over every column (a converged column's x_s is zero: its last replacement folded it in)
@@ -622,7 +684,7 @@ __global__ void k_m_to32(long n, float* __restrict__ d, const double* __restrict
 // ---- host side
 struct MultiWork {
     int n = 0, G = 0, ncol = 0;
-    const Pattern* pat = nullptr;
+    std::shared_ptr<Pattern> pat;
     DevArray<int> tiles;                // row tiles of the products (for_tile_rows)
     int ntiles = 0;
     DevArray<double> x, b, r, p, q;    // FP64 interleaved (x, b also the refinement's solution and RHS)
@@ -640,118 +702,27 @@ struct MultiWork {
 };
 
 // Grid of a row-tile kernel: as many workgroups as are resident at once (occupancy per CU times the
-// CUs), at most kMGrid. Each workgroup takes a contiguous range of tiles, so with the whole grid resident
-// from the start no workgroup waits for a second round (3D 8-RHS solve: FP64 298 -> 275 ms at 5
-// workgroups per CU, FP32 iterations 264 -> 205 ms at 7, against a fixed 2048).
+// CUs), at most kMGrid and one per tile. Each workgroup takes a contiguous range of tiles, so with the whole grid
+// resident from the start no workgroup waits for a second round.
 template <typename K>
-static int resident_grid(K kernel)
+static int resident_grid(K kernel, int ntiles)
 {
     int per_cu = 0, dev = 0, cus = 0;
-    PFEM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kernel), kBlock, 0));
+    PFEM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kernel), kMBlock, 0));
     PFEM_HIP(hipGetDevice(&dev));
     PFEM_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    return std::max(kBlock, std::min(kMGrid, per_cu * cus));
+    const int most = std::max(8, std::min(kMGrid, per_cu * cus) / 8 * 8);
+    return std::min(most, (ntiles + 7) / 8 * 8);
 }
 
-// One CG pass over the interleaved system (T = double: FP64 solve of b; T = float: inner FP32 solve from
-// x = 0). Ends with st copied to h[0].
-template <int G, typename T, typename VT>
-static void m_cg_run(Context* c, pfem_solver_t* s, MultiWork& w, const Pattern& P, const VT* val, const T* invd,
-                     T* x, const T* b, T* r, T* p, T* q, int x_zero, double tol, int tol_mode, int maxit, int ncol)
+// Polls the state every `batch` iterations until every column is done (or `slots` are spent), one batch ahead
+// of the copy it waits for. iterate() launches one iteration.
+template <typename F>
+static void m_iterate(Context* c, MultiWork& w, int batch, int slots, F iterate)
 {
-    const int n = P.n;
-    const bool jac = invd != nullptr;
-    MState init{};
-    init.tol = tol;
-    init.tol_mode = tol_mode;
-    init.maxit = maxit;
-    init.ncol = ncol;
-    PFEM_HIP(hipMemcpyAsync(w.st.p, &init, sizeof(MState), hipMemcpyHostToDevice, c->stream));
-    if (x_zero) PFEM_HIP(hipMemsetAsync(x, 0, sizeof(T) * (size_t)n * G, c->stream));
-    double* pa = w.part.p;
-    double* pb = w.part.p + (size_t)2 * G * kMGrid;
-    const dim3 gr(kMGrid), bl(kBlock);
-    const int ns = resident_grid(k_m_spmv<G, T, VT>);   // the tile kernels' grid
-    const dim3 gs(ns);
-    if (jac) hipLaunchKernelGGL((k_m_init<G, T, VT, true>), gs, bl, 0, c->stream, n, w.ntiles, w.tiles.p, P.rowptr.p, P.col.p, val, x, b, invd, r, p, pa, x_zero);
-    else hipLaunchKernelGGL((k_m_init<G, T, VT, false>), gs, bl, 0, c->stream, n, w.ntiles, w.tiles.p, P.rowptr.p, P.col.p, val, x, b, invd, r, p, pa, x_zero);
-    hipLaunchKernelGGL((k_m_begin<G>), dim3(1), bl, 0, c->stream, w.st.p, (const double*)pa, ns);
-    PFEM_HIP(hipGetLastError());
-    const int batch = s->poll;
-    int launched = 0, pend = -1, pend_launched = 0, slot = 0;
-    while (true) {
-        for (int jb = 0; jb < batch; ++jb) {
-            const int k = launched + jb;
-            hipLaunchKernelGGL((k_m_spmv<G, T, VT>), gs, bl, 0, c->stream, w.ntiles, w.tiles.p, P.rowptr.p, P.col.p, val, p, q, w.st.p, pa);
-            hipLaunchKernelGGL((k_m_alpha<G>), dim3(1), bl, 0, c->stream, w.st.p, (const double*)pa, ns, k);
-            if (jac) hipLaunchKernelGGL((k_m_update<G, T, true>), gr, bl, 0, c->stream, n, x, r, p, q, invd, w.st.p, pb);
-            else hipLaunchKernelGGL((k_m_update<G, T, false>), gr, bl, 0, c->stream, n, x, r, p, q, invd, w.st.p, pb);
-            hipLaunchKernelGGL((k_m_beta<G>), dim3(1), bl, 0, c->stream, w.st.p, (const double*)pb, kMGrid, k);
-            if (jac) hipLaunchKernelGGL((k_m_p<G, T, true>), gr, bl, 0, c->stream, n, p, r, invd, w.st.p);
-            else hipLaunchKernelGGL((k_m_p<G, T, false>), gr, bl, 0, c->stream, n, p, r, invd, w.st.p);
-        }
-        launched += batch;
-        PFEM_HIP(hipGetLastError());
-        PFEM_HIP(hipMemcpyAsync(w.h + slot, w.st.p, sizeof(MState), hipMemcpyDeviceToHost, c->stream));
-        PFEM_HIP(hipEventRecord(w.ev[slot], c->stream));
-        if (pend >= 0) {
-            PFEM_HIP(hipEventSynchronize(w.ev[pend]));
-            if (w.h[pend].all_done || pend_launched > maxit + batch) break;
-        }
-        pend = slot;
-        pend_launched = launched;
-        slot ^= 1;
-    }
-    PFEM_HIP(hipMemcpyAsync(w.h, w.st.p, sizeof(MState), hipMemcpyDeviceToHost, c->stream));
-    PFEM_HIP(hipStreamSynchronize(c->stream));
-}
-
-// Reliable-update PCG over the interleaved system (x, b in w.x, w.b); ends with the state in h[0]
-template <int G>
-static void m_ru_run(Context* c, pfem_solver_t* s, MultiWork& w, const Pattern& P, pfem_csr_t* a, bool jac)
-{
-    const int n = P.n;
-    const size_t m = (size_t)n * G;
-    if (!w.x32.p) {
-        w.x32.alloc(m); w.r32.alloc(m); w.p32.alloc(m); w.q32.alloc(m);
-    }
-    if (!a->val32.p) a->val32.alloc(P.nnz);
-    hipLaunchKernelGGL(k_m_to32, dim3(blocks_for(P.nnz)), dim3(kBlock), 0, c->stream, (long)P.nnz, a->val32.p, a->val.p);
-    const double* invd = jac ? s->pc->invd.p : nullptr;
-    const float* invd32 = jac ? s->pc->invd32.p : nullptr;
-    PFEM_REQUIRE(!jac || invd32, "FP32 Jacobi diagonal missing");
-    MState init{};
-    init.tol = s->tol;
-    init.tol_mode = s->tol_mode;
-    init.maxit = s->maxit;
-    init.ncol = w.ncol;
-    init.drop = std::pow(10.0, -s->replace_digits);
-    PFEM_HIP(hipMemcpyAsync(w.st.p, &init, sizeof(MState), hipMemcpyHostToDevice, c->stream));
-    double* pa = w.part.p;
-    double* pb = w.part.p + (size_t)2 * G * kMGrid;
-    float *xs = w.x32.p, *rs = w.r32.p, *ps = w.p32.p, *qs = w.q32.p;
-    const dim3 gr(kMGrid), bl(kBlock);
-    const int ns = jac ? resident_grid(k_mr_spmv<G, true>) : resident_grid(k_mr_spmv<G, false>);
-    const dim3 gs(ns);
-    if (jac) hipLaunchKernelGGL((k_mr_init<G, true>), gs, bl, 0, c->stream, w.ntiles, w.tiles.p, P.rowptr.p, P.col.p, a->val.p, (const double*)w.x.p, (const double*)w.b.p, invd, invd32, rs, ps, xs, pa);
-    else hipLaunchKernelGGL((k_mr_init<G, false>), gs, bl, 0, c->stream, w.ntiles, w.tiles.p, P.rowptr.p, P.col.p, a->val.p, (const double*)w.x.p, (const double*)w.b.p, invd, invd32, rs, ps, xs, pa);
-    hipLaunchKernelGGL((k_mr_begin<G>), dim3(1), bl, 0, c->stream, w.st.p, (const double*)pa, ns);
-    PFEM_HIP(hipGetLastError());
-    const int batch = s->poll;
     int launched = 0, pend = -1, slot = 0;
-    // a replacement takes one extra slot per tenfold residual drop; the slot budget allows for them
-    const int slots = s->maxit + s->maxit / 4 + 64;
     while (true) {
-        for (int jb = 0; jb < batch; ++jb) {
-            if (jac) hipLaunchKernelGGL((k_mr_spmv<G, true>), gs, bl, 0, c->stream, w.ntiles, w.tiles.p, P.rowptr.p, P.col.p, (const float*)a->val32.p, (const double*)a->val.p, (const float*)ps, qs, (const double*)w.x.p, (const double*)w.b.p, invd, rs, (const MState*)w.st.p, pa);
-            else hipLaunchKernelGGL((k_mr_spmv<G, false>), gs, bl, 0, c->stream, w.ntiles, w.tiles.p, P.rowptr.p, P.col.p, (const float*)a->val32.p, (const double*)a->val.p, (const float*)ps, qs, (const double*)w.x.p, (const double*)w.b.p, invd, rs, (const MState*)w.st.p, pa);
-            hipLaunchKernelGGL((k_mr_alpha<G>), dim3(1), bl, 0, c->stream, w.st.p, (const double*)pa, ns);
-            if (jac) hipLaunchKernelGGL((k_mr_update<G, true>), gr, bl, 0, c->stream, n, xs, rs, (const float*)ps, (const float*)qs, invd32, (const MState*)w.st.p, pb);
-            else hipLaunchKernelGGL((k_mr_update<G, false>), gr, bl, 0, c->stream, n, xs, rs, (const float*)ps, (const float*)qs, invd32, (const MState*)w.st.p, pb);
-            hipLaunchKernelGGL((k_mr_beta<G>), dim3(1), bl, 0, c->stream, w.st.p, (const double*)pb, kMGrid);
-            if (jac) hipLaunchKernelGGL((k_mr_p<G, true>), gr, bl, 0, c->stream, n, ps, (const float*)rs, invd32, w.x.p, xs, (const MState*)w.st.p);
-            else hipLaunchKernelGGL((k_mr_p<G, false>), gr, bl, 0, c->stream, n, ps, (const float*)rs, invd32, w.x.p, xs, (const MState*)w.st.p);
-        }
+        for (int jb = 0; jb < batch; ++jb) iterate();
         launched += batch;
         PFEM_HIP(hipGetLastError());
         PFEM_HIP(hipMemcpyAsync(w.h + slot, w.st.p, sizeof(MState), hipMemcpyDeviceToHost, c->stream));
@@ -763,8 +734,80 @@ static void m_ru_run(Context* c, pfem_solver_t* s, MultiWork& w, const Pattern& 
         pend = slot;
         slot ^= 1;
     }
+}
+
+static void m_state(Context* c, pfem_solver_t* s, MultiWork& w)
+{
+    MState init[2]{};
+    init[0].tol = s->tol;
+    init[0].tol_mode = s->tol_mode;
+    init[0].maxit = s->maxit;
+    init[0].ncol = w.ncol;
+    init[0].drop = std::pow(10.0, -s->replace_digits);
+    init[1] = init[0];
+    PFEM_HIP(hipMemcpyAsync(w.st.p, init, sizeof init, hipMemcpyHostToDevice, c->stream));
+}
+
+// FP64 CG over the interleaved system. Ends with the state in h[0].
+template <int G, bool JAC>
+static void m_cg_run(Context* c, pfem_solver_t* s, MultiWork& w, const Pattern& P, pfem_csr_t* a)
+{
+    const int n = P.n;
+    const double* invd = JAC ? s->pc->invd.p : nullptr;
+    const double* val = a->val.p;
+    double *x = w.x.p, *b = w.b.p, *r = w.r.p, *p = w.p.p, *q = w.q.p;
+    MState *s0 = w.st.p, *s1 = w.st.p + 1;
+    m_state(c, s, w);
+    double* pa = w.part.p;
+    double* pb = w.part.p + (size_t)2 * G * kMGrid;
+    const int ni = resident_grid(k_m_init<G, JAC>, w.ntiles), ns = resident_grid(k_m_spmv<G>, w.ntiles);
+    const int nu = (int)std::min<long>(kMStream, ((long)n * G + kMBlock - 1) / kMBlock);
+    const dim3 bl(kMBlock);
+    hipLaunchKernelGGL((k_m_init<G, JAC>), dim3(ni), bl, 0, c->stream, w.ntiles, w.tiles.p, P.rowptr.p, P.col.p, val, x, b, invd, r, p, pa);
+    hipLaunchKernelGGL((k_m_begin<G>), dim3(1), bl, 0, c->stream, s0, (const double*)pa, ni);
+    PFEM_HIP(hipGetLastError());
+    m_iterate(c, w, s->poll, s->maxit, [&] {
+        hipLaunchKernelGGL((k_m_spmv<G>), dim3(ns), bl, 0, c->stream, w.ntiles, w.tiles.p, P.rowptr.p, P.col.p, val, p, q, s0, pa);
+        hipLaunchKernelGGL((k_m_update<G, JAC>), dim3(nu), bl, 0, c->stream, n, r, q, invd, s0, s1, (const double*)pa, ns, pb);
+        hipLaunchKernelGGL((k_m_p<G, JAC>), dim3(nu), bl, 0, c->stream, n, x, p, r, invd, s1, s0, (const double*)pb, nu);
+    });
+    PFEM_HIP(hipMemcpyAsync(w.h, w.st.p, sizeof(MState), hipMemcpyDeviceToHost, c->stream));
+    PFEM_HIP(hipStreamSynchronize(c->stream));
+}
+
+// Reliable-update PCG over the interleaved system (x, b in w.x, w.b); ends with the state in h[0]
+template <int G, bool JAC>
+static void m_ru_run(Context* c, pfem_solver_t* s, MultiWork& w, const Pattern& P, pfem_csr_t* a)
+{
+    const int n = P.n;
+    const size_t m = (size_t)n * G;
+    if (!w.x32.p) {
+        w.x32.alloc(m); w.r32.alloc(m); w.p32.alloc(m); w.q32.alloc(m);
+    }
+    if (!a->val32.p) a->val32.alloc(P.nnz);
+    hipLaunchKernelGGL(k_m_to32, dim3(blocks_for(P.nnz)), dim3(kBlock), 0, c->stream, (long)P.nnz, a->val32.p, a->val.p);
+    const double* invd = JAC ? s->pc->invd.p : nullptr;
+    const float* invd32 = JAC ? s->pc->invd32.p : nullptr;
+    PFEM_REQUIRE(!JAC || invd32, "FP32 Jacobi diagonal missing");
+    MState *s0 = w.st.p, *s1 = w.st.p + 1;
+    m_state(c, s, w);
+    double* pa = w.part.p;
+    double* pb = w.part.p + (size_t)2 * G * kMGrid;
+    float *xs = w.x32.p, *rs = w.r32.p, *ps = w.p32.p, *qs = w.q32.p;
+    const int ni = resident_grid(k_mr_init<G, JAC>, w.ntiles), ns = resident_grid(k_mr_spmv<G, JAC>, w.ntiles);
+    const int nu = (int)std::min<long>(kMStream, ((long)n * G + kMBlock - 1) / kMBlock);
+    const dim3 bl(kMBlock);
+    hipLaunchKernelGGL((k_mr_init<G, JAC>), dim3(ni), bl, 0, c->stream, w.ntiles, w.tiles.p, P.rowptr.p, P.col.p, a->val.p, (const double*)w.x.p, (const double*)w.b.p, invd, invd32, rs, ps, xs, pa);
+    hipLaunchKernelGGL((k_m_begin<G>), dim3(1), bl, 0, c->stream, s0, (const double*)pa, ni);
+    PFEM_HIP(hipGetLastError());
+    // a replacement takes one extra slot per tenfold residual drop; the slot budget allows for them
+    m_iterate(c, w, s->poll, s->maxit + s->maxit / 4 + 64, [&] {
+        hipLaunchKernelGGL((k_mr_spmv<G, JAC>), dim3(ns), bl, 0, c->stream, w.ntiles, w.tiles.p, P.rowptr.p, P.col.p, (const float*)a->val32.p, (const double*)a->val.p, (const float*)ps, qs, (const double*)w.x.p, (const double*)w.b.p, invd, rs, s0, pa);
+        hipLaunchKernelGGL((k_mr_update<G, JAC>), dim3(nu), bl, 0, c->stream, n, rs, (const float*)qs, invd32, s0, s1, (const double*)pa, ns, pb);
+        hipLaunchKernelGGL((k_mr_p<G, JAC>), dim3(nu), bl, 0, c->stream, n, ps, (const float*)rs, invd32, w.x.p, xs, s1, s0, (const double*)pb, nu);
+    });
     // columns still iterating at the slot limit keep their FP64 part; their FP32 correction is folded in
-    hipLaunchKernelGGL(k_mr_fold, dim3(blocks_for((long)m)), bl, 0, c->stream, (long)m, w.x.p, (const float*)xs);
+    hipLaunchKernelGGL(k_mr_fold, dim3(blocks_for((long)m)), dim3(kBlock), 0, c->stream, (long)m, w.x.p, (const float*)xs);
     PFEM_HIP(hipMemcpyAsync(w.h, w.st.p, sizeof(MState), hipMemcpyDeviceToHost, c->stream));
     PFEM_HIP(hipStreamSynchronize(c->stream));
 }
@@ -775,17 +818,17 @@ static void solve_multi_g(Context* c, pfem_solver_t* s, pfem_csr_t* a, int ncol,
 {
     const Pattern& P = *a->pat;
     const int n = P.n;
-    if (!s->multi || s->multi->G != G || s->multi->n != n || s->multi->pat != &P) {
+    if (!s->multi || s->multi->G != G || s->multi->n != n || s->multi->pat != a->pat) {
         s->multi.reset(new MultiWork());
         MultiWork& w = *s->multi;
         w.n = n;
         w.G = G;
-        w.pat = &P;
+        w.pat = a->pat;
         std::vector<int> tiles;
         for (int r = 0; r < n;) {
             int r1 = r;
             const int base = P.h_rowptr[r];
-            while (r1 < n && r1 - r < kMRows * kBlock / G && (P.h_rowptr[r1 + 1] - base <= kMTileNnz || r1 == r)) ++r1;
+            while (r1 < n && r1 - r < tile_rows<G> && (P.h_rowptr[r1 + 1] - base <= kMTileNnz || r1 == r)) ++r1;
             tiles.push_back(r);
             tiles.push_back(r1);
             r = r1;
@@ -795,7 +838,7 @@ static void solve_multi_g(Context* c, pfem_solver_t* s, pfem_csr_t* a, int ncol,
         const size_t m = (size_t)n * G;
         w.x.alloc(m); w.b.alloc(m); w.r.alloc(m); w.p.alloc(m); w.q.alloc(m);
         w.part.alloc((size_t)4 * G * kMGrid);
-        w.st.alloc(1);
+        w.st.alloc(2);
         PFEM_HIP(hipHostMalloc((void**)&w.h, 2 * sizeof(MState), hipHostMallocDefault));
         for (hipEvent_t& e : w.ev) PFEM_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     }
@@ -808,24 +851,18 @@ static void solve_multi_g(Context* c, pfem_solver_t* s, pfem_csr_t* a, int ncol,
     hipLaunchKernelGGL((k_m_pack<G, double>), dim3(gp), dim3(kBlock), 0, c->stream, n, ncol, (const double*)X, w.x.p);
     hipLaunchKernelGGL((k_m_pack<G, double>), dim3(gp), dim3(kBlock), 0, c->stream, n, ncol, B, w.b.p);
     std::vector<pfem_solve_stats> st(ncol);
-    if (s->precision != PFEM_PRECISION_MIXED) {
-        m_cg_run<G, double, double>(c, s, w, P, a->val.p, jac ? s->pc->invd.p : nullptr, w.x.p, w.b.p, w.r.p, w.p.p,
-                                    w.q.p, 0, s->tol, s->tol_mode, s->maxit, ncol);
-        for (int j = 0; j < ncol; ++j) {
-            st[j].converged = w.h->converged[j];
-            st[j].iterations = w.h->it[j];
-            st[j].final_residual = w.h->res[j];
-            st[j].nan_detected = w.h->nan[j];
-        }
-    } else {
-        m_ru_run<G>(c, s, w, P, a, jac);
-        for (int j = 0; j < ncol; ++j) {
-            st[j].converged = w.h->converged[j];
-            st[j].iterations = w.h->it[j];
-            st[j].final_residual = w.h->res[j];
-            st[j].nan_detected = w.h->nan[j];
-            st[j].refinements = w.h->nrep[j];
-        }
+    const bool mixed = s->precision == PFEM_PRECISION_MIXED;
+    if (mixed && jac) m_ru_run<G, true>(c, s, w, P, a);
+    else if (mixed) m_ru_run<G, false>(c, s, w, P, a);
+    else if (jac) m_cg_run<G, true>(c, s, w, P, a);
+    else m_cg_run<G, false>(c, s, w, P, a);
+    for (int j = 0; j < ncol; ++j) {
+        const MCol& e = w.h->col[j];
+        st[j].converged = e.converged;
+        st[j].iterations = e.it;
+        st[j].final_residual = e.res;
+        st[j].nan_detected = e.nan;
+        if (mixed) st[j].refinements = e.nrep;
     }
     hipLaunchKernelGGL((k_m_unpack<G>), dim3(gp), dim3(kBlock), 0, c->stream, n, ncol, (const double*)w.x.p, X);
     PFEM_HIP(hipGetLastError());
