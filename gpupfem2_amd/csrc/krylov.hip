@@ -14,6 +14,7 @@
 #include "device.hpp"
 #include "internal.hpp"
 #include "resident.hpp"
+#include "resident_ic0.hpp"
 #include "solver.hpp"
 #include "spmv.hpp"
 #include "sync.hpp"
@@ -720,6 +721,16 @@ static void cg_run(Context* c, pfem_solver_t* s, const KArgs<T>& A, CgState* st,
         hipLaunchKernelGGL((k_cg_start<T>), dim3(g), dim3(kBlock), 0, c->stream, n, A.r, A.z, A.p, A.b, t, s->pa);
     }
     hipLaunchKernelGGL(k_cg_begin, dim3(1), dim3(kBlock), 0, c->stream, st, (const double*)s->pa, nb0);
+    // The iterations as one launch (resident_ic0.hip): up to 262144 rows (256 workgroups of 1024) with at most 12
+    // neighbours each, which is the quicker at every size that fits: 11.4 us an iteration against 26.0 at 13k rows,
+    // 13.5 against 31.4 at 256k.
+    if constexpr (sizeof(T) == 8)
+        if (xp_in_sweep && A.pc->contiguous && A.val == A.pc->aval.p) {
+            if (!s->resident_ic0) s->resident_ic0.reset(new ResidentIc0());
+            if (s->resident_ic0->plan(c, A.pc) &&
+                s->resident_ic0->solve(c, A.pc, A.pc_fp32, A.x, A.r, A.p, st, hst))
+                return;
+        }
     if (fused2) {
         hipLaunchKernelGGL((k_fill_sentinel<double>), dim3(blocks_for(P.ntiles)), dim3(kBlock), 0, c->stream,
                            (long)P.ntiles, s->pa);

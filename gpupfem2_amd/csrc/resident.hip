@@ -34,7 +34,7 @@
 #include "internal.hpp"
 #include "resident.hpp"
 #include "solver.hpp"
-#include "sync.hpp"
+#include "resident_wait.hpp"
 
 namespace pfem {
 
@@ -42,7 +42,6 @@ constexpr int kResLanes = 1024;            // rows and lanes of a workgroup
 constexpr int kResTiles = kResLanes / kBlock;
 constexpr int kResHalo = 2 * kResLanes;    // halo columns a workgroup can hold (two per lane)
 constexpr int kResTable = 4096;            // hash table for the halo's columns
-constexpr int kResPause = 64;              // solves that take the other path after a wait has failed
 
 template <typename T>
 struct ResArgs {
@@ -67,44 +66,7 @@ struct ResArgs {
     double drop;             // reliable updates: replacement after gamma fell by this factor
 };
 
-// Values the first poll does not find are polled until they are published, the limit is reached or another
-// workgroup has given up.
-template <typename T>
-__device__ __forceinline__ T res_await(typename Sentinel<T>::U* q, typename Sentinel<T>::U v, int* err, long limit,
-                                       int* fail)
-{
-    constexpr typename Sentinel<T>::U sent = Sentinel<T>::bits;
-    for (long spins = 0; v == sent; ++spins) {
-        if (spins >= limit ||
-            ((spins & 1023) == 1023 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
-            *fail = 1;
-            __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            break;
-        }
-        // workgroups of a batch's next system may wait for its last ones to start: they must not crowd the
-        // fabric that the running systems exchange through
-        if (spins >= 16) __builtin_amdgcn_s_sleep(16);
-        v = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    return __builtin_bit_cast(T, v);
-}
-
 __device__ __forceinline__ unsigned res_hash(int c) { return ((unsigned)c * 2654435761u) >> 20; }   // 12 bits
-
-// A value that is the same in every lane, kept in scalar registers
-__device__ __forceinline__ double uniform(double t)
-{
-    const unsigned long long u = __builtin_bit_cast(unsigned long long, t);
-    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(u >> 32));
-    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)u);
-    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
-
-// ((v0 + v1) + v2) + v3 of lanes i .. i + 3 (within 16), in lane i: the order block_sum adds its waves in
-__device__ __forceinline__ double sum4(double v)
-{
-    return ((v + lane_down<1>(v)) + lane_down<2>(v)) + lane_down<3>(v);
-}
 
 struct ResShared {
     double wave[2 * (kResLanes / 64)];   // wave sums

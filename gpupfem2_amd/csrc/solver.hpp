@@ -60,6 +60,10 @@ __device__ __forceinline__ int slot_col(int e, const int* __restrict__ col32, co
 }
 
 struct MultiWork;   // multi-RHS PCG work space (multi.hip)
+struct ResidentIc0;
+struct ResidentIc0Deleter {
+    void operator()(ResidentIc0* w) const;
+};
 struct MultiWorkDeleter {
     void operator()(MultiWork* w) const;
 };
@@ -283,6 +287,7 @@ struct pfem_solver_t {
     std::unique_ptr<pfem::MultiWork, pfem::MultiWorkDeleter> multi;   // pfem_solver_solve_multi
     std::unique_ptr<pfem::BatchWork, pfem::BatchWorkDeleter> batch;   // pfem_solver_solve_batched
     std::unique_ptr<pfem::ResidentWork, pfem::ResidentWorkDeleter> resident;   // single-launch Jacobi PCG
+    std::unique_ptr<pfem::ResidentIc0, pfem::ResidentIc0Deleter> resident_ic0;
     std::vector<int> batch_tiling;   // {row bound, tile rows, tile non-zeros} per size bucket (empty: defaults)
     pfem::DevArray<pfem::CgState> cg;
     pfem::DevArray<pfem::GmState> gm;
