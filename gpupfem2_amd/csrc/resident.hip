@@ -419,6 +419,12 @@ Kernel<T> kernel_for(int width, bool jac, bool rel, bool two_per_cu)
 }
 }  // namespace
 
+std::mutex& resident_mutex(int device)
+{
+    static std::mutex m[64];
+    return m[device & 63];
+}
+
 int resident_blocks(int rows) { return (rows + kResLanes - 1) / kResLanes; }
 
 bool ResidentWork::plan(Context* c, std::shared_ptr<Pattern> p, const std::vector<int>& rows, bool single)
@@ -515,6 +521,7 @@ bool ResidentWork::solve(Context* c, const T* val, const T* invd, const T* b, T*
     a.x_zero = x_zero ? 1 : 0;
     a.drop = drop;
     T* keep = reinterpret_cast<T*>(zbuf.p) + 3 * (size_t)P.n;
+    std::lock_guard<std::mutex> alone(resident_mutex(c->device));
     const long nfill = std::max({3L * P.n, 4L * tiles, (long)nsys});
     hipLaunchKernelGGL(k_resident_prepare<T>, dim3(blocks_for(nfill)), dim3(kBlock), 0, c->stream, 3L * P.n,
                        reinterpret_cast<typename Sentinel<T>::U*>(zbuf.p), 4L * tiles, a.ring, nsys, out.p, err.p,

@@ -476,7 +476,9 @@ static bool launch(Context* c, ResidentIc0& w, pfem_precond_t* pc, const TS* f, 
     a.st = st;
     a.out = w.out.p;
     a.err = w.err.p;
-    a.limit = pc->spin_limit / 4;   // 18 ms at the default of 65536 and about 1.1 us a poll
+    // 0.6 s at the default of 65536 and about 1.1 us a poll: other work on the device may hold back some of the
+    // workgroups, and the launch-per-kernel path's sums are grouped differently (other last bits)
+    a.limit = 8L * pc->spin_limit;
     const long nfill = std::max({4L * w.places, 4L * w.blocks, 1L});
     hipLaunchKernelGGL(k_ic0_arm, dim3(blocks_for(nfill)), dim3(kBlock), 0, c->stream, 4L * w.places,
                        reinterpret_cast<unsigned long long*>(w.buf.p), 4 * w.blocks, a.ring, w.err.p);
@@ -493,6 +495,7 @@ bool ResidentIc0::solve(Context* c, pfem_precond_t* pc, bool reduced, double* x,
         --pause;
         return false;
     }
+    std::lock_guard<std::mutex> alone(resident_mutex(c->device));
     const bool half = reduced && pc->factor_bits == 16 && pc->half_ok;
     const bool ran = half ? launch<_Float16>(c, *this, pc, pc->split16.p, pc->scale16.p, x, r, p, st)
                      : reduced ? launch<float>(c, *this, pc, pc->split32.p, nullptr, x, r, p, st)

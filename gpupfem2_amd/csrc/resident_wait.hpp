@@ -1,10 +1,17 @@
 // Device helpers of the solves that run as one launch (resident.hip, resident_ic0.hip).
 #pragma once
 
+#include <mutex>
+
 #include "device.hpp"
 #include "sync.hpp"
 
 namespace pfem {
+
+// Held from the launch of such a solve to its end: the workgroups of two of them (two threads, two contexts of one
+// process) could otherwise share the device so that neither is complete, and both would wait out their limits.
+// One after the other they take no longer, since each of them waits rather than computes.
+std::mutex& resident_mutex(int device);
 
 constexpr int kResPause = 64;   // solves that take the other path after a wait has failed
 
