@@ -412,13 +412,30 @@ __global__ __launch_bounds__(kBlock) void k_gm_arnoldi_spmv(const int* __restric
     if (row < r1) w[row] = JAC ? av * invd[row] : av;
 }
 
-// partials of (V_{i0+t}, w), t < cnt <= 8, stored as coefficient i0+t of part
+// One system's part in the kernels of an Arnoldi step, which take one or two systems of n rows (blockIdx.z)
 template <typename T>
-__global__ void k_gm_multidot(int n, const T* __restrict__ V, long ld, int i0, int cnt, const T* __restrict__ w,
-                              const GmState* st, double* __restrict__ part)
+struct GmSys {
+    T* V;
+    T* x;
+    GmState* st;
+    double *pb, *pn;
+};
+template <typename T>
+struct GmPair {
+    int n;
+    GmSys<T> sys[2];
+};
+
+// partials of (V_i, w), i <= j, w = V_{j+1}, stored as coefficient i of pb; blockIdx.y takes eight of them
+template <typename T>
+__global__ void k_gm_multidot(GmPair<T> a, int j)
 {
     __shared__ double sh[8][kWaves];
-    if (st->cycle_done) return;
+    const GmSys<T> S = a.sys[blockIdx.z];
+    if (S.st->cycle_done) return;
+    const int n = a.n, i0 = 8 * blockIdx.y, cnt = min(8, j + 1 - i0);
+    const T* __restrict__ V = S.V + (size_t)i0 * n;
+    const T* __restrict__ w = S.V + (size_t)(j + 1) * n;
     double v[8];
 #pragma unroll
     for (int t = 0; t < 8; ++t) v[t] = 0.0;
@@ -426,7 +443,7 @@ __global__ void k_gm_multidot(int n, const T* __restrict__ V, long ld, int i0, i
         const T wi = w[i];
 #pragma unroll
         for (int t = 0; t < 8; ++t)
-            if (t < cnt) v[t] += (double)(V[(size_t)(i0 + t) * ld + i] * wi);
+            if (t < cnt) v[t] += (double)(V[(size_t)t * n + i] * wi);
     }
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
 #pragma unroll
@@ -441,16 +458,19 @@ __global__ void k_gm_multidot(int n, const T* __restrict__ V, long ld, int i0, i
         const int t = threadIdx.x;
         double s = sh[t][0];
         for (int w2 = 1; w2 < kWaves; ++w2) s += sh[t][w2];
-        part[(size_t)(i0 + t) * gridDim.x + blockIdx.x] = s;
+        S.pb[(size_t)(i0 + t) * gridDim.x + blockIdx.x] = s;
     }
 }
 
 // block i sums the partials of coefficient i: hc_i, and h_{i,j} stored (pass 0) or corrected (pass 1)
-__global__ void k_gm_reduce_h(GmState* st, const double* __restrict__ part, int nb, int pass)
+template <typename T>
+__global__ void k_gm_reduce_h(GmPair<T> a, int nb, int pass)
 {
+    const GmSys<T> S = a.sys[blockIdx.z];
+    GmState* st = S.st;
     if (st->cycle_done) return;
     double tot[1];
-    sum_partials<1>(part + (size_t)blockIdx.x * nb, nb, tot);
+    sum_partials<1>(S.pb + (size_t)blockIdx.x * nb, nb, tot);
     if (threadIdx.x == 0) {
         const int i = blockIdx.x;
         double* h = st->H + (size_t)st->k * st->m;
@@ -461,61 +481,108 @@ __global__ void k_gm_reduce_h(GmState* st, const double* __restrict__ part, int 
 
 // w -= sum_i hc_i V_i (i <= j); on the last pass also the partials of ||w||^2
 template <typename T>
-__global__ void k_gm_orth(int n, const T* __restrict__ V, long ld, T* __restrict__ w, const GmState* st,
-                          double* __restrict__ pn, int last_pass)
+__global__ void k_gm_orth(GmPair<T> a, int j, int last_pass)
 {
     __shared__ double hc[kMaxRestart + 1];
-    if (st->cycle_done) return;
-    const int j = st->k;
-    for (int i = threadIdx.x; i <= j; i += blockDim.x) hc[i] = st->hc[i];
+    const GmSys<T> S = a.sys[blockIdx.z];
+    if (S.st->cycle_done) return;
+    const int n = a.n;
+    const T* __restrict__ V = S.V;
+    T* __restrict__ w = S.V + (size_t)(j + 1) * n;
+    for (int i = threadIdx.x; i <= j; i += blockDim.x) hc[i] = S.st->hc[i];
     __syncthreads();
     double v[1] = {0.0};
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         T wi = w[i];
-        for (int t = 0; t <= j; ++t) wi -= (T)hc[t] * V[(size_t)t * ld + i];
+        constexpr int kU = 8;
+        for (int t0 = 0; t0 <= j; t0 += kU) {   // eight loads in flight, subtracted in order
+            T b[kU];
+#pragma unroll
+            for (int u = 0; u < kU; ++u)
+                if (t0 + u <= j) b[u] = V[(size_t)(t0 + u) * n + i];
+#pragma unroll
+            for (int u = 0; u < kU; ++u)
+                if (t0 + u <= j) wi -= (T)hc[t0 + u] * b[u];
+        }
         w[i] = wi;
         v[0] += (double)(wi * wi);
     }
-    if (last_pass) block_partials<1>(v, pn);
+    if (last_pass) block_partials<1>(v, S.pn);
 }
 
-// end of Arnoldi step j from the ||w||^2 partials (one block)
-__global__ void k_gm_finish(GmState* st, const double* __restrict__ pn, int nb)
-{
-    if (st->cycle_done) return;
-    double tot[1];
-    sum_partials<1>(pn, nb, tot);
-    if (threadIdx.x == 0) gm_arnoldi_finish(st, sqrt(tot[0]));
-}
-
-// y = H^-1 beta (cublasDtrsv, upper, non-unit; linear_solver.cu:508-511)
-__global__ void k_gm_solve_y(GmState* st)
-{
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    st->apply_update = (st->converged || st->restarted) && st->k > 0 && !st->nan ? 1 : 0;
-    if (!st->apply_update) return;
-    const int k = st->k, m = st->m;
-    for (int i = 0; i < k; ++i) st->y[i] = st->beta[i];
-    for (int i = k - 1; i >= 0; --i) {
-        double s = st->y[i];
-        for (int j = i + 1; j < k; ++j) s -= st->H[(size_t)m * j + i] * st->y[j];
-        st->y[i] = s / st->H[(size_t)m * i + i];
-    }
-}
-
-// x += V y (cublasDgemv with alpha = beta = 1; linear_solver.cu:513-514); clears cycle_done for a restart
+// End of Arnoldi step j: every workgroup adds the ||w||^2 partials for itself and divides its rows of w
+// (scaleVector with divide = true, linear_solver.cu:493); workgroup 0 moves the state on. A workgroup that finds
+// the cycle already ended by it leaves its rows of w as they are: nothing reads that vector any more.
 template <typename T>
-__global__ void k_gm_update_x(int n, const T* __restrict__ V, long ld, T* __restrict__ x, const GmState* st)
+__global__ void k_gm_finish(GmPair<T> a, int j, int nb)
+{
+    const GmSys<T> S = a.sys[blockIdx.z];
+    __shared__ int over;
+    if (threadIdx.x == 0) over = __hip_atomic_load(&S.st->cycle_done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (over) return;
+    double tot[1];
+    sum_partials<1>(S.pn, nb, tot);
+    const double norm = sqrt(tot[0]);
+    if (blockIdx.x == 0 && threadIdx.x == 0) gm_arnoldi_finish(S.st, norm);
+    T* __restrict__ w = S.V + (size_t)(j + 1) * a.n;
+    const T nrm = (T)norm;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += gridDim.x * blockDim.x) w[i] = w[i] / nrm;
+}
+
+// y = H^-1 beta (cublasDtrsv, upper, non-unit; linear_solver.cu:508-511). One chain of operations; its operands
+// wait in LDS, where they fit, rather than in memory (20 steps: 23.6 -> 15.2 us).
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_gm_solve_y(GmPair<T> a)
+{
+    constexpr int kK = 64;
+    __shared__ double h[kK * kK], b[kK];
+    GmState* st = a.sys[blockIdx.z].st;
+    const int k = st->k, m = st->m;
+    const bool apply = (st->converged || st->restarted) && k > 0 && !st->nan;
+    if (apply && k <= kK)
+        for (int t = threadIdx.x; t < k * k; t += kBlock) h[t] = st->H[(size_t)m * (t / k) + t % k];
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    st->apply_update = apply ? 1 : 0;
+    if (!apply) return;
+    double* y = k <= kK ? b : st->y;
+    const double* H = k <= kK ? h : st->H;
+    const size_t ld = k <= kK ? k : m;
+    for (int i = 0; i < k; ++i) y[i] = st->beta[i];
+    for (int i = k - 1; i >= 0; --i) {
+        double s = y[i];
+        for (int c = i + 1; c < k; ++c) s -= H[ld * c + i] * y[c];
+        y[i] = s / H[ld * i + i];
+    }
+    if (k <= kK)
+        for (int i = 0; i < k; ++i) st->y[i] = y[i];
+}
+
+// x += V y (cublasDgemv with alpha = beta = 1; linear_solver.cu:513-514)
+template <typename T>
+__global__ void k_gm_update_x(GmPair<T> a)
 {
     __shared__ double y[kMaxRestart];
-    if (!st->apply_update) return;
-    const int k = st->k;
-    for (int i = threadIdx.x; i < k; i += blockDim.x) y[i] = st->y[i];
+    const GmSys<T> S = a.sys[blockIdx.z];
+    if (!S.st->apply_update) return;
+    const int k = S.st->k, n = a.n;
+    const T* __restrict__ V = S.V;
+    for (int i = threadIdx.x; i < k; i += blockDim.x) y[i] = S.st->y[i];
     __syncthreads();
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         T s = 0;
-        for (int j = 0; j < k; ++j) s += V[(size_t)j * ld + i] * (T)y[j];
-        x[i] = s + x[i];
+        constexpr int kU = 8;
+        for (int j0 = 0; j0 < k; j0 += kU) {
+            T b[kU];
+#pragma unroll
+            for (int u = 0; u < kU; ++u)
+                if (j0 + u < k) b[u] = V[(size_t)(j0 + u) * n + i];
+#pragma unroll
+            for (int u = 0; u < kU; ++u)
+                if (j0 + u < k) s += b[u] * (T)y[j0 + u];
+        }
+        S.x[i] = s + S.x[i];
     }
 }
 
@@ -943,31 +1010,8 @@ struct GmresSys {
         if (jac()) hipLaunchKernelGGL((k_gm_arnoldi_spmv<T, true>), dim3(P.ntiles), dim3(kBlock), 0, c->stream, P.tiles.p, P.rowptr.p, P.col.p, A.val, v(j), A.invd, v(j + 1), st);
         else hipLaunchKernelGGL((k_gm_arnoldi_spmv<T, false>), dim3(P.ntiles), dim3(kBlock), 0, c->stream, P.tiles.p, P.rowptr.p, P.col.p, A.val, v(j), A.invd, v(j + 1), st);
     }
-    // the rest of Arnoldi step j: preconditioner (other than Jacobi), Gram-Schmidt, Givens, normalisation
-    void arnoldi_rest(int j)
-    {
-        const int nn = n();
-        const unsigned gg = g();
-        const long ld = nn;
-        T* w = v(j + 1);
-        if (!jac() && !none()) papply<T>(c, A, w, w);
-        const int passes = s->reorth ? 2 : 1;
-        for (int pass = 0; pass < passes; ++pass) {
-            for (int i0 = 0; i0 <= j; i0 += 8)
-                hipLaunchKernelGGL((k_gm_multidot<T>), dim3(gg), dim3(kBlock), 0, c->stream, nn, A.V, ld, i0, std::min(8, j + 1 - i0), w, st, s->pb);
-            hipLaunchKernelGGL(k_gm_reduce_h, dim3(j + 1), dim3(kBlock), 0, c->stream, st, (const double*)s->pb, (int)gg, pass);
-            hipLaunchKernelGGL((k_gm_orth<T>), dim3(gg), dim3(kBlock), 0, c->stream, nn, A.V, ld, w, st, s->pn, pass == passes - 1 ? 1 : 0);
-        }
-        hipLaunchKernelGGL(k_gm_finish, dim3(1), dim3(kBlock), 0, c->stream, st, (const double*)s->pn, (int)gg);
-        hipLaunchKernelGGL((k_gm_scale<T>), dim3(gg), dim3(kBlock), 0, c->stream, nn, w, st);
-    }
+    GmSys<T> part() const { return GmSys<T>{A.V, A.x, st, s->pb, s->pn}; }
     void read_state() { PFEM_HIP(hipMemcpyAsync(hst, st, sizeof(GmState), hipMemcpyDeviceToHost, c->stream)); }
-    // y = H^-1 beta, x += V y (when the cycle converged, or every cycle of GMRES(m))
-    void finish_cycle()
-    {
-        hipLaunchKernelGGL(k_gm_solve_y, dim3(1), dim3(64), 0, c->stream, st);
-        hipLaunchKernelGGL((k_gm_update_x<T>), dim3(g()), dim3(kBlock), 0, c->stream, n(), A.V, (long)n(), A.x, st);
-    }
     // after finish_cycle and a state read: true when the solve is over, else the next cycle is armed
     bool next_cycle()
     {
@@ -980,10 +1024,51 @@ struct GmresSys {
     }
 };
 
+// One system, or two of one size whose step then costs one sequence of launches: at 65k to 256k rows a launch of
+// these kernels is mostly its start and its tail. A step of two systems of 65k rows, FP32, was 21 launches of 2.3
+// to 4.0 us and the product; it is 7 of 2.5 to 4.6. One system of 256k rows, FP64, 20 steps: 827 -> 686 us.
+template <typename T>
+struct GmresStep {
+    Context* c = nullptr;
+    GmPair<T> a{};
+    int count = 0, passes = 1;
+    GmresSys<T>* sys[2] = {nullptr, nullptr};
+
+    void add(GmresSys<T>& g)
+    {
+        c = g.c;
+        a.n = g.n();
+        passes = g.s->reorth ? 2 : 1;
+        sys[count] = &g;
+        a.sys[count++] = g.part();
+    }
+    // the rest of Arnoldi step j: preconditioner (other than Jacobi), Gram-Schmidt, Givens, normalisation
+    void arnoldi_rest(int j)
+    {
+        const unsigned gg = vec_grid(a.n);
+        for (int q = 0; q < count; ++q)
+            if (!sys[q]->jac() && !sys[q]->none()) papply<T>(c, sys[q]->A, sys[q]->v(j + 1), sys[q]->v(j + 1));
+        for (int pass = 0; pass < passes; ++pass) {
+            hipLaunchKernelGGL((k_gm_multidot<T>), dim3(gg, j / 8 + 1, count), dim3(kBlock), 0, c->stream, a, j);
+            hipLaunchKernelGGL((k_gm_reduce_h<T>), dim3(j + 1, 1, count), dim3(kBlock), 0, c->stream, a, (int)gg, pass);
+            hipLaunchKernelGGL((k_gm_orth<T>), dim3(gg, 1, count), dim3(kBlock), 0, c->stream, a, j, pass == passes - 1 ? 1 : 0);
+        }
+        hipLaunchKernelGGL((k_gm_finish<T>), dim3(gg, 1, count), dim3(kBlock), 0, c->stream, a, j, (int)gg);
+    }
+    // y = H^-1 beta, x += V y (when the cycle converged, or every cycle of GMRES(m))
+    void finish_cycle()
+    {
+        hipLaunchKernelGGL((k_gm_solve_y<T>), dim3(1, 1, count), dim3(kBlock), 0, c->stream, a);
+        hipLaunchKernelGGL((k_gm_update_x<T>), dim3(vec_grid(a.n), 1, count), dim3(kBlock), 0, c->stream, a);
+    }
+};
+
 template <typename T>
 static void gmres_run(Context* c, pfem_solver_t* s, const KArgs<T>& A, GmState* st, GmState* hst)
 {
     GmresSys<T> g{c, s, A, st, hst};
+    GmresStep<T> step;
+    step.add(g);
     g.init();
     while (true) {
         g.cycle_start();
@@ -991,14 +1076,14 @@ static void gmres_run(Context* c, pfem_solver_t* s, const KArgs<T>& A, GmState* 
             const int j1 = std::min(s->m, j0 + s->poll);
             for (int j = j0; j < j1; ++j) {
                 g.spmv(j);
-                g.arnoldi_rest(j);
+                step.arnoldi_rest(j);
             }
             PFEM_HIP(hipGetLastError());
             g.read_state();
             PFEM_HIP(hipStreamSynchronize(c->stream));
             if (hst->cycle_done) break;
         }
-        g.finish_cycle();
+        step.finish_cycle();
         PFEM_HIP(hipGetLastError());
         g.read_state();
         PFEM_HIP(hipStreamSynchronize(c->stream));
@@ -1049,6 +1134,14 @@ static void gmres_run_pair(Context* c, GmresSys<T>& g0, GmresSys<T>& g1)
     while (!g0.done || !g1.done) {
         for (auto* x : g)
             if (!x->done) x->cycle_start();
+        // the systems still at work: in one sequence of launches if they are alike
+        std::vector<GmresStep<T>> steps;
+        for (auto* x : g)
+            if (!x->done) {
+                if (steps.empty() || g0.n() != g1.n() || g0.s->m != g1.s->m || g0.s->reorth != g1.s->reorth)
+                    steps.emplace_back();
+                steps.back().add(*x);
+            }
         const int m = std::max(g0.s->m, g1.s->m), poll = std::min(g0.s->poll, g1.s->poll);
         for (int j0 = 0; j0 < m; j0 += poll) {
             const int j1 = std::min(m, j0 + poll);
@@ -1068,8 +1161,8 @@ static void gmres_run_pair(Context* c, GmresSys<T>& g0, GmresSys<T>& g1)
                     for (auto* x : g)
                         if (!x->done && j < x->s->m) x->spmv(j);
                 }
-                for (auto* x : g)
-                    if (!x->done && j < x->s->m) x->arnoldi_rest(j);
+                for (auto& t : steps)
+                    if (j < t.sys[0]->s->m) t.arnoldi_rest(j);
             }
             PFEM_HIP(hipGetLastError());
             for (auto* x : g)
@@ -1077,8 +1170,7 @@ static void gmres_run_pair(Context* c, GmresSys<T>& g0, GmresSys<T>& g1)
             PFEM_HIP(hipStreamSynchronize(c->stream));
             if ((g0.done || g0.hst->cycle_done) && (g1.done || g1.hst->cycle_done)) break;
         }
-        for (auto* x : g)
-            if (!x->done) x->finish_cycle();
+        for (auto& t : steps) t.finish_cycle();
         PFEM_HIP(hipGetLastError());
         for (auto* x : g)
             if (!x->done) x->read_state();
