@@ -243,11 +243,15 @@ int pfem_pfem2_create(pfem_mesh2d m, pfem_particles ph, const pfem_step_config* 
         if (cfg->pred_solver == PFEM_SOLVER_GMRES)
             check(pfem_solver_set_option(s->s_pred, PFEM_SOLVER_OPT_GS_PASSES, cfg->pred_gs_passes == 2 ? 2 : 1),
                   s->ctx);
-        if (cfg->pred_solver == PFEM_SOLVER_GMRES && cfg->precision == PFEM_PRECISION_MIXED) {
-            // the second component's own solver: in mixed precision the two prediction systems are solved
-            // as a pair (pfem_solver_solve_pair: lockstep Arnoldi steps, one SpMV launch streaming the
-            // pattern once). In FP64 they run one after the other: there the pair measured slower
-            // (cylinder, 2M triangles: 6.75 against 6.20 ms per step; mixed: 5.44 against 5.77 ms).
+        if (cfg->pred_solver == PFEM_SOLVER_GMRES &&
+            (cfg->precision == PFEM_PRECISION_MIXED || cfg->pred_precond == PFEM_PRECOND_JACOBI ||
+             cfg->pred_precond == PFEM_PRECOND_NONE)) {
+            // the second component's own solver: the two prediction systems are solved as a pair
+            // (pfem_solver_solve_pair: lockstep Arnoldi steps in one launch sequence, one SpMV launch streaming
+            // the pattern once; the bits of two single solves). Prediction phase, ms a step in FP64, one after the other and as a
+            // pair: 1k nodes 1.45 and 0.73, 40k 0.95 and 0.56, 65k (cylinder, two outer iterations) 2.41 and 1.46,
+            // 1.01M 5.26 and 4.69. In FP64 an IC0/ILU0 prediction is solved one after the other: solve() repeats
+            // a solve whose sweeps have failed level by level.
             make_solver(s.get(), s->A1, cfg->pred_solver, cfg->pred_precond, PFEM_ORDER_NATURAL, &s->pc_pred1,
                         &s->s_pred1);
             check(pfem_solver_set_option(s->s_pred1, PFEM_SOLVER_OPT_GS_PASSES, cfg->pred_gs_passes == 2 ? 2 : 1),
