@@ -234,6 +234,21 @@ __device__ __forceinline__ bool substep(const CellField& f, double dts, double2&
     return true;
 }
 
+// The one cell of a wave's particles (c = -1: none), -1 if there are none, -2 if there are several; of one cell
+// also the particles' number and subcells
+__device__ __forceinline__ int one_cell(int c, uint32_t& bits, int& number)
+{
+    const unsigned long long here = __ballot(c >= 0);
+    if (!here) return -1;
+    const int one = __builtin_amdgcn_readlane(c, __ffsll(here) - 1);
+    if (!__all(c < 0 || c == one)) return -2;
+    number = __popcll(here);
+    if (c < 0) bits = 0u;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) bits |= __shfl_xor(bits, off, 64);
+    return one;
+}
+
 // The census of a wave's particles (c = -1: none)
 __device__ __forceinline__ void census(int c, uint32_t bits, int lane, uint32_t* __restrict__ mask, int* __restrict__ live)
 {
@@ -251,7 +266,8 @@ __device__ __forceinline__ void census(int c, uint32_t bits, int lane, uint32_t*
 }
 
 // Particles that leave their cell in substep s: {particle, s} into left_p / left_s, a range of kBlock per
-// workgroup, their number in left_n
+// workgroup, their number in left_n. A workgroup whose particles share one cell takes its census at once: the atomics
+// of a crowded cell all meet in one place (1M particles in one cell: 1.91 -> 0.18 ms).
 __global__ __launch_bounds__(kBlock) void k_advect(
     const long* __restrict__ pst, int substeps, double dts, const int* __restrict__ cell, double2* __restrict__ lam12,
     double* __restrict__ lam3, double2* __restrict__ pos, const int* __restrict__ tri, const double4* __restrict__ invJ,
@@ -259,7 +275,8 @@ __global__ __launch_bounds__(kBlock) void k_advect(
     uint32_t* __restrict__ mask, int* __restrict__ live, uint32_t* __restrict__ left_p, uint32_t* __restrict__ left_s,
     int* __restrict__ left_n)
 {
-    __shared__ int wn[kWaves];
+    __shared__ int wn[kWaves], wc[kWaves], wl[kWaves];
+    __shared__ uint32_t wb[kWaves];
     const long p = (long)blockIdx.x * kBlock + threadIdx.x;
     const long P = pst[0];
     if ((long)blockIdx.x * kBlock >= P) return;   // a whole workgroup past the count (the grid covers the capacity)
@@ -281,21 +298,40 @@ __global__ __launch_bounds__(kBlock) void k_advect(
         bits = 1u << subcell(L, step, l[0], l[1], l[2]);
     }
     const unsigned long long left = __ballot(leaves);
-    if (lane == 0) wn[wid] = __popcll(left);
+    const int stays = leaves ? -1 : c;
+    uint32_t subcells = bits;
+    int number = 0;
+    const int one = one_cell(stays, subcells, number);
+    if (lane == 0) {
+        wn[wid] = __popcll(left);
+        wc[wid] = one;
+        wl[wid] = number;
+        wb[wid] = subcells;
+    }
     __syncthreads();
-    int at = 0, all = 0;
+    int at = 0, all = 0, shared = -1;
+    number = 0;
+    subcells = 0u;
     for (int w = 0; w < kWaves; ++w) {
         if (w < wid) at += wn[w];
         all += wn[w];
+        if (wc[w] == -1) continue;
+        shared = shared == -1 || shared == wc[w] ? wc[w] : -2;
+        number += wl[w];
+        subcells |= wb[w];
     }
     if (threadIdx.x == 0) left_n[blockIdx.x] = all;
     if (leaves) {
         const size_t q = (size_t)blockIdx.x * kBlock + at + __popcll(left & ((1ull << lane) - 1ull));
         left_p[q] = (uint32_t)p;
         left_s[q] = (uint32_t)s;   // the substeps taken
-        c = -1;
     }
-    census(c, bits, lane, mask, live);
+    if (shared == -2) {
+        census(stays, bits, lane, mask, live);
+    } else if (threadIdx.x == 0 && shared >= 0) {
+        atomicOr(&mask[shared], subcells);
+        atomicAdd(&live[shared], number);
+    }
 }
 
 // One wave per RANGES lists of k_advect: four make full waves where few particles leave, one gives a set of
@@ -494,7 +530,9 @@ void exclusive_scan_int(Context* c, const int* in, int* out, long n, int* total_
 // among its cell's particles, which keeps their order stable and the result deterministic. Refilled
 // particles are written straight to their places, the last of their cell.
 constexpr int kTileOut = 1024;    // places a workgroup of k_reorder fills
-constexpr int kLongCell = 1024;   // more particles in a cell are ordered by k_order_long
+// More particles in a cell are ordered by k_order_long; ranking them is quadratic. A step of 2M particles, ranked and
+// ordered: 256 a cell 238 and 315 us, 400 a cell 276 and 332, 512 a cell 315 and 288, 1000 a cell 666 and 292.
+constexpr int kLongCell = 512;
 constexpr int kWindow = kTileOut + 2 * (kLongCell + 16);
 
 // 64-bit sums {places of a cell: low, refilled: high}: the tile-local exclusive prefixes and the tile sums
@@ -585,12 +623,15 @@ __global__ void k_cells(int nt, const long* __restrict__ pst, const int* __restr
     for (int p = first + n; p < last; ++p) order[p] = kRefill | (uint32_t)c;
 }
 
-// Every live particle takes a place of its cell: the lanes of a run of equal cells take theirs together
-// (kPlaceRuns waves' worth of particles per wave, so that their atomics overlap: 0.29 -> 0.19 ms for 53M)
+// Every live particle takes a place of its cell (in `list`, if k_order_long sorts the cell): the lanes of a run of
+// equal cells take theirs together
+// (kPlaceRuns waves' worth of particles per wave, so that their atomics overlap: 0.29 -> 0.19 ms for 53M). Of a
+// crowded cell's atomics, which all meet in one place, a wave makes one (1M particles in one cell: 1.16 -> 0.95 ms).
 constexpr int kPlaceRuns = 4;
 
 __global__ __launch_bounds__(kBlock) void k_place(const long* __restrict__ pst, const int* __restrict__ cell,
-                                                  int* __restrict__ cursor, uint32_t* __restrict__ order)
+                                                  const int* __restrict__ live, int* __restrict__ cursor,
+                                                  uint32_t* __restrict__ order, uint32_t* __restrict__ list)
 {
     const long P = pst[0];
     const int lane = threadIdx.x & 63;
@@ -599,6 +640,29 @@ __global__ __launch_bounds__(kBlock) void k_place(const long* __restrict__ pst, 
     int c[kPlaceRuns], at[kPlaceRuns], h[kPlaceRuns];
 #pragma unroll
     for (int r = 0; r < kPlaceRuns; ++r) c[r] = p0 + 64 * r < P ? cell[p0 + 64 * r] : -1;
+    // the cell of the first particle, if half of the wave's particles are in it: one atomic for all of them
+    const int first = __builtin_amdgcn_readfirstlane(c[0]);
+    unsigned long long in[kPlaceRuns];
+    int many = 0;
+#pragma unroll
+    for (int r = 0; r < kPlaceRuns; ++r) {
+        in[r] = __ballot(c[r] == first);
+        many += __popcll(in[r]);
+    }
+    if (first >= 0 && many >= 32 * kPlaceRuns) {
+        int base = 0;
+        if (lane == 0) base = atomicAdd(&cursor[first], many);
+        base = __builtin_amdgcn_readfirstlane(base);
+        uint32_t* __restrict__ const to = live[first] > kLongCell ? list : order;
+#pragma unroll
+        for (int r = 0; r < kPlaceRuns; ++r) {
+            if (c[r] == first) {
+                to[base + __popcll(in[r] & ((1ull << lane) - 1ull))] = (uint32_t)(p0 + 64 * r);
+                c[r] = -1;
+            }
+            base += __popcll(in[r]);
+        }
+    }
 #pragma unroll
     for (int r = 0; r < kPlaceRuns; ++r) {
         int length;
@@ -606,70 +670,127 @@ __global__ __launch_bounds__(kBlock) void k_place(const long* __restrict__ pst, 
         const unsigned long long heads = __ballot(head);
         h[r] = 63 - __clzll((long long)(heads & (~0ull >> (63 - lane))));   // this run's first lane
         at[r] = 0;
-        if (head && c[r] >= 0) at[r] = atomicAdd(&cursor[c[r]], length);
+        if (head && c[r] >= 0) {
+            const bool crowded = live[c[r]] > kLongCell;
+            at[r] = atomicAdd(&cursor[c[r]], length);
+            if (crowded) at[r] = ~at[r];
+        }
     }
 #pragma unroll
     for (int r = 0; r < kPlaceRuns; ++r) {
         const int a = __shfl(at[r], h[r], 64);
-        if (c[r] >= 0) order[a + lane - h[r]] = (uint32_t)(p0 + 64 * r);
+        if (c[r] < 0) continue;
+        if (a >= 0) order[a + lane - h[r]] = (uint32_t)(p0 + 64 * r);
+        else list[~a + lane - h[r]] = (uint32_t)(p0 + 64 * r);
     }
 }
 
-// Cells of more than kLongCell particles: their places' particles into ascending order, one workgroup per
-// cell (stable LSD radix sort, four 8-bit digits; `order` holds the result)
-__global__ __launch_bounds__(kBlock) void k_order_long(const int* __restrict__ counters, const int* __restrict__ long_cells,
-                                                       const int* __restrict__ start, const int* __restrict__ live,
-                                                       uint32_t* __restrict__ order, uint32_t* __restrict__ order2)
+// Cells of more than kLongCell particles: the particles that took their places (in `list`, in any order) into `order`
+// in ascending order. The particles' indices are distinct, so one bit each in LDS sorts them: a pass of a
+// workgroup marks those of one window of 2^kOrderShift indices, counts the smaller ones and writes the marked ones
+// out behind them. A cell's particles come from its own range of the array and its neighbours' ranges, mostly in
+// runs of consecutive indices: a run is marked at once, and windows without particles are passed over. Where
+// there are fewer such cells than workgroups, a team of workgroups takes a cell's windows in turn. 1M particles in
+// one cell: 13.2 -> 0.25 ms, against radix passes by one workgroup.
+constexpr int kOrderLanes = 1024, kOrderBlocks = 256, kOrderShift = 17;
+
+__global__ __launch_bounds__(kOrderLanes) void k_order_long(const int* __restrict__ counters,
+                                                            const int* __restrict__ long_cells,
+                                                            const int* __restrict__ start, const int* __restrict__ live,
+                                                            const uint32_t* __restrict__ list, uint32_t* __restrict__ order)
 {
-    __shared__ int base[kBlock];
-    __shared__ int wcnt[kWaves][kBlock];
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nlong = counters[2];
-    const unsigned long long lt = (1ull << lane) - 1ull;
-    for (int q = blockIdx.x; q < nlong; q += gridDim.x) {
-        const int c = long_cells[q], n = live[c];
-        uint32_t *src = order + start[c], *dst = order2 + start[c];
-        for (int shift = 0; shift < 32; shift += 8) {
-            base[threadIdx.x] = 0;
-            for (int w = 0; w < kWaves; ++w) wcnt[w][threadIdx.x] = 0;
-            __syncthreads();
-            for (int i = threadIdx.x; i < n; i += kBlock) atomicAdd(&base[(src[i] >> shift) & 255u], 1);
-            __syncthreads();
-            int total;
-            const int pre = block_exclusive_scan(base[threadIdx.x], &total);
-            base[threadIdx.x] = pre;
-            __syncthreads();
-            for (int i0 = 0; i0 < n; i0 += kBlock) {
-                const int i = i0 + (int)threadIdx.x;
-                const bool valid = i < n;
-                const uint32_t key = valid ? src[i] : 0u;
-                const uint32_t d = (key >> shift) & 255u;
-                unsigned long long peers = __ballot(valid);
+    constexpr int kW = kOrderLanes / 64, kWords = (1 << kOrderShift) / 64, kGroups = kWords / kOrderLanes;
+    constexpr int kU = 8;
+    __shared__ unsigned long long bits[kWords];
+    __shared__ uint32_t least;
+    __shared__ int below, wn[kW];
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, nlong = counters[2];
+    int teams = 1;
+    while (nlong > 0 && 2 * teams * nlong <= kOrderBlocks) teams *= 2;
+    const uint32_t turn = blockIdx.x & (teams - 1);
+    for (int q = blockIdx.x / teams; q < nlong; q += kOrderBlocks / teams) {
+        const int c = long_cells[q], n = live[c], first = start[c];
+        const uint32_t* __restrict__ src = list + first;
+        auto ours = [&](uint32_t key) { return ((key >> kOrderShift) & (teams - 1)) == turn; };
+        auto publish_least = [&](uint32_t m) {
 #pragma unroll
-                for (int b = 0; b < 8; ++b) {
-                    const bool bit = (d >> b) & 1u;
-                    const unsigned long long bal = __ballot(bit);
-                    peers &= bit ? bal : ~bal;
-                }
-                const int rank = __popcll(peers & lt);
-                if (valid && rank == 0) wcnt[wid][d] = __popcll(peers);
-                __syncthreads();
-                if (valid) {
-                    int off = base[d] + rank;
-                    for (int w = 0; w < wid; ++w) off += wcnt[w][d];
-                    dst[off] = key;
-                }
-                __syncthreads();
-                int sum = 0;
-                for (int w = 0; w < kWaves; ++w) {
-                    sum += wcnt[w][threadIdx.x];
-                    wcnt[w][threadIdx.x] = 0;
-                }
-                base[threadIdx.x] += sum;
-                __syncthreads();
+            for (int off = 32; off > 0; off >>= 1) m = min(m, (uint32_t)__shfl_down(m, off, 64));
+            if (lane == 0) atomicMin(&least, m);
+        };
+        __syncthreads();
+        if (tid == 0) least = ~0u;
+        __syncthreads();
+        uint32_t m = ~0u;
+        for (int i0 = tid; i0 < n; i0 += kU * kOrderLanes)
+#pragma unroll
+            for (int u = 0; u < kU; ++u) {
+                const int i = i0 + u * kOrderLanes;
+                const uint32_t key = src[min(i, n - 1)];
+                if (ours(key)) m = min(m, key);
             }
-            uint32_t* t = src;
-            src = dst;
-            dst = t;
+        publish_least(m);
+        __syncthreads();
+        while (least != ~0u) {
+            const uint32_t w0 = least >> kOrderShift << kOrderShift;
+            __syncthreads();
+            if (tid == 0) {
+                least = ~0u;
+                below = 0;
+            }
+            for (int w = tid; w < kWords; w += kOrderLanes) bits[w] = 0ull;
+            __syncthreads();
+            m = ~0u;
+            int smaller = 0;
+            for (int i0 = 0; i0 < n; i0 += kU * kOrderLanes) {
+                uint32_t keys[kU];
+#pragma unroll
+                for (int u = 0; u < kU; ++u) keys[u] = src[min(i0 + u * kOrderLanes + tid, n - 1)];
+#pragma unroll
+                for (int u = 0; u < kU; ++u) {
+                    const bool valid = i0 + u * kOrderLanes + tid < n;
+                    const uint32_t key = keys[u], d = key - w0;
+                    const bool in = valid && d < (1u << kOrderShift);
+                    if (valid && key < w0) ++smaller;
+                    else if (valid && !in && ours(key)) m = min(m, key);
+                    // runs of consecutive indices over the wave's lanes: the first lane marks its run
+                    const unsigned long long ins = __ballot(in);
+                    if (!ins) continue;
+                    const uint32_t before = __shfl_up(d, 1, 64);
+                    const bool head = in && (lane == 0 || !((ins >> (lane - 1)) & 1ull) || d != before + 1u);
+                    const unsigned long long stops = __ballot(head) | ~ins;
+                    if (head) {
+                        const unsigned long long after = lane < 63 ? stops >> (lane + 1) : 0ull;
+                        const int len = after ? __ffsll(after) : 64 - lane, at = (int)(d & 63u);
+                        const unsigned long long ones = ~0ull >> (64 - len);
+                        atomicOr(&bits[d >> 6], ones << at);
+                        if (at + len > 64) atomicOr(&bits[(d >> 6) + 1], ones >> (64 - at));
+                    }
+                }
+            }
+            publish_least(m);
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) smaller += __shfl_down(smaller, off, 64);
+            if (lane == 0) atomicAdd(&below, smaller);
+            __syncthreads();
+            // wave w's words: kGroups groups of 64 from 64 kGroups w on
+            int mine = 0;
+#pragma unroll
+            for (int g = 0; g < kGroups; ++g) mine += __popcll(bits[(wid * kGroups + g) * 64 + lane]);
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) mine += __shfl_down(mine, off, 64);
+            if (lane == 0) wn[wid] = mine;
+            __syncthreads();
+            int at = first + below;
+            for (int w = 0; w < wid; ++w) at += wn[w];
+            for (int g = 0; g < kGroups; ++g) {
+                const int b0 = (wid * kGroups + g) * 64;
+                for (unsigned long long some = __ballot(bits[b0 + lane] != 0ull); some; some &= some - 1ull) {
+                    const int w = b0 + __ffsll(some) - 1;
+                    const unsigned long long word = bits[w];
+                    if ((word >> lane) & 1ull) order[at + __popcll(word & ((1ull << lane) - 1ull))] = w0 + 64u * w + lane;
+                    at += __popcll(word);
+                }
+            }
         }
     }
 }
@@ -997,9 +1118,9 @@ void particles_advect_launch(pfem_particles_t* ph, int b, const double* u0, cons
     hipLaunchKernelGGL(k_cells, per_cell, bl, 0, c->stream, nt, pst, ph->live, ph->prefix.p, ph->tile_sums.p, ph->mask.p,
                        ph->ns, ph->cell_start.p, ph->cursor.p, ph->order.p, ph->tile_cell.p, ph->long_cells.p, ph->counters);
     hipLaunchKernelGGL(k_place, dim3(blocks_for(cap, kBlock * kPlaceRuns)), bl, 0, c->stream, pst, ph->cell[b].p,
-                       ph->cursor.p, ph->order.p);
-    hipLaunchKernelGGL(k_order_long, dim3(64), bl, 0, c->stream, ph->counters, ph->long_cells.p, ph->cell_start.p,
-                       ph->live, ph->order.p, ph->order2.p);
+                       ph->live, ph->cursor.p, ph->order.p, ph->order2.p);
+    hipLaunchKernelGGL(k_order_long, dim3(kOrderBlocks), dim3(kOrderLanes), 0, c->stream, ph->counters, ph->long_cells.p,
+                       ph->cell_start.p, ph->live, ph->order2.p, ph->order.p);
     hipLaunchKernelGGL(k_reorder, dim3(blocks_for(cap, kTileOut)), bl, 0, c->stream, ph->pst.p, ph->ns, ph->cell_start.p,
                        ph->live, ph->tile_cell.p, ph->order.p, ph->mask.p, ph->prefix.p, ph->tile_sums.p, m->xy.p, m->tri.p,
                        centers_of(ph), u0, u1, ph->cell[b].p, ph->lam12[b].p, ph->lam3[b].p, ph->pos[b].p, ph->vel[b].p,
