@@ -51,6 +51,7 @@ struct pfem_particles_t {
     // cells with more particles than a workgroup orders in LDS
     pfem::DevArray<uint32_t> order, order2;
     pfem::DevArray<int> tile_cell, long_cells, left_n;
+    pfem::DevArray<int> crowded, ncrowded;   // cells that k_proj_crowded sums
     pfem::DevArray<double> part;
     long deleted_last = 0, added_last = 0;
     // device state {count, next ID, deleted, added} of the last step, its pinned host copy and the event
@@ -923,21 +924,41 @@ __global__ void k_cell_start(const long* __restrict__ pst, const int* __restrict
 // Per cell the sums of l_i u, l_i v and l_i over its particles, in array order. A workgroup takes 64 cells
 // and streams their particles (consecutive in the arrays) through LDS in chunks with coalesced loads; wave
 // i sums shape function i of the cells on its lanes. A lane per cell that walks its particles in memory
-// instead reads 400 bytes away from its neighbours. 53M particles: 1.23 -> 0.47 ms.
-constexpr int kProjCells = 64, kProjChunk = 1024;
+// instead reads 400 bytes away from its neighbours. 53M particles: 1.23 -> 0.47 ms. Cells of more than kProjMany
+// particles are listed for k_proj_crowded: a chunk holds few of them, and most lanes would wait (2M particles, 4000
+// a cell: 19.2 ms, here 0.09). Half of the cells on either side of the line is the worst there is, so it lies where
+// that is no slower than a lane per cell: 2M particles, us with a line at 32, 64 and 128, all streamed, a lane
+// per cell: 64 a cell 68, 78, 57, 53, 76; 100 a cell 63, 71, 89, 85, 106; 128 a cell 60, 63, 125, 121, 130;
+// 200 a cell 55, 55, 65, 260, 192.
+constexpr int kProjCells = 64, kProjChunk = 1024, kProjMany = 128;
 
 __global__ __launch_bounds__(kBlock) void k_proj_cells(int nt, const int* __restrict__ start,
                                                        const double2* __restrict__ lam12,
                                                        const double* __restrict__ lam3, const double2* __restrict__ vel,
-                                                       double* __restrict__ part)
+                                                       double* __restrict__ part, int* __restrict__ crowded,
+                                                       int* __restrict__ ncrowded)
 {
     __shared__ double l[3][kProjChunk], vx[kProjChunk], vy[kProjChunk];
     const int lane = threadIdx.x & 63, i = threadIdx.x >> 6;
     const int c0 = blockIdx.x * kProjCells, c = c0 + lane;
+    const int s0 = c < nt ? start[c] : 0;
+    int s1 = c < nt ? start[c + 1] : 0;
+    const bool many = s1 - s0 > kProjMany;
+    if (many) {
+        if (i == 0) crowded[atomicAdd(ncrowded, 1)] = c;
+        s1 = s0;
+    }
+    const bool some = __any(many);
     const int p0 = start[c0], p1 = start[min(c0 + kProjCells, nt)];
-    const int s0 = c < nt ? start[c] : 0, s1 = c < nt ? start[c + 1] : 0;
     double sx = 0.0, sy = 0.0, w = 0.0;
     for (int b = p0; b < p1; b += kProjChunk) {
+        if (some) {   // on to the first particle of a cell that is summed here (every wave holds all the cells)
+            int next = s1 > b && s0 < s1 ? max(s0, b) : p1;
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) next = min(next, __shfl_xor(next, off, 64));
+            b = next;
+            if (b >= p1) break;
+        }
         const int m = min(kProjChunk, p1 - b);
 #pragma unroll
         for (int k = threadIdx.x; k < kProjChunk; k += kBlock)
@@ -961,7 +982,7 @@ __global__ __launch_bounds__(kBlock) void k_proj_cells(int nt, const int* __rest
         }
         __syncthreads();
     }
-    if (i < 3 && c < nt) {
+    if (i < 3 && c < nt && !many) {
         double* o = part + 9 * (size_t)c + 3 * i;
         o[0] = sx;
         o[1] = sy;
@@ -969,10 +990,72 @@ __global__ __launch_bounds__(kBlock) void k_proj_cells(int nt, const int* __rest
     }
 }
 
+// The listed cells, one to a wave: the particles pass through LDS, the next chunk's loads in flight, and nine lanes
+// add one sum each, in array order (w as l_i times one). The chain of additions bounds it: 7 ns a particle of the
+// largest cell.
+constexpr int kCrowdChunk = 256, kCrowdBlocks = 2048;
+
+__global__ __launch_bounds__(64) void k_proj_crowded(const int* __restrict__ ncrowded, const int* __restrict__ crowded,
+                                                     const int* __restrict__ start, const double2* __restrict__ lam12,
+                                                     const double* __restrict__ lam3, const double2* __restrict__ vel,
+                                                     double* __restrict__ part)
+{
+    constexpr int R = kCrowdChunk / 64, kU = 8;
+    __shared__ __align__(16) double l[3][kCrowdChunk], v[3][kCrowdChunk];
+    const int lane = threadIdx.x, n = *ncrowded;
+    for (int q = blockIdx.x; q < n; q += kCrowdBlocks) {
+        const int c = crowded[q], s0 = start[c], s1 = start[c + 1];
+        double2 l12[R], vv[R];
+        double l3[R];
+        auto fetch = [&](int b) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int p = min(b + lane + 64 * r, s1 - 1);
+                l12[r] = lam12[p];
+                l3[r] = lam3[p];
+                vv[r] = vel[p];
+            }
+        };
+        fetch(s0);
+        double s = 0.0;
+        for (int b = s0; b < s1; b += kCrowdChunk) {
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int k = lane + 64 * r;
+                l[0][k] = l12[r].x;
+                l[1][k] = l12[r].y;
+                l[2][k] = l3[r];
+                v[0][k] = vv[r].x;
+                v[1][k] = vv[r].y;
+                v[2][k] = 1.0;
+            }
+            __syncthreads();
+            if (b + kCrowdChunk < s1) fetch(b + kCrowdChunk);
+            const int m = min(kCrowdChunk, s1 - b);
+            if (lane < 9) {
+                const double *lp = l[lane / 3], *vp = v[lane % 3];
+                int k = 0;
+                for (; k + kU <= m; k += kU) {
+                    double t[kU];
+#pragma unroll
+                    for (int u = 0; u < kU; ++u) t[u] = lp[k + u] * vp[k + u];
+#pragma unroll
+                    for (int u = 0; u < kU; ++u) s += t[u];
+                }
+                for (; k < m; ++k) s += lp[k] * vp[k];
+            }
+        }
+        if (lane < 9) part[9 * (size_t)c + lane] = s;
+    }
+}
+
 __global__ void k_proj_nodes(int nv, const int* __restrict__ inc_off, const int* __restrict__ inc_code,
-                             const double* __restrict__ part, double* __restrict__ u0, double* __restrict__ u1)
+                             const double* __restrict__ part, double* __restrict__ u0, double* __restrict__ u1,
+                             int* __restrict__ ncrowded)
 {
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
+    if (v == 0) *ncrowded = 0;   // for the next projection
     if (v >= nv) return;
     double sx = 0.0, sy = 0.0, w = 0.0;
     for (int e = inc_off[v]; e < inc_off[v + 1]; ++e) {
@@ -1003,6 +1086,7 @@ static void alloc_state(pfem_particles_t* ph, long cap)
     ph->left_n.alloc(blocks);
     ph->tile_cell.alloc(cap / kTileOut + 2);
     ph->long_cells.alloc(cap / kLongCell + 1);
+    ph->crowded.alloc(cap / kProjMany + 1);
     ph->capacity = cap;
     ++ph->generation;
 }
@@ -1154,9 +1238,11 @@ void particles_project(pfem_particles_t* ph, double* u0, double* u1)
     pfem_mesh2d_t* m = ph->mesh;
     const int b = ph->cur;
     hipLaunchKernelGGL(k_proj_cells, dim3(blocks_for(m->nt, kProjCells)), dim3(kBlock), 0, c->stream, m->nt, ph->cell_start.p,
-                       ph->lam12[b].p, ph->lam3[b].p, ph->vel[b].p, ph->part.p);
+                       ph->lam12[b].p, ph->lam3[b].p, ph->vel[b].p, ph->part.p, ph->crowded.p, ph->ncrowded.p);
+    hipLaunchKernelGGL(k_proj_crowded, dim3(kCrowdBlocks), dim3(64), 0, c->stream, ph->ncrowded.p, ph->crowded.p,
+                       ph->cell_start.p, ph->lam12[b].p, ph->lam3[b].p, ph->vel[b].p, ph->part.p);
     hipLaunchKernelGGL(k_proj_nodes, dim3(blocks_for(m->nv)), dim3(kBlock), 0, c->stream, m->nv, m->inc.off.p,
-                       m->inc.code.p, ph->part.p, u0, u1);
+                       m->inc.code.p, ph->part.p, u0, u1, ph->ncrowded.p);
     PFEM_HIP(hipGetLastError());
 }
 
@@ -1218,9 +1304,11 @@ int pfem_particles_create(pfem_mesh2d m, int level, pfem_particles* out)
         ph->cell_start.alloc(m->nt + 1);
         ph->part.alloc(9 * (size_t)m->nt);
         ph->pst.alloc(8);
+        ph->ncrowded.alloc(1);
         PFEM_HIP(hipHostMalloc((void**)&ph->h_pst, 4 * sizeof(long), hipHostMallocDefault));
         PFEM_HIP(hipEventCreateWithFlags(&ph->pst_ev, hipEventDisableTiming));
         zero_async(c, ph->mask.p, ph->mask.bytes());
+        zero_async(c, ph->ncrowded.p, ph->ncrowded.bytes());
         alloc_state(ph.get(), 1024);
         put_device_state(c, ph.get());
         zero_async(c, ph->cell_start.p, ph->cell_start.bytes());   // no particles: every cell's range is empty

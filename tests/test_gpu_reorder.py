@@ -87,9 +87,10 @@ def best_of(ctx, call, prepare=lambda: None):
 
 def test_crowded_cells_cost(ctx):
     """1M particles: 100 in every cell, half of them in one cell, 4000 in every cell. With one workgroup that sorted a
-    crowded cell by radix passes the second set's step took 51 times the first's; now 3."""
+    crowded cell by radix passes the second set's step took 51 times the first's, now 3; with 64 cells to a
+    workgroup whatever they held the third's projection took 240 times the first's, now as long."""
     from gpupfem2_amd import capi, meshgen
-    step = []
+    step, projection = [], []
     for nx, ny, hot in ((100, 50, False), (100, 50, True), (16, 8, False)):
         xy, tri = meshgen.rectangle(0.0, 2.0, 0.0, 1.0, nx, ny, jitter=0.2, seed=1)
         nt = tri.shape[0]
@@ -99,5 +100,7 @@ def test_crowded_cells_cost(ctx):
         state = particles(xy, tri, count)
         u, v = ctx.to_device(0.2 / nx * np.cos(3.0 * xy[:, 1])), ctx.zeros(xy.shape[0])
         step.append(best_of(ctx, lambda: ph.advect(u, v, 0.1, 2), lambda: ph.set(state, state["cell"].size)))
-    print("crowded", step, flush=True)
+        projection.append(best_of(ctx, lambda: ph.project(u, v)))
+    print("crowded", step, projection, flush=True)
     assert max(step) < 10 * step[0], step
+    assert projection[2] < 10 * projection[0], projection
