@@ -154,14 +154,17 @@ __global__ __launch_bounds__(kBlock, 1) void k_band_sweep(BandArgs<TV, TS, TF> a
             }
         }
     } else if (wid > 0) {
-        // the halo in the order of its first use, 64 values to a wave
+        // The halo in the order of its first use, 64 values to a wave. All bands that fit the device start at once,
+        // so the wait of a band for its first value spans the chains of all bands before it: up to 8192 levels
+        // of 0.15 to 0.24 us each, 2 ms, for which it has another quarter of the limit, about 7 ms at the default.
+        const long limit = a.limit + (long)(a.limit / 4) * blockIdx.x;
         for (int h = tid - 64; h < nh; h += kBlock - 128) {
             U* const q = reinterpret_cast<U*>(mine + a.halo[h0 + h]);
-            int spins = 0;
+            long spins = 0;
             for (bool open = true; __any(open);) {
                 if (!open) continue;
                 U u = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (u == sent && spins++ < a.limit) continue;
+                if (u == sent && spins++ < limit) continue;
                 if (u == sent) {   // given up (the host reports it)
                     __hip_atomic_store(a.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     u = Sentinel<TF>::nan;

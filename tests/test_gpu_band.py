@@ -94,3 +94,22 @@ def test_band_solves(ctx, kind, solver, precision):
         assert st.converged
         x.append(d.download())
     assert np.linalg.norm(x[1] - x[0]) < 1e-8 * np.linalg.norm(x[0])
+
+
+@pytest.mark.parametrize("kind", [2, 3])
+def test_band_long_chain(ctx, kind):
+    """200000 levels in 25 bands that all start together: the last band waits 30 ms for its first value, more than the
+    default spin limit of one wait"""
+    from gpupfem2_amd import capi
+    print("band long chain", kind, flush=True)
+    a, keep = chain(ctx, 200000)
+    src = ctx.to_device(np.random.default_rng(3).standard_normal(a.n))
+    out = []
+    pc = capi.Preconditioner(a, kind, capi.ORDER_NATURAL)
+    pc.initialize(a)
+    for sweep in (True, False):
+        pc.set_sweep(sweep)
+        z = ctx.zeros(a.n)
+        pc.apply(z, src)
+        out.append(z.download())
+    assert np.array_equal(out[0], out[1])
