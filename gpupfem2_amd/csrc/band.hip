@@ -19,6 +19,7 @@
 // levels 1299 -> 187 us; tridiagonal, 8192 levels 13.2 -> 2.35 ms.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "band.hpp"
 #include "device.hpp"
@@ -246,117 +247,176 @@ __global__ __launch_bounds__(kBlock, 1) void k_band_sweep(BandArgs<TV, TS, TF> a
     }
 }
 
-// The slices with new factor values f, one lane per slot
+// Row i's entries of a triangle in the factor: strictly lower, or strictly upper
+__device__ __forceinline__ int2 band_entries(bool upper, int i, const int* __restrict__ rowptr, const int* __restrict__ diag)
+{
+    return upper ? make_int2(diag[i] + 1, rowptr[i + 1]) : make_int2(rowptr[i], diag[i]);
+}
+
+constexpr unsigned kBandZero = kBandRows + kBandHalo, kBandIdle = kBandZero + 1;   // places of unused entries and lanes
+
+// The planes of places, which only the pattern decides, one lane per slot
 template <typename TS, int W>
-__global__ void k_band_fill(int slots, const int* __restrict__ pos, const int* __restrict__ grow,
-                            const unsigned short* __restrict__ place, const int* __restrict__ diag,
-                            const TS* __restrict__ f, char* __restrict__ data)
+__global__ void k_band_places(long slots, int rows, bool upper, const int* __restrict__ row, const int* __restrict__ rowptr,
+                              const int* __restrict__ diag, const unsigned short* __restrict__ place,
+                              char* __restrict__ data)
 {
     using P = SlicePlanes<W, TS>;
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    const long s = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= slots) return;
     char* p = data + (size_t)(s >> 6) * P::bytes;
-    const int lane = s & 63;
-    constexpr int per = 16 / (int)sizeof(TS);
-    for (int k = 0; k < W; ++k) {
-        const int q = pos[(size_t)s * W + k];
-        reinterpret_cast<TS*>(p + 1024 * (k / per) + 16 * lane)[k % per] = q >= 0 ? f[q] : (TS)0;
+    const int lane = (int)(s & 63), i = row[s];
+    const int2 e = i >= 0 ? band_entries(upper, i, rowptr, diag) : make_int2(0, 0);
+    for (int k = 0; k < W; ++k)
         reinterpret_cast<unsigned*>(p + P::place + 1024 * (k / 4) + 16 * lane)[k % 4] =
-            8u * place[(size_t)s * (W + 1) + k];
-    }
-    reinterpret_cast<unsigned*>(p + P::row)[lane] = 8u * place[(size_t)s * (W + 1) + W];
-    const double d = grow[s] >= 0 ? (double)f[diag[grow[s]]] : 1.0;
+            8u * (e.x + k < e.y ? place[e.x + k] : kBandZero);
+    reinterpret_cast<unsigned*>(p + P::row)[lane] = 8u * (i >= 0 ? (unsigned)(i % rows) : kBandIdle);
+}
+
+// The other planes from the factor's values f
+template <typename TS, int W>
+__global__ void k_band_values(long slots, bool upper, const int* __restrict__ row, const int* __restrict__ rowptr,
+                              const int* __restrict__ diag, const TS* __restrict__ f, char* __restrict__ data)
+{
+    using P = SlicePlanes<W, TS>;
+    const long s = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= slots) return;
+    char* p = data + (size_t)(s >> 6) * P::bytes;
+    const int lane = (int)(s & 63), i = row[s];
+    constexpr int per = 16 / (int)sizeof(TS);
+    const int2 e = i >= 0 ? band_entries(upper, i, rowptr, diag) : make_int2(0, 0);
+    for (int k = 0; k < W; ++k)
+        reinterpret_cast<TS*>(p + 1024 * (k / per) + 16 * lane)[k % per] = e.x + k < e.y ? f[e.x + k] : (TS)0;
+    const double d = i >= 0 ? (double)f[diag[i]] : 1.0;
     double* o = reinterpret_cast<double*>(p + P::diag + 16 * lane);
     o[0] = d;
     o[1] = fabs(d) >= 0x1p-100 && fabs(d) <= 0x1p100 ? 1.0 / d : __builtin_nan("");
 }
 
-// ---- host side
-// One triangle (part 0 strictly lower, 1 strictly upper); false if a band's halo or a row does not fit.
-static bool build_triangle(Context* c, const Pattern& F, const std::vector<int>& lev, int part, int rows, int bands,
-                           BandTriangle& T, int& slices, int& max_halo)
+// f(W as a type) for the triangle's width
+template <typename F>
+static auto with_width(int width, F f)
 {
-    const int n = F.n;
-    auto k0 = [&](int i) { return part == 1 ? F.h_diag[i] + 1 : F.h_rowptr[i]; };
-    auto k1 = [&](int i) { return part == 0 ? F.h_diag[i] : F.h_rowptr[i + 1]; };
-    int width = 0;
-    for (int i = 0; i < n; ++i) width = std::max(width, k1(i) - k0(i));
-    if (width > 16) return false;
-    const int W = T.width = width <= 4 ? 4 : width <= 8 ? 8 : 16;
-    std::vector<int> soff(1, 0), hoff(1, 0), halo, pos, grow;
-    std::vector<unsigned short> at_all;
-    std::vector<int> place(n, -1), order, slice_of(n);
-    slices = max_halo = 0;
-    const unsigned short zero = kBandRows + kBandHalo, idle = zero + 1;
-    auto pad = [&](int slots) {
-        pos.resize((size_t)slots * W, -1);
-        for (size_t q = grow.size(); q < (size_t)slots; ++q) {
-            at_all.insert(at_all.end(), W, zero);
-            at_all.push_back(idle);
+    if (width == 4) return f(std::integral_constant<int, 4>());
+    if (width == 8) return f(std::integral_constant<int, 8>());
+    return f(std::integral_constant<int, 16>());
+}
+
+template <typename TS>
+static size_t slice_bytes(int width)
+{
+    return with_width(width, [](auto w) { return (size_t)SlicePlanes<decltype(w)::value, TS>::bytes; });
+}
+
+// ---- host side
+// One triangle (upper or lower) while it is planned
+struct BandPlan {
+    const Pattern& F;
+    const std::vector<int>& lev;
+    bool upper;
+    int rows, bands, width = 0;
+    std::vector<int> order;        // the rows of band b from b * rows on, by level, ascending within a level
+    std::vector<int> soff;         // slices of each band
+    int k0(int i) const { return upper ? F.h_diag[i] + 1 : F.h_rowptr[i]; }
+    int k1(int i) const { return upper ? F.h_rowptr[i + 1] : F.h_diag[i]; }
+    long slots() const { return 64L * (soff[bands] + 8); }   // the last band's loads run eight slices ahead
+
+    // false if a row does not fit
+    bool schedule()
+    {
+        const int n = F.n;
+        for (int i = 0; i < n; ++i) width = std::max(width, k1(i) - k0(i));
+        if (width > 16) return false;
+        width = width <= 4 ? 4 : width <= 8 ? 8 : 16;
+        std::vector<int> at(*std::max_element(lev.begin(), lev.end()) + 2, 0), by_level(n), next(bands);
+        for (int l : lev) ++at[l + 1];
+        for (size_t l = 1; l < at.size(); ++l) at[l] += at[l - 1];
+        for (int i = 0; i < n; ++i) by_level[at[lev[i]]++] = i;
+        order.resize(n);
+        for (int b = 0; b < bands; ++b) next[b] = b * rows;
+        for (int i : by_level) order[next[i / rows]++] = i;
+        soff.assign(1, 0);
+        for (int b = 0; b < bands; ++b) {
+            long slot = 0;
+            for (int o = b * rows; o < std::min(n, (b + 1) * rows); ++o, ++slot)
+                if (o > b * rows && lev[order[o]] != lev[order[o - 1]]) slot = (slot + 63) / 64 * 64;
+            soff.push_back(soff[b] + (int)((slot + 511) / 512 * 8));
         }
-        grow.resize(slots, -1);
-    };
-    for (int b = 0; b < bands; ++b) {
-        const int r0 = b * rows, r1 = std::min(n, r0 + rows);
-        order.resize(r1 - r0);
-        for (int i = r0; i < r1; ++i) order[i - r0] = i;
-        std::stable_sort(order.begin(), order.end(), [&](int u, int v) { return lev[u] < lev[v]; });
-        int slot = 64 * soff[b];
-        for (size_t o = 0; o < order.size(); ++o) {
-            if (o > 0 && lev[order[o]] != lev[order[o - 1]]) slot = (slot + 63) / 64 * 64;
-            pad(slot + 1);
-            const int i = order[o];
-            grow[slot] = i;
-            slice_of[i] = slot / 64 - soff[b];
-            at_all[(size_t)slot * (W + 1) + W] = (unsigned short)(i - r0);
-            for (int k = k0(i); k < k1(i); ++k) {
-                const int j = F.h_col[k];
-                int at = j - r0;
-                if (j < r0 || j >= r1) {
-                    if (place[j] < hoff[b]) {
-                        place[j] = (int)halo.size();
-                        halo.push_back(j);
+        return true;
+    }
+
+    // The triangle's tables; place: of every entry. False if a band's halo does not fit.
+    bool build(Context* c, BandTriangle& T, std::vector<unsigned short>& place) const
+    {
+        const int n = F.n;
+        std::vector<int> hoff(1, 0), halo, slot_row(slots(), -1), halo_at(n, -1), slice_of(n);
+        for (int b = 0; b < bands; ++b) {
+            const int r0 = b * rows, r1 = std::min(n, r0 + rows);
+            long slot = 64L * soff[b];
+            for (int o = r0; o < r1; ++o, ++slot) {
+                const int i = order[o];
+                if (o > r0 && lev[i] != lev[order[o - 1]]) slot = (slot + 63) / 64 * 64;
+                slot_row[slot] = i;
+                slice_of[i] = (int)(slot / 64) - soff[b];
+                for (int k = k0(i); k < k1(i); ++k) {
+                    const int j = F.h_col[k];
+                    int at = j - r0;
+                    if (j < r0 || j >= r1) {
+                        if (halo_at[j] < hoff[b]) {
+                            halo_at[j] = (int)halo.size();
+                            halo.push_back(j);
+                        }
+                        if (halo_at[j] - hoff[b] >= kBandHalo) return false;
+                        at = kBandRows + halo_at[j] - hoff[b];
                     }
-                    at = kBandRows + place[j] - hoff[b];
-                    if (place[j] - hoff[b] >= kBandHalo) return false;
+                    place[k] = (unsigned short)at;
                 }
-                pos[(size_t)slot * W + (k - k0(i))] = k;
-                at_all[(size_t)slot * (W + 1) + (k - k0(i))] = (unsigned short)at;
             }
-            ++slot;
+            hoff.push_back((int)halo.size());
         }
-        const int used = (slot + 63) / 64 - soff[b];
-        slices = std::max(slices, used);
-        soff.push_back(soff[b] + (used + 7) / 8 * 8);
-        pad(64 * soff[b + 1]);
-        hoff.push_back((int)halo.size());
-        max_halo = std::max(max_halo, hoff[b + 1] - hoff[b]);
+        // the rows other bands wait for, by the slice that solves them
+        std::vector<int> ooff(1, 0), out_at, mine;
+        std::vector<char> wanted(n, 0);
+        for (int j : halo) wanted[j] = 1;
+        for (int b = 0; b < bands; ++b) {
+            for (int o = b * rows; o < std::min(n, (b + 1) * rows); ++o)
+                if (wanted[order[o]]) out_at.insert(out_at.end(), {order[o] - b * rows, slice_of[order[o]]});
+            ooff.push_back((int)out_at.size() / 2);
+        }
+        if (out_at.empty()) out_at.push_back(0);
+        if (halo.empty()) halo.push_back(0);
+        T.width = width;
+        T.slots = slots();
+        upload(c, T.soff, soff);
+        upload(c, T.hoff, hoff);
+        upload(c, T.halo, halo);
+        upload(c, T.ooff, ooff);
+        upload(c, T.out_at, out_at);
+        upload(c, T.row, slot_row);
+        return true;
     }
-    pad(64 * (soff[bands] + 8));   // the last band's loads run ahead
-    // the rows other bands wait for, by the slice that solves them
-    std::vector<int> ooff(1, 0), out_at, mine;
-    std::vector<char> wanted(n, 0);
-    for (int j : halo) wanted[j] = 1;
-    for (int b = 0; b < bands; ++b) {
-        mine.clear();
-        for (int i = b * rows; i < std::min(n, (b + 1) * rows); ++i)
-            if (wanted[i]) mine.push_back(i);
-        std::stable_sort(mine.begin(), mine.end(), [&](int u, int v) { return slice_of[u] < slice_of[v]; });
-        for (int i : mine) out_at.insert(out_at.end(), {i - b * rows, slice_of[i]});
-        ooff.push_back((int)out_at.size() / 2);
-    }
-    if (out_at.empty()) out_at.push_back(0);
-    T.slices = soff[bands] + 8;
-    if (halo.empty()) halo.push_back(0);
-    upload(c, T.soff, soff);
-    upload(c, T.hoff, hoff);
-    upload(c, T.halo, halo);
-    upload(c, T.ooff, ooff);
-    upload(c, T.out_at, out_at);
-    upload(c, T.pos, pos);
-    upload(c, T.grow, grow);
-    upload(c, T.place, at_all);
-    return true;
+};
+
+template <typename TS>
+static void lay_out(Context* c, const BandSweeps& b, const Pattern& F, bool upper, DevArray<char>& data)
+{
+    const BandTriangle& t = upper ? b.upper : b.lower;
+    data.alloc((size_t)(t.slots / 64) * slice_bytes<TS>(t.width));
+    with_width(t.width, [&](auto w) {
+        hipLaunchKernelGGL((k_band_places<TS, decltype(w)::value>), dim3(blocks_for(t.slots)), dim3(kBlock), 0, c->stream,
+                           t.slots, b.rows, upper, t.row.p, F.rowptr.p, F.diag.p, b.place.p, data.p);
+    });
+}
+
+// A slice has 64 lanes however few rows of a level the band holds, so the slices grow with the levels times the
+// bands: 0.6 KB a row and triangle for a mesh of 1000 lines, 4.6 KB for a chain. They may take a sixteenth of the
+// device's memory (19 of 309 GB: meshes of 2500 lines, chains of 2M rows) and a quarter of what is free. Systems
+// beyond take the chunked sweeps, whose tables are the factor's size.
+static bool affordable(size_t bytes)
+{
+    size_t free = 0, total = 0;
+    PFEM_HIP(hipMemGetInfo(&free, &total));
+    return bytes <= std::min(total / 16, free / 4);
 }
 
 std::unique_ptr<BandSweeps> band_build(Context* c, const Pattern& F, const std::vector<int>& lev,
@@ -369,37 +429,42 @@ std::unique_ptr<BandSweeps> band_build(Context* c, const Pattern& F, const std::
     // levels (a random numbering: 18 levels at 65k rows) stay with the chunked sweeps, 103 us, which use the
     // whole chip for a level. The bound is the chunk size, where both have work for every workgroup.
     if (F.n / std::max(1, nlevels) > 256 * b->bands) return nullptr;
-    int sl = 0, su = 0, hl = 0, hu = 0;
-    if (!build_triangle(c, F, lev, 0, b->rows, b->bands, b->lower, sl, hl)) return nullptr;
-    if (!build_triangle(c, F, ulev, 1, b->rows, b->bands, b->upper, su, hu)) return nullptr;
-    b->max_halo = std::max(hl, hu);
+    BandPlan lower{F, lev, false, b->rows, b->bands}, upper{F, ulev, true, b->rows, b->bands};
+    if (!lower.schedule() || !upper.schedule()) return nullptr;
+    size_t bytes = 0;
+    for (const BandPlan* p : {&lower, &upper}) bytes += (size_t)(p->slots() / 64) * (slice_bytes<double>(p->width) + 256);
+    if (!affordable(bytes)) return nullptr;
+    std::vector<unsigned short> place(F.nnz, 0);
+    if (!lower.build(c, b->lower, place) || !upper.build(c, b->upper, place)) return nullptr;
+    upload(c, b->place, place);
+    lay_out<double>(c, *b, F, false, b->lower.data);
+    lay_out<double>(c, *b, F, true, b->upper.data);
     PFEM_HIP(hipStreamSynchronize(c->stream));
     return b;
 }
 
-template <typename TS, int W>
-static void fill(Context* c, const BandTriangle& t, const Pattern& F, const TS* f, DevArray<char>& data)
+bool band_refresh(Context* c, BandSweeps& b, const Pattern& F, const double* fac, const float* fac32)
 {
-    const int slots = 64 * t.slices;
-    if (!data.p) data.alloc((size_t)t.slices * SlicePlanes<W, TS>::bytes);
-    hipLaunchKernelGGL((k_band_fill<TS, W>), dim3(blocks_for(slots)), dim3(kBlock), 0, c->stream, slots, t.pos.p, t.grow.p,
-                       t.place.p, F.diag.p, f, data.p);
-}
-
-template <typename TS>
-static void fill(Context* c, const BandTriangle& t, const Pattern& F, const TS* f, DevArray<char>& data)
-{
-    if (t.width == 4) fill<TS, 4>(c, t, F, f, data);
-    else if (t.width == 8) fill<TS, 8>(c, t, F, f, data);
-    else fill<TS, 16>(c, t, F, f, data);
-}
-
-void band_refresh(Context* c, BandSweeps& b, const Pattern& F, const double* fac, const float* fac32)
-{
-    for (BandTriangle* t : {&b.lower, &b.upper}) {
-        fill<double>(c, *t, F, fac, t->data);
-        if (fac32) fill<float>(c, *t, F, fac32, t->data32);
+    if (fac32 && !b.lower.data32.p) {
+        size_t bytes = 0;
+        for (const BandTriangle* t : {&b.lower, &b.upper}) bytes += (size_t)(t->slots / 64) * slice_bytes<float>(t->width);
+        if (!affordable(bytes)) return false;
+        lay_out<float>(c, b, F, false, b.lower.data32);
+        lay_out<float>(c, b, F, true, b.upper.data32);
     }
+    for (bool upper : {false, true}) {
+        BandTriangle& t = upper ? b.upper : b.lower;
+        with_width(t.width, [&](auto w) {
+            constexpr int W = decltype(w)::value;
+            const dim3 g(blocks_for(t.slots)), bl(kBlock);
+            hipLaunchKernelGGL((k_band_values<double, W>), g, bl, 0, c->stream, t.slots, upper, t.row.p, F.rowptr.p,
+                               F.diag.p, fac, t.data.p);
+            if (fac32)
+                hipLaunchKernelGGL((k_band_values<float, W>), g, bl, 0, c->stream, t.slots, upper, t.row.p, F.rowptr.p,
+                                   F.diag.p, fac32, t.data32.p);
+        });
+    }
+    return true;
 }
 
 template <typename TV, typename TS, typename TF, bool UPPER, bool UNIT>
@@ -411,10 +476,10 @@ static void launch_triangle(Context* c, int bands, const BandTriangle& t, BandAr
     a.ooff = t.ooff.p;
     a.out_at = t.out_at.p;
     a.data = sizeof(TS) == 8 ? t.data.p : t.data32.p;
-    const dim3 g(bands), bl(kBlock);
-    if (t.width == 4) hipLaunchKernelGGL((k_band_sweep<TV, TS, TF, 4, UPPER, UNIT>), g, bl, 0, c->stream, a);
-    else if (t.width == 8) hipLaunchKernelGGL((k_band_sweep<TV, TS, TF, 8, UPPER, UNIT>), g, bl, 0, c->stream, a);
-    else hipLaunchKernelGGL((k_band_sweep<TV, TS, TF, 16, UPPER, UNIT>), g, bl, 0, c->stream, a);
+    with_width(t.width, [&](auto w) {
+        hipLaunchKernelGGL((k_band_sweep<TV, TS, TF, decltype(w)::value, UPPER, UNIT>), dim3(bands), dim3(kBlock), 0,
+                           c->stream, a);
+    });
 }
 
 template <typename TV, typename TS, typename TF>

@@ -12,27 +12,26 @@ namespace pfem {
 // (places as byte offsets).
 struct BandTriangle {
     int width = 0;                  // W: 4, 8 or 16 entries a row
-    int slices = 0;                 // padding included
+    long slots = 0;                 // lanes of all slices, padding included
     DevArray<int> soff, hoff;       // slice and halo ranges of each band (bands + 1)
     DevArray<int> halo;             // columns of other bands, in the order of their first use
     DevArray<int> ooff, out_at;     // {place, slice} of the rows other bands use, and each band's range of them
-    DevArray<int> pos;              // factor slot of entry k of slot s (64 s' + lane): pos[s W + k], -1 unused
-    DevArray<int> grow;             // row of each slot (-1 unused)
-    DevArray<unsigned short> place; // of entry k of slot s (s (W + 1) + k) and of the slot's own value (k = W)
+    DevArray<int> row;              // row of each slot (-1 unused)
     DevArray<char> data, data32;    // the slices with the FP64 factor and with its FP32 copy
 };
 
 struct BandSweeps {
-    int rows = 0, bands = 0, max_halo = 0;
+    int rows = 0, bands = 0;
     BandTriangle lower, upper;
+    DevArray<unsigned short> place; // of every factor entry's value in its band's LDS
 };
 
 // The plan of a factor pattern with its forward and backward levels, or null where the chunked sweeps are
-// the better form (large levels, a halo that does not fit).
+// the better form (large levels, a halo that does not fit, slices that take too much memory).
 std::unique_ptr<BandSweeps> band_build(Context* c, const Pattern& F, const std::vector<int>& lev,
                                        const std::vector<int>& ulev, int nlevels);
-// New factor values (fac32 may be null)
-void band_refresh(Context* c, BandSweeps& b, const Pattern& F, const double* fac, const float* fac32);
+// New factor values (fac32 may be null); false if the FP32 slices would take too much memory
+bool band_refresh(Context* c, BandSweeps& b, const Pattern& F, const double* fac, const float* fac32);
 // out = U^-1 L^-1 src (unit: L has a unit diagonal) through the published buffers sy and sw; part (or null)
 // receives the partials of (src, out), one per band. Returns the bands.
 template <typename TV, typename TS, typename TF>

@@ -1537,7 +1537,7 @@ void precond_initialize(Context* c, pfem_precond_t* pc, pfem_csr_t* a)
                                pc->sell_u.p);
         }
     }
-    if (pc->band) band_refresh(c, *pc->band, F, pc->fac.p, pc->fac32.p);
+    if (pc->band && !band_refresh(c, *pc->band, F, pc->fac.p, pc->fac32.p)) pc->band.reset();
     if (pc->split16.p) {
         // the scale from the largest factor entry, then c L in 16 bits
         const long nl = (long)pc->sell_l.n, nu = (long)pc->sell_u.n;

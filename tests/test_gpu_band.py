@@ -113,3 +113,18 @@ def test_band_long_chain(ctx, kind):
         pc.apply(z, src)
         out.append(z.download())
     assert np.array_equal(out[0], out[1])
+
+
+def test_band_memory(ctx):
+    """a chain of 2.6M rows: its slices would take 24 GB (the tables alone took 10); the sweeps take the form whose
+    tables are the factor's size"""
+    from gpupfem2_amd import capi
+    from test_gpu_resources import free_bytes
+    a, keep = chain(ctx, 2600000)
+    ctx.sync()
+    before = free_bytes()
+    pc = capi.Preconditioner(a, 2, capi.ORDER_NATURAL)
+    ctx.sync()
+    took = (before - free_bytes()) / 1e9
+    print("band memory", took, "GB", flush=True)
+    assert took < 1.0
