@@ -317,6 +317,7 @@ struct BandPlan {
     int rows, bands, width = 0;
     std::vector<int> order;        // the rows of band b from b * rows on, by level, ascending within a level
     std::vector<int> soff;         // slices of each band
+    double us = 0.0;               // of a solve, estimated
     int k0(int i) const { return upper ? F.h_diag[i] + 1 : F.h_rowptr[i]; }
     int k1(int i) const { return upper ? F.h_rowptr[i + 1] : F.h_diag[i]; }
     long slots() const { return 64L * (soff[bands] + 8); }   // the last band's loads run eight slices ahead
@@ -343,6 +344,29 @@ struct BandPlan {
             soff.push_back(soff[b] + (int)((slot + 511) / 512 * 8));
         }
         return true;
+    }
+
+    // The time of a solve from that of a slice and of a value's way to another band; bands run ahead of each other as
+    // far as their dependencies let them
+    void estimate()
+    {
+        const double slice = width == 4 ? 0.144 : width == 8 ? 0.174 : 0.238, hop = 1.2;
+        const int n = F.n;
+        std::vector<double> solved(n);
+        for (int q = 0; q < bands; ++q) {
+            const int r0 = (upper ? bands - 1 - q : q) * rows, r1 = std::min(n, r0 + rows);
+            double t = 0.0;
+            for (int o = r0; o < r1;) {
+                int end = o;   // of the slice
+                while (end < r1 && end - o < 64 && lev[order[end]] == lev[order[o]]) ++end;
+                for (int p = o; p < end; ++p)
+                    for (int k = k0(order[p]); k < k1(order[p]); ++k)
+                        if (const int j = F.h_col[k]; j < r0 || j >= r1) t = std::max(t, solved[j] + hop);
+                t += slice;
+                for (; o < end; ++o) solved[order[o]] = t;
+            }
+            us = std::max(us, t);
+        }
     }
 
     // The triangle's tables; place: of every entry. False if a band's halo does not fit.
@@ -425,15 +449,19 @@ std::unique_ptr<BandSweeps> band_build(Context* c, const Pattern& F, const std::
     auto b = std::make_unique<BandSweeps>();
     b->bands = (F.n + kBandRows - 1) / kBandRows;
     b->rows = (F.n + b->bands - 1) / b->bands;
-    // A level of more rows than the bands have lanes takes several slices in turn in each of them: few large
-    // levels (a random numbering: 18 levels at 65k rows) stay with the chunked sweeps, 103 us, which use the
-    // whole chip for a level. The bound is the chunk size, where both have work for every workgroup.
-    if (F.n / std::max(1, nlevels) > 256 * b->bands) return nullptr;
     BandPlan lower{F, lev, false, b->rows, b->bands}, upper{F, ulev, true, b->rows, b->bands};
     if (!lower.schedule() || !upper.schedule()) return nullptr;
     size_t bytes = 0;
     for (const BandPlan* p : {&lower, &upper}) bytes += (size_t)(p->slots() / 64) * (slice_bytes<double>(p->width) + 256);
     if (!affordable(bytes)) return nullptr;
+    // The chunked sweeps use the whole chip for a level and take 1.06 to 1.6 us for a level of up to 7000 rows. A band
+    // takes a level's rows 64 at a time, and bands whose levels do not overlap follow one another, so large levels
+    // are slower here: us a solve in chunks and in bands (estimate), half bandwidths 2000 and 2001, 200k rows,
+    // 100 levels: 136 and 640 (384); 1000, 60k rows, 60 levels: 64 and 173 (130); 300, 200 levels: 177 and 170 (148);
+    // unit square of 40k rows, 401 levels: 650 and 80 (62); its numbering shuffled, 15 levels: 53 (62).
+    lower.estimate();
+    upper.estimate();
+    if (lower.us + upper.us > 2.0 * nlevels) return nullptr;
     std::vector<unsigned short> place(F.nnz, 0);
     if (!lower.build(c, b->lower, place) || !upper.build(c, b->upper, place)) return nullptr;
     upload(c, b->place, place);

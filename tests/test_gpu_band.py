@@ -128,3 +128,37 @@ def test_band_memory(ctx):
     took = (before - free_bytes()) / 1e9
     print("band memory", took, "GB", flush=True)
     assert took < 1.0
+
+
+def test_large_levels_cost(ctx):
+    """half bandwidths 2000 and 2001: 100 levels of 2000 rows, none of which overlaps another. A band would take
+    such a level 64 rows at a time (1.3 ms an apply); one launch per triangle must not be slower than one per
+    level, with the same bits"""
+    import time
+    from gpupfem2_amd import capi
+    n = 200000
+    i = np.arange(n)
+    col = np.stack([i - 2001, i - 2000, i, i + 2000, i + 2001], 1)
+    val = np.tile([-1.0, -1.0, 4.5, -1.0, -1.0], (n, 1))
+    keep = (col >= 0) & (col < n)
+    rowptr = np.concatenate([[0], np.cumsum(keep.sum(1))]).astype(np.int32)
+    a = capi.CSR(ctx, rowptr=rowptr, col=col[keep].astype(np.int32), val=val[keep])
+    pc = capi.Preconditioner(a, 2, capi.ORDER_NATURAL)
+    pc.initialize(a)
+    src = ctx.to_device(np.random.default_rng(1).standard_normal(n))
+    took, out = [], []
+    for sweep in (True, False):
+        pc.set_sweep(sweep)
+        z = ctx.zeros(n)
+        best = np.inf
+        for _ in range(5):
+            ctx.sync()
+            t = time.perf_counter()
+            pc.apply(z, src)
+            ctx.sync()
+            best = min(best, time.perf_counter() - t)
+        took.append(best)
+        out.append(z.download())
+    print("large levels", took, flush=True)
+    assert took[0] < took[1], took
+    assert np.array_equal(out[0], out[1])
