@@ -5,18 +5,17 @@ Each column is compared with a direct FP64 solve. The stopping test bounds the r
 r^T D^-1 r <= tol^2 b^T D^-1 b, and x - x* = A^-1 r, so |x - x*|_2 <= |A^-1|_2 max(D)^(1/2) tol (b^T D^-1 b)^(1/2);
 to that come the rounding of the recurrence and of the direct solve, 100 cond(A) eps |x*| together.
 """
+import time
+
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("mixed", [False, True])
-@pytest.mark.parametrize("nrhs", [1, 2, 3, 5, 8])
-@pytest.mark.parametrize("spokes", [7, 127, 128, 511, 512, 2046, 2300])
-def test_multi_tiles(ctx, oracle, spokes, nrhs, mixed):
+def wheel(ctx, spokes):
+    """the matrix of a fan of triangles, every fifth rim node held: its hub's row has spokes + 1 entries"""
     from gpupfem2_amd import capi
-    print("multi tiles", spokes, nrhs, mixed, flush=True)
     t = 2 * np.pi * np.arange(spokes) / spokes
     xy = np.ascontiguousarray(np.concatenate([[[0.0, 0.0]], np.stack([np.cos(t), np.sin(t)], 1)]))
     k = np.arange(spokes)
@@ -27,6 +26,17 @@ def test_multi_tiles(ctx, oracle, spokes, nrhs, mixed):
     capi.assemble_poisson2d(m, a, rhs, coeff=1.0, rhs_kind=2, rhs_param=0.0)
     fixed = np.arange(1, n, 5, dtype=np.int32)
     capi.Dirichlet(ctx, n, fixed, np.zeros(fixed.size)).apply(a, rhs, 1)
+    return m, a, fixed
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("nrhs", [1, 2, 3, 5, 8])
+@pytest.mark.parametrize("spokes", [7, 127, 128, 511, 512, 2046, 2300])
+def test_multi_tiles(ctx, oracle, spokes, nrhs, mixed):
+    from gpupfem2_amd import capi
+    print("multi tiles", spokes, nrhs, mixed, flush=True)
+    m, a, fixed = wheel(ctx, spokes)
+    n = spokes + 1
     rp, col, val = a.download()
     A = np.zeros((n, n))
     A[np.repeat(np.arange(n), np.diff(rp)), col] = val
@@ -49,3 +59,29 @@ def test_multi_tiles(ctx, oracle, spokes, nrhs, mixed):
                  + 100 * w[-1] / w[0] * 2.3e-16 * np.linalg.norm(want))
         assert np.linalg.norm(Xh[j, free] - want) <= bound, (j, np.linalg.norm(Xh[j, free] - want), bound)
         assert not Xh[j, fixed].any()
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+def test_multi_long_row_cost(ctx, mixed):
+    """a row of 2001 entries is staged, one of 5001 is not: walked by one lane it took 600 us a product"""
+    from gpupfem2_amd import capi
+    took = []
+    for spokes in (2000, 5000):
+        m, a, fixed = wheel(ctx, spokes)
+        b = np.random.default_rng(1).standard_normal(spokes + 1)
+        b[fixed] = 0.0
+        d = ctx.to_device(b)
+        s = capi.Solver(a, capi.SOLVER_CG, 1e-30, 60, 0, capi.TOL_RELATIVE, capi.Preconditioner(a, capi.PRECOND_JACOBI))
+        if mixed:
+            s.set_precision(capi.PRECISION_MIXED)
+        best = np.inf
+        for _ in range(4):
+            x = ctx.zeros(spokes + 1)
+            ctx.sync()
+            t = time.perf_counter()
+            st = s.solve_multi(a, x, d, 1)
+            ctx.sync()
+            best = min(best, (time.perf_counter() - t) / max(st[0].iterations, 1))
+        took.append(best)
+    print("multi long row", mixed, took, flush=True)
+    assert took[1] < 2 * took[0], took
