@@ -20,7 +20,7 @@ SOLVER_CG, SOLVER_GMRES = 0, 1
 TOL_ABSOLUTE, TOL_RELATIVE = 0, 1
 PRECISION_FP64, PRECISION_MIXED, PRECISION_MIXED_PRECOND = 0, 1, 2
 SOLVER_OPT_FACTOR_ORDER, SOLVER_OPT_POLL, SOLVER_OPT_FUSE, SOLVER_OPT_REPLACE, SOLVER_OPT_GRAPH = 1, 2, 3, 4, 5
-SOLVER_OPT_GS_PASSES = 6
+SOLVER_OPT_GS_PASSES, SOLVER_OPT_SINGLE_LAUNCH = 6, 7
 
 
 class SolveStats(C.Structure):
@@ -161,6 +161,8 @@ SIGNATURES = {
     "pfem_solver_solve_pair": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "pfem_solver_set_batch_tiles": (_i, [_vp, _i, _vp, _vp, _vp]),
     "pfem_pfem2_sweep_fallbacks": (_i, [_vp]),
+    "pfem_solver_single_launches": (_i, [_vp, C.POINTER(_l), C.POINTER(_l)]),
+    "pfem_pfem2_single_launches": (_i, [_vp, C.POINTER(_l), C.POINTER(_l)]),
     "pfem_export_vtk": (_i, [_vp, C.c_char_p, _i, _vp, _vp]),
     "pfem_export_vtk3d": (_i, [_vp, C.c_char_p, _i, _vp, _vp]),
 }
@@ -494,8 +496,15 @@ class Solver(_Handle):
 
     def set_option(self, option, value):
         """SOLVER_OPT_FACTOR_ORDER (0/1), SOLVER_OPT_POLL (iterations between convergence polls) or
-        SOLVER_OPT_FUSE (0/1/2/3, default 3), SOLVER_OPT_REPLACE, SOLVER_OPT_GRAPH (0/1, default 0) or SOLVER_OPT_GS_PASSES (GMRES: 1/2, default 2)."""
+        SOLVER_OPT_FUSE (0/1/2/3, default 3), SOLVER_OPT_REPLACE, SOLVER_OPT_GRAPH (0/1, default 0), SOLVER_OPT_GS_PASSES (GMRES: 1/2, default 2) or
+        SOLVER_OPT_SINGLE_LAUNCH (0/1, default 1)."""
         self.ctx.check(lib().pfem_solver_set_option(self.h, option, int(value)))
+
+    def single_launches(self):
+        """(solves that ran as a single launch, single launches given up) since the solver was created"""
+        t, g = C.c_long(), C.c_long()
+        self.ctx.check(lib().pfem_solver_single_launches(self.h, C.byref(t), C.byref(g)))
+        return t.value, g.value
 
     def set_precision(self, precision, inner_tol=0.0, max_refinements=0):
         self.ctx.check(lib().pfem_solver_set_precision(self.h, precision, inner_tol, max_refinements))
@@ -745,6 +754,12 @@ class Pfem2(_Handle):
     def sweep_fallbacks(self):
         """solves re-run with per-level sweeps after a single-pass wait exceeded its spin limit"""
         return lib().pfem_pfem2_sweep_fallbacks(self.h)
+
+    def single_launches(self):
+        """(solves that ran as a single launch, single launches given up) of the stepper's solvers together"""
+        t, g = C.c_long(), C.c_long()
+        self.ctx.check(lib().pfem_pfem2_single_launches(self.h, C.byref(t), C.byref(g)))
+        return t.value, g.value
 
     def matrix_handle(self, which):
         """raw pfem_csr of the stepper: 0 prediction x, 1 prediction y, 2 pressure, 3 correction"""

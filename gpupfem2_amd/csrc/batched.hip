@@ -614,6 +614,7 @@ static void b_ru_run(Context* c, pfem_solver_t* s, BatchWork& w, pfem_csr_t* a, 
 static bool solve_resident(Context* c, pfem_solver_t* s, pfem_csr_t* a, const std::vector<int>& rows, double* x,
                            const double* b, pfem_solve_stats* stats, double* time_ms)
 {
+    if (!s->single_launch) return false;
     for (size_t k = 0; k + 2 < s->batch_tiling.size(); k += 3)
         if (s->batch_tiling[k + 1] != kBlock || s->batch_tiling[k + 2] != kTileNnz) return false;
     if (!s->resident) s->resident.reset(new ResidentWork());
@@ -626,6 +627,7 @@ static bool solve_resident(Context* c, pfem_solver_t* s, pfem_csr_t* a, const st
     if (!w.solve<double>(c, a->val.p, jac ? s->pc->invd.p : nullptr, b, x, false, s->tol, s->tol_mode, s->maxit,
                          mixed ? std::pow(10.0, -s->replace_digits) : 0.0, s->pc ? s->pc->spin_limit : 1 << 16))
         return false;
+    ++s->single_taken;
     int rate_khz = 0;
     PFEM_HIP(hipDeviceGetAttribute(&rate_khz, hipDeviceAttributeWallClockRate, c->device));
     for (int q = 0; q < w.nsys; ++q) {

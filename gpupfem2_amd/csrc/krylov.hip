@@ -724,6 +724,7 @@ static bool cg_resident(Context* c, pfem_solver_t* s, const KArgs<T>& A, CgState
     if (!w.solve<T>(c, A.val, A.invd, A.b, A.x, A.x_zero, A.tol, A.tol_mode, A.maxit, 0.0,
                     A.pc ? A.pc->spin_limit : 1 << 16))
         return false;
+    ++s->single_taken;
     const ResOut& o = w.h_out[0];
     *hst = CgState{};
     hst->it = o.it;
@@ -741,7 +742,7 @@ static void cg_run(Context* c, pfem_solver_t* s, const KArgs<T>& A, CgState* st,
     const int n = P.n;
     const unsigned g = vec_grid(n);
     const bool jac = A.kind == PFEM_PRECOND_JACOBI, none = A.kind == PFEM_PRECOND_NONE;
-    if ((jac || none) && cg_resident<T>(c, s, A, hst)) return;
+    if ((jac || none) && s->single_launch && cg_resident<T>(c, s, A, hst)) return;
     // x/r update fused into the forward sweep: multicolour IC0/ILU0, single-pass sweeps, factor ordering
     // (a blocked factor has the fused forms in their tagged form only)
     const bool fused = A.factor_order && A.pc && A.pc->sweep &&
@@ -792,11 +793,13 @@ static void cg_run(Context* c, pfem_solver_t* s, const KArgs<T>& A, CgState* st,
     // neighbours each, which is the quicker at every size that fits: 11.4 us an iteration against 26.0 at 13k rows,
     // 13.5 against 31.4 at 256k.
     if constexpr (sizeof(T) == 8)
-        if (xp_in_sweep && A.pc->contiguous && A.val == A.pc->aval.p) {
+        if (xp_in_sweep && s->single_launch && A.pc->contiguous && A.val == A.pc->aval.p) {
             if (!s->resident_ic0) s->resident_ic0.reset(new ResidentIc0());
             if (s->resident_ic0->plan(c, A.pc) &&
-                s->resident_ic0->solve(c, A.pc, A.pc_fp32, A.x, A.r, A.p, st, hst))
+                s->resident_ic0->solve(c, A.pc, A.pc_fp32, A.x, A.r, A.p, st, hst)) {
+                ++s->single_taken;
                 return;
+            }
         }
     if (fused2) {
         hipLaunchKernelGGL((k_fill_sentinel<double>), dim3(blocks_for(P.ntiles)), dim3(kBlock), 0, c->stream,
@@ -1596,6 +1599,7 @@ int pfem_solver_set_option(pfem_solver s, int option, int value)
             s->replace_digits = value;
             break;
         case PFEM_SOLVER_OPT_GRAPH: s->graph = value ? 1 : 0; break;
+        case PFEM_SOLVER_OPT_SINGLE_LAUNCH: s->single_launch = value ? 1 : 0; break;
         case PFEM_SOLVER_OPT_GS_PASSES:
             PFEM_REQUIRE(value == 1 || value == 2, "Gram-Schmidt passes must be 1 or 2");
             s->reorth = value == 2 ? 1 : 0;
@@ -1606,6 +1610,15 @@ int pfem_solver_set_option(pfem_solver s, int option, int value)
             break;
         default: throw Error(PFEM_EINVAL, "unknown solver option");
         }
+    });
+}
+
+int pfem_solver_single_launches(pfem_solver s, long* taken, long* given_up)
+{
+    PFEM_TRY(s ? s->ctx : nullptr, {
+        PFEM_REQUIRE(s, "null solver");
+        if (taken) *taken = s->single_taken;
+        if (given_up) *given_up = (s->resident ? s->resident->given_up : 0) + (s->resident_ic0 ? s->resident_ic0->given_up : 0);
     });
 }
 

@@ -446,6 +446,24 @@ int pfem_pfem2_sweep_fallbacks(pfem_pfem2 s)
     return s ? s->sweep_fallbacks : PFEM_EINVAL;
 }
 
+int pfem_pfem2_single_launches(pfem_pfem2 s, long* taken, long* given_up)
+{
+    PFEM_TRY(s ? s->ctx : nullptr, {
+        PFEM_REQUIRE(s, "null argument");
+        long sum[2] = {0, 0};
+        for (pfem_solver q : {s->s_pred, s->s_pred1, s->s_pres, s->s_corr}) {
+            if (!q) continue;
+            long t = 0;
+            long g = 0;
+            check(pfem_solver_single_launches(q, &t, &g), s->ctx);
+            sum[0] += t;
+            sum[1] += g;
+        }
+        if (taken) *taken = sum[0];
+        if (given_up) *given_up = sum[1];
+    });
+}
+
 int pfem_pfem2_matrix(pfem_pfem2 s, int which, pfem_csr* out)
 {
     if (!s || !out || which < 0 || which > 3) return PFEM_EINVAL;

@@ -534,7 +534,10 @@ bool ResidentWork::solve(Context* c, const T* val, const T* invd, const T* b, T*
     PFEM_HIP(hipStreamSynchronize(c->stream));
     if (*h_err == 0) return true;
     if (*h_err == 2) fits = false;   // a halo that never fits
-    else if (spin_limit > 0) pause = kResPause;
+    else {
+        ++given_up;
+        if (spin_limit > 0) pause = kResPause;
+    }
     if (!x_zero) PFEM_HIP(hipMemcpyAsync(x, keep, sizeof(T) * (size_t)P.n, hipMemcpyDeviceToDevice, c->stream));
     return false;
 }

@@ -24,6 +24,7 @@ struct ResidentWork {
     int nsys = 0, blocks = 0, tiles = 0, largest = 0, width = 0;
     bool fits = false, tiles_permuted = false;
     int pause = 0;                      // solves to come that do not try: a wait has failed
+    long given_up = 0;                  // solves in which one did
     DevArray<ResSys> sys;
     DevArray<double> ring, zbuf;
     DevArray<ResOut> out;

@@ -505,6 +505,7 @@ bool ResidentIc0::solve(Context* c, pfem_precond_t* pc, bool reduced, double* x,
     PFEM_HIP(hipMemcpyAsync(h_err, err.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     PFEM_HIP(hipStreamSynchronize(c->stream));
     if (*h_err) {
+        ++given_up;
         if (pc->spin_limit > 0) pause = kResPause;
         return false;
     }

@@ -12,6 +12,7 @@ struct ResidentIc0 {
     bool fits = false;
     int blocks = 0, width = 0, places = 0;
     int pause = 0;                  // solves to come that do not try: a wait has failed
+    long given_up = 0;              // solves in which one did
     DevArray<int> rows, halo, steps;   // per lane: row, halo row (or -1); per workgroup: sweep steps
     DevArray<int> post, from;          // per lane: exchange places of a row on a patch's rim, of a halo row
     DevArray<uint32_t> info, hinfo;

@@ -282,6 +282,8 @@ struct pfem_solver_t {
     // sweeps (IC0: three launches per iteration)
     int fuse = 3;
     int graph = 0;                        // fused PCG: replay a captured batch of iterations
+    int single_launch = 1;                // solves that fit as one launch
+    long single_taken = 0;                // those that ran so
     int replace_digits = 2;   // reliable updates (multi/batched MIXED): replace after gamma fell 10^-digits
     hipEvent_t ev[2] = {nullptr, nullptr};   // pipelined polls of the device state
     std::unique_ptr<pfem::MultiWork, pfem::MultiWorkDeleter> multi;   // pfem_solver_solve_multi

@@ -212,9 +212,11 @@ int pfem_precond_download(pfem_precond pc, double* factor, int* n_levels, int* p
 int pfem_precond_set_sweep(pfem_precond pc, int single_pass);
 /* Polls a single-pass wait makes before it is declared failed (no counterpart in the reference; default
  * 65536, about 0.1 s). A failed wait does not hang or fault: the launch completes, and the solve or apply
- * reports PFEM_ENUMERIC and re-arms the sweep buffers. 0 fails every wait that is not satisfied at once. With a
- * Jacobi preconditioner or none it scales the waits of the single-launch PCG, which falls back to one
- * launch per kernel, with the same results, when a wait fails. */
+ * reports PFEM_ENUMERIC and re-arms the sweep buffers. 0 fails every wait that is not satisfied at once. (Natural
+ * ordering with many small levels: polls come two to three times as often, and a wait's limit grows with the
+ * number of row blocks before it.) The waits of the single-launch PCG (PFEM_SOLVER_OPT_SINGLE_LAUNCH) scale with it
+ * too: a quarter of it for a Jacobi or unpreconditioned system, about 18 ms at the default, and eight
+ * times it, about 0.6 s, for a batch and for IC0. */
 int pfem_precond_set_spin_limit(pfem_precond pc, int polls);
 /* Storage of the reduced-precision factor copy that PFEM_PRECISION_MIXED_PRECOND applies to FP64 vectors
  * (no counterpart in the reference, whose factor is FP64): 32 (default) or 16 bits per value (IEEE half;
@@ -268,7 +270,23 @@ int pfem_solver_set_precision(pfem_solver s, int precision, double inner_tol, in
                                     with IC0 the forward sweep ends the iteration with gamma = (y, y),
                                     y = L^-1 r, equal to (r, z) in exact arithmetic, and the backward
                                     sweep applies the x and p updates (three launches per iteration) */
+#define PFEM_SOLVER_OPT_SINGLE_LAUNCH 7 /* PCG, default 1: a solve whose vectors and matrix fit the registers and LDS
+                                    of the device runs as one launch; 0: always one launch per kernel and iteration.
+                                    Fit: Jacobi or no preconditioner, up to 262144 rows of up to 16 entries
+                                    (FP64, the inner solves of MIXED, batches); multicolour IC0 at fusion level 3, up
+                                    to 262144 rows of up to 12 neighbours (the iterations; MIXED_PRECOND too). Such a
+                                    solve holds the compute units it runs on until it ends, and such solves of
+                                    several threads run one after the other. If other work holds so much of the device that one of its
+                                    waits exceeds its limit (pfem_precond_set_spin_limit), it is given up, the
+                                    solve is done launch by launch, and so are the next 64 of this solver. The
+                                    results are the same bits either way for Jacobi or no preconditioner (single
+                                    solves, MIXED, FP64 batches). They are not for IC0, whose sums are grouped
+                                    differently (the same iterates to rounding), nor for a batch in MIXED, which
+                                    iterates in FP64 in a single launch and in FP32 launch by launch */
 int pfem_solver_set_option(pfem_solver s, int option, int value);
+/* Since the solver was created: solves that ran as a single launch (every inner solve of MIXED counts, a batch counts
+ * as one), and those given up because a wait exceeded its limit. Either may be NULL. */
+int pfem_solver_single_launches(pfem_solver s, long* taken, long* given_up);
 int pfem_solver_destroy(pfem_solver s);
 /* LinearSolver::solve(A, x, b) -> bool (linear_solver.cu:146-154, 301-376, 421-521): warm start from x,
  * the preconditioner is re-initialised from A first. stats may be NULL. */
@@ -451,6 +469,8 @@ int pfem_pfem2_set_graphs(pfem_pfem2 s, int on);
  * counterpart in the reference, whose SpSV has no such wait): such a solve is repeated from the same start
  * with per-level sweeps and the FP64 factor instead of failing the step, and a line goes to stderr. */
 int pfem_pfem2_sweep_fallbacks(pfem_pfem2 s);
+/* pfem_solver_single_launches of the stepper's solvers together */
+int pfem_pfem2_single_launches(pfem_pfem2 s, long* taken, long* given_up);
 /* the stepper's matrices (borrowed, owned by s): 0 prediction x, 1 prediction y, 2 pressure,
  * 3 correction; and its preconditioners: 0 prediction, 1 pressure, 2 correction */
 int pfem_pfem2_matrix(pfem_pfem2 s, int which, pfem_csr* out);

@@ -1,8 +1,8 @@
-"""Two contexts (two streams) on one GPU solving at the same time from two host threads: the fused
-multicolour IC0-PCG (single-pass sweeps that wait on values published by earlier workgroups of their own
-launch) and the blocked one, each interleaved on the device with the other's launches. Each solve must give
-the bits and iteration count it gives alone: a launch only ever waits on workgroups of its own grid, which
-were dispatched before it whatever else the device runs.
+"""Two contexts (two streams) on one GPU solving at the same time from two host threads: the multicolour IC0-PCG as
+single launches, and as fused launches (single-pass sweeps that wait on values published by earlier workgroups of
+their own launch), and the blocked one, each interleaved on the device with the other's launches. Each solve must
+give the bits and iteration count it gives alone: a sweep only ever waits on workgroups of its own grid, which
+were dispatched before it whatever else the device runs, and single launches run one after the other.
 """
 import threading
 
@@ -23,10 +23,11 @@ def pressure_system(ctx, case):
     return m, a, rhs
 
 
+@pytest.mark.parametrize("single", [1, 0])
 @pytest.mark.parametrize("orderings", [(1, 1), (1, 2)])
-def test_concurrent_solves_two_streams(orderings):
+def test_concurrent_solves_two_streams(orderings, single):
     from gpupfem2_amd import capi, cases
-    print("concurrent solves", orderings, flush=True)
+    print("concurrent solves", orderings, single, flush=True)
     case = cases.cylinder_case(h=1.0 / 56)
     n = case.xy.shape[0]
     ctxs = [capi.Context(0), capi.Context(0)]
@@ -37,6 +38,7 @@ def test_concurrent_solves_two_streams(orderings):
         m, a, rhs = systems[k]
         s = capi.Solver(a, capi.SOLVER_CG, 1e-12, 20000, 0, capi.TOL_RELATIVE,
                         capi.Preconditioner(a, capi.PRECOND_IC0, orderings[k]))
+        s.set_option(capi.SOLVER_OPT_SINGLE_LAUNCH, single)
         return s
 
     def solve(k, s, out):
@@ -62,6 +64,8 @@ def test_concurrent_solves_two_streams(orderings):
         for k in range(2):
             assert together[k][0] and together[k][1] == alone[k][1], (rep, k, together[k][1], alone[k][1])
             assert np.array_equal(together[k][2], alone[k][2]), (rep, k)
+    for k in range(2):
+        assert solvers[k].single_launches() == (4 if single and orderings[k] == 1 else 0, 0)
     for c in ctxs:
         c.sync()
     # the handles before the contexts they were made on

@@ -1,10 +1,28 @@
-"""GPU: the single-launch (resident) PCG against the launch-per-kernel PCG, which a zero spin limit forces
-(every wait that is not satisfied at once fails, and the solve falls back): the same bits of the solution and the
-same iteration count, since both add the same partials in the same order."""
+"""GPU: the single-launch (resident) PCG against the launch-per-kernel PCG (SOLVER_OPT_SINGLE_LAUNCH 0), and against a
+single launch given up for it (a zero spin limit fails every wait that is not satisfied at once): the same bits of
+the solution and the same iteration count, since both add the same partials in the same order. The solver's
+counts tell which path each solve took."""
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
+
+
+# single launches, launch per kernel, single launches given up
+WAYS = ((1, 1 << 16), (0, 1 << 16), (1, 0))
+
+
+def check_way(s, way, rows):
+    """the path that the solver's solves took; systems of up to 1024 rows are one workgroup, which never waits"""
+    taken, given_up = s.single_launches()
+    if way == WAYS[0]:
+        assert taken >= 1 and given_up == 0, (taken, given_up)
+    elif way == WAYS[1]:
+        assert (taken, given_up) == (0, 0)
+    elif rows > 1024:
+        assert taken == 0 and given_up >= 1, (taken, given_up)
+    else:
+        assert taken >= 1 and given_up == 0, (taken, given_up)
 
 
 def poisson(ctx, nx, ny, seed, jitter=0.2):
@@ -33,19 +51,21 @@ def test_resident_same_bits(ctx, nx, ny, kind, precision):
     n = a.n
     start = np.random.default_rng(5).standard_normal(n) * 1e-3
     out = []
-    for limit in (1 << 16, 0):
+    for way in WAYS:
         pc = capi.Preconditioner(a, kind)
-        pc.set_spin_limit(limit)
+        pc.set_spin_limit(way[1])
         s = capi.Solver(a, capi.SOLVER_CG, 1e-11, 8000, 0, capi.TOL_RELATIVE, pc)
+        s.set_option(capi.SOLVER_OPT_SINGLE_LAUNCH, way[0])
         if precision:
             s.set_precision(precision, 1e-5, 30)
         x = ctx.to_device(start)
         d = ctx.to_device(b)
         st = s.solve(a, x, d)
         assert st.converged and not st.nan_detected
+        check_way(s, way, n)
         out.append((x.download(), st.iterations, st.final_residual, st.refinements))
-    assert out[0][1:] == out[1][1:]
-    assert np.array_equal(out[0][0], out[1][0])
+    assert out[0][1:] == out[1][1:] == out[2][1:]
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][0], out[2][0])
 
 
 def test_resident_iteration_limit_and_zero(ctx):
@@ -53,17 +73,19 @@ def test_resident_iteration_limit_and_zero(ctx):
     from gpupfem2_amd import capi
     m, a, b = poisson(ctx, 60, 60, seed=2)
     out = []
-    for limit in (1 << 16, 0):
+    for way in WAYS:
         pc = capi.Preconditioner(a, 1)
-        pc.set_spin_limit(limit)
+        pc.set_spin_limit(way[1])
         s = capi.Solver(a, capi.SOLVER_CG, 1e-11, 17, 0, capi.TOL_RELATIVE, pc)
+        s.set_option(capi.SOLVER_OPT_SINGLE_LAUNCH, way[0])
         x = ctx.zeros(a.n)
         st = s.solve(a, x, ctx.to_device(b))
         assert not st.converged and st.iterations == 17
         out.append(x.download())
         st = s.solve(a, ctx.zeros(a.n), ctx.zeros(a.n))
-        assert st.iterations <= 17
-    assert np.array_equal(out[0], out[1])
+        assert st.converged and st.iterations == 0
+        check_way(s, way, a.n)
+    assert np.array_equal(out[0], out[1]) and np.array_equal(out[0], out[2])
 
 
 @pytest.mark.parametrize("precision", [0, 1])
@@ -75,20 +97,34 @@ def test_resident_batch(ctx, precision):
     mesh, a, b = cases.build_batched_poisson(ctx, case)
     rows, n = case["sys_rows"], case["sys_rows"][-1]
     out = []
-    for limit in (1 << 16, 0):
+    for way in WAYS:
         pc = capi.Preconditioner(a, 1)
-        pc.set_spin_limit(limit)
+        pc.set_spin_limit(way[1])
         s = capi.Solver(a, capi.SOLVER_CG, 1e-11, 20000, 0, capi.TOL_RELATIVE, pc)
+        s.set_option(capi.SOLVER_OPT_SINGLE_LAUNCH, way[0])
         if precision:
             s.set_precision(precision, 1e-5, 30)
         x = ctx.zeros(n)
         st, ms = s.solve_batched(a, rows, x, b)
         assert all(q.converged and not q.nan_detected for q in st)
         assert (ms > 0).all()
+        check_way(s, way, n)
         out.append((x.download(), [q.iterations for q in st], [q.refinements for q in st]))
     if precision:
         assert all(r >= 1 for r in out[0][2])
         assert np.linalg.norm(out[0][0] - out[1][0]) < 1e-8 * np.linalg.norm(out[1][0])
+        assert out[1][1] == out[2][1] and np.array_equal(out[1][0], out[2][0])
     else:
-        assert out[0][1] == out[1][1]
-        assert np.array_equal(out[0][0], out[1][0])
+        assert out[0][1] == out[1][1] == out[2][1]
+        assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][0], out[2][0])
+
+
+def test_stepper_counts(ctx):
+    """the stepper reports its solvers' single launches: every solve of a small channel step is one"""
+    from gpupfem2_amd import cases
+    mesh, ph, stepper = cases.build_gpu(ctx, cases.poiseuille_case(nx=40, ny=10, ppc=4, dt=1e-2))
+    assert stepper.single_launches() == (0, 0)
+    stepper.step()
+    first = stepper.single_launches()
+    stepper.step()
+    assert first[0] > 0 and first[1] == 0 and stepper.single_launches()[0] > first[0]
