@@ -29,6 +29,8 @@
 // solves with the launch-per-kernel path instead.
 #include <algorithm>
 #include <climits>
+#include <condition_variable>
+#include <mutex>
 
 #include "device.hpp"
 #include "internal.hpp"
@@ -419,10 +421,38 @@ Kernel<T> kernel_for(int width, bool jac, bool rel, bool two_per_cu)
 }
 }  // namespace
 
-std::mutex& resident_mutex(int device)
+namespace {
+struct Seats {
+    std::mutex m;
+    std::condition_variable freed;
+    int used = 0;
+    unsigned long next = 0, serving = 0;   // tickets
+};
+Seats& seats(int device)
 {
-    static std::mutex m[64];
-    return m[device & 63];
+    static Seats s[64];
+    return s[device & 63];
+}
+}  // namespace
+
+ResidentSeats::ResidentSeats(int device, int blocks, int cus)
+    : device_(device), taken_(std::min((blocks + 7) / 8 * 8, cus))
+{
+    Seats& s = seats(device_);
+    std::unique_lock<std::mutex> lock(s.m);
+    const unsigned long ticket = s.next++;
+    s.freed.wait(lock, [&] { return s.serving == ticket && s.used + taken_ <= cus; });
+    s.used += taken_;
+    ++s.serving;
+    s.freed.notify_all();
+}
+
+ResidentSeats::~ResidentSeats()
+{
+    Seats& s = seats(device_);
+    std::lock_guard<std::mutex> lock(s.m);
+    s.used -= taken_;
+    s.freed.notify_all();
 }
 
 int resident_blocks(int rows) { return (rows + kResLanes - 1) / kResLanes; }
@@ -521,7 +551,7 @@ bool ResidentWork::solve(Context* c, const T* val, const T* invd, const T* b, T*
     a.x_zero = x_zero ? 1 : 0;
     a.drop = drop;
     T* keep = reinterpret_cast<T*>(zbuf.p) + 3 * (size_t)P.n;
-    std::lock_guard<std::mutex> alone(resident_mutex(c->device));
+    const ResidentSeats held(c->device, blocks, cus);
     const long nfill = std::max({3L * P.n, 4L * tiles, (long)nsys});
     hipLaunchKernelGGL(k_resident_prepare<T>, dim3(blocks_for(nfill)), dim3(kBlock), 0, c->stream, 3L * P.n,
                        reinterpret_cast<typename Sentinel<T>::U*>(zbuf.p), 4L * tiles, a.ring, nsys, out.p, err.p,

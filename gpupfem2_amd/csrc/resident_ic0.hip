@@ -440,15 +440,11 @@ bool ResidentIc0::plan(Context* c, const pfem_precond_t* pc)
 }
 
 template <typename TS>
-static bool launch(Context* c, ResidentIc0& w, pfem_precond_t* pc, const TS* f, const double* scale, const double* x,
+static void launch(Context* c, ResidentIc0& w, pfem_precond_t* pc, const TS* f, const double* scale, const double* x,
                    const double* r, const double* p, const CgState* st)
 {
     const Pattern& P = *w.pat;
     auto k = w.width == 8 ? k_resident_ic0<TS, 8> : k_resident_ic0<TS, 12>;
-    int per_cu = 0, cus = 0;
-    PFEM_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
-    PFEM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k, kIcLanes, 0));
-    if (w.blocks > per_cu * cus) return false;
     IcArgs<TS> a{};
     a.rows = w.rows.p;
     a.halo = w.halo.p;
@@ -484,7 +480,15 @@ static bool launch(Context* c, ResidentIc0& w, pfem_precond_t* pc, const TS* f, 
                        reinterpret_cast<unsigned long long*>(w.buf.p), 4 * w.blocks, a.ring, w.err.p);
     hipLaunchKernelGGL(k, dim3(w.blocks), dim3(kIcLanes), 0, c->stream, a);
     PFEM_HIP(hipGetLastError());
-    return true;
+}
+
+template <typename TS>
+static bool fits_device(const ResidentIc0& w, int cus)
+{
+    auto k = w.width == 8 ? k_resident_ic0<TS, 8> : k_resident_ic0<TS, 12>;
+    int per_cu = 0;
+    PFEM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k, kIcLanes, 0));
+    return w.blocks <= per_cu * cus;
 }
 
 bool ResidentIc0::solve(Context* c, pfem_precond_t* pc, bool reduced, double* x, const double* r, const double* p,
@@ -495,12 +499,15 @@ bool ResidentIc0::solve(Context* c, pfem_precond_t* pc, bool reduced, double* x,
         --pause;
         return false;
     }
-    std::lock_guard<std::mutex> alone(resident_mutex(c->device));
     const bool half = reduced && pc->factor_bits == 16 && pc->half_ok;
-    const bool ran = half ? launch<_Float16>(c, *this, pc, pc->split16.p, pc->scale16.p, x, r, p, st)
-                     : reduced ? launch<float>(c, *this, pc, pc->split32.p, nullptr, x, r, p, st)
-                               : launch<double>(c, *this, pc, pc->split.p, nullptr, x, r, p, st);
-    if (!ran) return false;
+    int cus = 0;
+    PFEM_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
+    if (!(half ? fits_device<_Float16>(*this, cus) : reduced ? fits_device<float>(*this, cus) : fits_device<double>(*this, cus)))
+        return false;
+    const ResidentSeats held(c->device, blocks, cus);
+    if (half) launch<_Float16>(c, *this, pc, pc->split16.p, pc->scale16.p, x, r, p, st);
+    else if (reduced) launch<float>(c, *this, pc, pc->split32.p, nullptr, x, r, p, st);
+    else launch<double>(c, *this, pc, pc->split.p, nullptr, x, r, p, st);
     PFEM_HIP(hipMemcpyAsync(hst, out.p, sizeof(CgState), hipMemcpyDeviceToHost, c->stream));
     PFEM_HIP(hipMemcpyAsync(h_err, err.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     PFEM_HIP(hipStreamSynchronize(c->stream));

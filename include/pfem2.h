@@ -275,8 +275,9 @@ int pfem_solver_set_precision(pfem_solver s, int precision, double inner_tol, in
                                     Fit: Jacobi or no preconditioner, up to 262144 rows of up to 16 entries
                                     (FP64, the inner solves of MIXED, batches); multicolour IC0 at fusion level 3, up
                                     to 262144 rows of up to 12 neighbours (the iterations; MIXED_PRECOND too). Such a
-                                    solve holds the compute units it runs on until it ends, and such solves of
-                                    several threads run one after the other. If other work holds so much of the device that one of its
+                                    solve holds the compute units it runs on until it ends; solves of
+                                    several threads run side by side as far as they fit the device together and
+                                    wait for one another otherwise. If other work holds so much of the device that one of its
                                     waits exceeds its limit (pfem_precond_set_spin_limit), it is given up, the
                                     solve is done launch by launch, and so are the next 64 of this solver. The
                                     results are the same bits either way for Jacobi or no preconditioner (single

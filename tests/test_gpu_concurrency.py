@@ -2,9 +2,11 @@
 single launches, and as fused launches (single-pass sweeps that wait on values published by earlier workgroups of
 their own launch), and the blocked one, each interleaved on the device with the other's launches. Each solve must
 give the bits and iteration count it gives alone: a sweep only ever waits on workgroups of its own grid, which
-were dispatched before it whatever else the device runs, and single launches run one after the other.
+were dispatched before it whatever else the device runs, and a single launch runs only where all its workgroups
+fit the device beside those of the others.
 """
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -117,3 +119,59 @@ def test_concurrent_steppers_with_graphs():
     del together, alone, threads
     for c in ctxs:
         c.close()
+
+
+@pytest.mark.parametrize("kind,order,nx,ny", [(1, 0, 100, 50), (2, 1, 100, 50), (1, 0, 511, 255)])
+def test_concurrent_single_launches(kind, order, nx, ny):
+    """Four threads' single-launch solves of 6 workgroups each wait rather than compute, and fit the device many
+    times over: together they take well under the time of one thread after the other (the same while one solve at a
+    time was let onto the device), with the bits each gives alone. Of 128 workgroups each, two fit at a time."""
+    from gpupfem2_amd import capi, meshgen
+    print("concurrent single launches", kind, nx, flush=True)
+    threads, reps = 4, 10 if nx == 100 else 3
+    xy, tri = meshgen.rectangle(0.0, 2.0, 0.0, 1.0, nx, ny, jitter=0.2, seed=3)
+    left = np.nonzero(xy[:, 0] < 1e-9)[0].astype(np.int32)
+    n = xy.shape[0]
+    b = np.random.default_rng(1).standard_normal(n)
+    b[left] = 0.0
+    ctxs = [capi.Context(0) for _ in range(threads)]
+    held = []
+    for c in ctxs:
+        m = capi.Mesh2D(c, xy, tri, fill_neighbors=False)
+        a, scratch = capi.CSR(c, mesh=m), c.zeros(n)
+        capi.assemble_poisson2d(m, a, scratch, coeff=1.0, rhs_kind=2, rhs_param=0.0)
+        capi.Dirichlet(c, n, left, np.zeros(left.size)).apply(a, scratch, 1)
+        s = capi.Solver(a, capi.SOLVER_CG, 1e-11, 8000, 0, capi.TOL_RELATIVE, capi.Preconditioner(a, kind, order))
+        held.append((m, a, s, c.to_device(b), c.zeros(n)))
+        del m, a, s, scratch
+
+    def work(k, out):
+        m, a, s, d, x = held[k]
+        for _ in range(reps):
+            x.zero()
+            assert s.solve(a, x, d).converged
+        out[k] = x.download()
+
+    out = [{}, {}]
+    for k in range(threads):
+        work(k, out[0])
+    t = time.perf_counter()
+    for k in range(threads):
+        work(k, out[0])
+    alone = time.perf_counter() - t
+    ts = [threading.Thread(target=work, args=(k, out[1])) for k in range(threads)]
+    t = time.perf_counter()
+    for q in ts:
+        q.start()
+    for q in ts:
+        q.join(timeout=60)
+    together = time.perf_counter() - t
+    assert not any(q.is_alive() for q in ts)
+    print("one after the other", alone, "together", together, flush=True)
+    for k in range(threads):
+        assert np.array_equal(out[0][k], out[0][0]) and np.array_equal(out[1][k], out[0][0])
+        assert held[k][2].single_launches() == (3 * reps, 0)
+    held.clear()
+    for c in ctxs:
+        c.close()
+    assert together < (0.75 if nx == 100 else 1.2) * alone
