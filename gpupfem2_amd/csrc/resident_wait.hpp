@@ -34,10 +34,10 @@ __device__ __forceinline__ T res_await(typename Sentinel<T>::U* q, typename Sent
 {
     constexpr typename Sentinel<T>::U sent = Sentinel<T>::bits;
     for (long spins = 0; v == sent; ++spins) {
-        if (spins >= limit ||
-            ((spins & 1023) == 1023 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
+        if (spins >= limit || ((spins == 63 || (spins & 1023) == 1023) &&
+                               __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
             *fail = 1;
-            __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_fetch_max(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // (a 2 stays)
             break;
         }
         // workgroups of a batch's next system may wait for its last ones to start: they must not crowd the

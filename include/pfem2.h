@@ -272,7 +272,8 @@ int pfem_solver_set_precision(pfem_solver s, int precision, double inner_tol, in
                                     sweep applies the x and p updates (three launches per iteration) */
 #define PFEM_SOLVER_OPT_SINGLE_LAUNCH 7 /* PCG, default 1: a solve whose vectors and matrix fit the registers and LDS
                                     of the device runs as one launch; 0: always one launch per kernel and iteration.
-                                    Fit: Jacobi or no preconditioner, up to 262144 rows of up to 16 entries
+                                    Fit: Jacobi or no preconditioner, up to 262144 rows of up to 16 entries, numbered
+                                    so that 1024 rows in sequence use at most 2048 columns outside themselves
                                     (FP64, the inner solves of MIXED, batches); multicolour IC0 at fusion level 3, up
                                     to 262144 rows of up to 12 neighbours (the iterations; MIXED_PRECOND too). Such a
                                     solve holds the compute units it runs on until it ends; solves of

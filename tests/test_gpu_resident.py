@@ -128,3 +128,35 @@ def test_stepper_counts(ctx):
     first = stepper.single_launches()
     stepper.step()
     assert first[0] > 0 and first[1] == 0 and stepper.single_launches()[0] > first[0]
+
+
+def test_resident_halo(ctx):
+    """nodes numbered at random: a workgroup's rows use more columns of others than it can hold, in all but the last of
+    the workgroups. The first launch sees it and none is tried again; in a batch with a system that fits the plan does
+    """
+    from gpupfem2_amd import capi, meshgen
+    xy, tri = meshgen.rectangle(0.0, 2.0, 0.0, 1.0, 100, 50, jitter=0.2, seed=3)
+    n = xy.shape[0]
+    new = np.random.default_rng(5).permutation(n)
+    shuffled = np.empty_like(xy)
+    shuffled[new] = xy
+    other, other_tri = meshgen.rectangle(0.0, 2.0, 2.0, 3.0, 60, 40, jitter=0.2, seed=4)
+    for batch in (False, True):
+        p, t = shuffled, new[tri]
+        if batch:
+            p, t = np.concatenate([p, other]), np.concatenate([t, other_tri + n])
+        m = capi.Mesh2D(ctx, np.ascontiguousarray(p), np.ascontiguousarray(t.astype(np.int32)), fill_neighbors=False)
+        a = capi.CSR(ctx, mesh=m)
+        scratch = ctx.zeros(a.n)
+        capi.assemble_poisson2d(m, a, scratch, coeff=1.0, rhs_kind=2, rhs_param=0.0)
+        left = np.nonzero(p[:, 0] < 1e-9)[0].astype(np.int32)
+        capi.Dirichlet(ctx, a.n, left, np.zeros(left.size)).apply(a, scratch)
+        b = np.random.default_rng(1).standard_normal(a.n)
+        b[left] = 0.0
+        d = ctx.to_device(b)
+        s = capi.Solver(a, capi.SOLVER_CG, 1e-9, 4000, 0, capi.TOL_RELATIVE, capi.Preconditioner(a, 1))
+        for _ in range(2 if batch else 66):
+            x = ctx.zeros(a.n)
+            st = s.solve_batched(a, [0, n, a.n], x, d)[0] if batch else [s.solve(a, x, d)]
+            assert all(q.converged for q in st)
+        assert s.single_launches() == (0, 0)
