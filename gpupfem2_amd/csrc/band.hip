@@ -11,8 +11,8 @@
 // of their use, ahead of the solving wave, and one wave publishes the band's own (the sentinel protocol
 // of sync.hpp; bands wait only on bands dispatched before them). Bands follow each other down the level
 // chain a few levels behind. A quotient by the diagonal is formed from its reciprocal and two corrections, which gives the
-// correctly rounded quotient (Markstein, "IA-64 and Elementary Functions", 2000) at a third of the
-// division's latency, so results are those of the sequential solve, bit for bit. A level takes 0.15 us.
+// correctly rounded quotient (quotient.hpp) at a third of the division's latency, so results are those of the
+// sequential solve, bit for bit. A level takes 0.15 us in a chain, 0.2 us in a mesh (an apply's two solves of 399 levels: 160 us).
 //
 // Measured (MI355X, FP64 IC0 apply, chunked sweeps -> here): unit square 40k rows, 401 levels 1292 -> 147 us,
 // 160k rows, 801 levels 4227 -> 321 us; cylinder 1M rows, 2689 levels 30.6 -> 1.64 ms; 3D box 133k rows, 151
@@ -23,6 +23,7 @@
 
 #include "band.hpp"
 #include "device.hpp"
+#include "quotient.hpp"
 #include "sync.hpp"
 
 namespace pfem {
@@ -88,20 +89,6 @@ __device__ __forceinline__ void band_load(BandSlot<W, TS>& t, const char* __rest
         t.ri = q.y;
     }
 }
-
-// s / d from ri = 1 / d (correctly rounded): the first quotient is within two units in the last place, the
-// second within one, and Markstein's theorem makes the third the correctly rounded one as long as no step
-// under- or overflows: |d| in [2^-100, 2^100] (else ri is stored as a NaN) and |q| >= 2^-800 or s = 0. A
-// result outside (NaNs included) is formed again by the division.
-__device__ __forceinline__ double quotient(double s, double d, double ri)
-{
-    const double q0 = s * ri;
-    const double q1 = fma(fma(-d, q0, s), ri, q0);
-    return __builtin_copysign(fma(fma(-d, q1, s), ri, q1), q0);   // (the sign of a zero)
-}
-__device__ __forceinline__ bool quotient_ok(double q) { return fabs(q) >= 0x1p-800 || q == 0.0; }
-__device__ __forceinline__ float quotient(float s, float d, double) { return s / d; }
-__device__ __forceinline__ bool quotient_ok(float q) { return q == q; }
 
 // A value in LDS: 8 bytes for FP32 too, so that places are the same byte offsets
 template <typename TF>

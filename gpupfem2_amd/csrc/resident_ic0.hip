@@ -31,6 +31,7 @@
 
 #include "device.hpp"
 #include "internal.hpp"
+#include "quotient.hpp"
 #include "resident_ic0.hpp"
 #include "resident_wait.hpp"
 
@@ -165,12 +166,6 @@ __global__ __launch_bounds__(kIcLanes, 4) void k_resident_ic0(IcArgs<TS> a)
     auto place = [&](const double* v, int e) {
         return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(v) + ((e & 1) ? cw[e / 2] >> 16 : cw[e / 2] & 0xFFFFu));
     };
-    // s / ld from the correctly rounded reciprocal: quotient, its exact remainder, correction (Markstein's
-    // theorem: the correctly rounded quotient), 3 operations on the colours' chain instead of a division
-    auto divided = [&](double s) {
-        const double q0 = s * li;
-        return __builtin_fma(__builtin_fma(-q0, ld, s), li, q0);
-    };
     int e = 0;
     __syncthreads();
     while (!done) {
@@ -201,7 +196,7 @@ __global__ __launch_bounds__(kIcLanes, 4) void k_resident_ic0(IcArgs<TS> a)
 #pragma unroll
                 for (int k = 0; k < W; ++k)
                     s -= (k < nl ? (double)lv[k] : 0.0) * place(yl, k);
-                y = divided(s);
+                y = quotient_near(s, ld, li);
                 yl[tid] = y;
                 if (rim) publish(yb + post, y);
             }
@@ -222,7 +217,7 @@ __global__ __launch_bounds__(kIcLanes, 4) void k_resident_ic0(IcArgs<TS> a)
 #pragma unroll
                 for (int k = 0; k < W; ++k)
                     s -= (k < nl ? 0.0 : (double)lv[k]) * place(yl, k);
-                y = divided(s);
+                y = quotient_near(s, ld, li);
                 yl[tid] = y;
                 if (rim) publish(zb + post, y);
             }
