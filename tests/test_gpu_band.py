@@ -1,5 +1,5 @@
-"""GPU: the band sweeps of natural-order IC0/ILU0 factors with many small levels against the per-level solves (one
-launch per level, selected with set_sweep): the same bits."""
+"""GPU: the single-pass sweeps of natural-order IC0/ILU0 factors, in bands (many small levels) and in chunks (what the
+bands do not take), against the per-level solves (one launch per level, selected with set_sweep): the same bits."""
 import numpy as np
 import pytest
 
@@ -72,6 +72,78 @@ def test_band_sweeps_same_bits(ctx, name, kind):
         pc.apply(src, src)      # in place
         assert np.array_equal(src.download(), first)
         out.append(first)
+    assert np.array_equal(out[0], out[1])
+
+
+def shuffled(ctx, n):
+    """a mesh numbered at random: few levels, each of a good part of the rows"""
+    from gpupfem2_amd import capi, meshgen
+    xy, tri = meshgen.unit_square(n, jitter=0.2, seed=n)
+    new = np.random.default_rng(4).permutation(xy.shape[0])
+    q = np.empty_like(xy)
+    q[new] = xy
+    m = capi.Mesh2D(ctx, q, np.ascontiguousarray(new[tri].astype(np.int32)), fill_neighbors=False)
+    a = capi.CSR(ctx, mesh=m)
+    rhs = ctx.zeros(a.n)
+    capi.assemble_poisson2d(m, a, rhs, coeff=1.0, rhs_kind=2, rhs_param=1.0)
+    edge = np.nonzero((np.abs(q - 0.5) > 0.5 - 1e-9).any(axis=1))[0].astype(np.int32)
+    capi.Dirichlet(ctx, a.n, edge, np.zeros(edge.size)).apply(a, rhs)
+    return a, m
+
+
+def wide(ctx, n):
+    """17 entries on either side of the diagonal, one more than a slice of a band holds"""
+    from gpupfem2_amd import capi
+    off = np.concatenate([-np.arange(17, 0, -1) * 3, [0], np.arange(1, 18) * 3])
+    col = np.arange(n)[:, None] + off[None, :]
+    val = np.where(off == 0, 40.0, -1.0)[None, :] + 0.1 * np.sin(np.arange(n))[:, None] * (off == 0)
+    keep = (col >= 0) & (col < n)
+    rowptr = np.concatenate([[0], np.cumsum(keep.sum(1))]).astype(np.int32)
+    return capi.CSR(ctx, rowptr=rowptr, col=col[keep].astype(np.int32), val=val[keep]), None
+
+
+def far(ctx, n):
+    """coupled to rows up to 6000 away: more columns of other bands than a band holds, in many levels"""
+    from gpupfem2_amd import capi
+    i = np.repeat(np.arange(n), 2)
+    j = i - np.random.default_rng(6).integers(1, 6000, i.size)
+    lower = sorted(set(zip(i[j >= 0].tolist(), j[j >= 0].tolist())))
+    rows = [[] for _ in range(n)]
+    for p, q in lower:
+        rows[p].append(q)
+        rows[q].append(p)
+    col, val, rowptr = [], [], [0]
+    for p in range(n):
+        r = sorted(rows[p] + [p])
+        col += r
+        val += [float(len(r)) if q == p else -1.0 for q in r]
+        rowptr.append(len(col))
+    return capi.CSR(ctx, rowptr=np.array(rowptr, np.int32), col=np.array(col, np.int32), val=np.array(val)), None
+
+
+# what the bands do not take: chunks of the whole factor's levels
+CHUNKED = {"shuffled_40": (shuffled, 40), "shuffled_200": (shuffled, 200), "wide_300": (wide, 300), "wide_3000": (wide, 3000),
+           "far_30000": (far, 30000)}
+
+
+@pytest.mark.parametrize("kind", [2, 3])
+@pytest.mark.parametrize("name", CHUNKED)
+def test_chunked_sweeps_same_bits(ctx, name, kind):
+    from gpupfem2_amd import capi
+    print("chunked sweeps", name, kind, flush=True)
+    make, size = CHUNKED[name]
+    a, keep = make(ctx, size)
+    r = np.random.default_rng(1).standard_normal(a.n)
+    out = []
+    for sweep in (True, False):
+        pc = capi.Preconditioner(a, kind, capi.ORDER_NATURAL)
+        pc.set_sweep(sweep)
+        pc.initialize(a)
+        src = ctx.to_device(r)
+        z = ctx.zeros(a.n)
+        for _ in range(3):
+            pc.apply(z, src)
+        out.append(z.download())
     assert np.array_equal(out[0], out[1])
 
 

@@ -174,4 +174,4 @@ def test_concurrent_single_launches(kind, order, nx, ny):
     held.clear()
     for c in ctxs:
         c.close()
-    assert together < (0.75 if nx == 100 else 1.2) * alone
+    assert together < (0.85 if nx == 100 else 1.2) * alone

@@ -73,6 +73,13 @@ def test_reorder_crowded_cell(ctx, oracle, speed):
     compare(ctx, oracle, np.where(np.arange(64) == 30, 1100000, 20), speed, 2)
 
 
+def test_relocate_four_lists(ctx, oracle):
+    """a set whose buffers hold 8388608 particles or more takes four lists of leaving particles to a wave; here the
+    buffers have held 7M particles before, the lists are full, short and missing ones"""
+    print("relocate four lists", flush=True)
+    compare(ctx, oracle, [(16, 40, 3)[c % 3] for c in range(64)], 0.9, 3, held=7000000)
+
+
 def best_of(ctx, call, prepare=lambda: None):
     best = np.inf
     for _ in range(4):
