@@ -42,7 +42,8 @@ struct pfem_particles_t {
     pfem::DevArray<double2> pos[2], vel[2];
     pfem::DevArray<uint32_t> id[2];
     // per cell: occupied subcells, live particles, the refill's and the cells' prefix sums, the next free place
-    // (live and counters {deleted, -, long cells, -} lie behind mask)
+    // (live and counters {deleted, -, long cells, cells of k_proj_crowded} lie behind mask; those cells' list has the
+    // place of the cells' next free places, which only the reorder uses)
     pfem::DevArray<uint32_t> mask;
     int *live = nullptr, *counters = nullptr;
     pfem::DevArray<int> cursor, cell_start;
@@ -51,7 +52,6 @@ struct pfem_particles_t {
     // cells with more particles than a workgroup orders in LDS
     pfem::DevArray<uint32_t> order, order2;
     pfem::DevArray<int> tile_cell, long_cells, left_n;
-    pfem::DevArray<int> crowded, ncrowded;   // cells that k_proj_crowded sums
     pfem::DevArray<double> part;
     long deleted_last = 0, added_last = 0;
     // device state {count, next ID, deleted, added} of the last step, its pinned host copy and the event
@@ -1086,7 +1086,6 @@ static void alloc_state(pfem_particles_t* ph, long cap)
     ph->left_n.alloc(blocks);
     ph->tile_cell.alloc(cap / kTileOut + 2);
     ph->long_cells.alloc(cap / kLongCell + 1);
-    ph->crowded.alloc(cap / kProjMany + 1);
     ph->capacity = cap;
     ++ph->generation;
 }
@@ -1238,11 +1237,11 @@ void particles_project(pfem_particles_t* ph, double* u0, double* u1)
     pfem_mesh2d_t* m = ph->mesh;
     const int b = ph->cur;
     hipLaunchKernelGGL(k_proj_cells, dim3(blocks_for(m->nt, kProjCells)), dim3(kBlock), 0, c->stream, m->nt, ph->cell_start.p,
-                       ph->lam12[b].p, ph->lam3[b].p, ph->vel[b].p, ph->part.p, ph->crowded.p, ph->ncrowded.p);
-    hipLaunchKernelGGL(k_proj_crowded, dim3(kCrowdBlocks), dim3(64), 0, c->stream, ph->ncrowded.p, ph->crowded.p,
+                       ph->lam12[b].p, ph->lam3[b].p, ph->vel[b].p, ph->part.p, ph->cursor.p, ph->counters + 3);
+    hipLaunchKernelGGL(k_proj_crowded, dim3(kCrowdBlocks), dim3(64), 0, c->stream, ph->counters + 3, ph->cursor.p,
                        ph->cell_start.p, ph->lam12[b].p, ph->lam3[b].p, ph->vel[b].p, ph->part.p);
     hipLaunchKernelGGL(k_proj_nodes, dim3(blocks_for(m->nv)), dim3(kBlock), 0, c->stream, m->nv, m->inc.off.p,
-                       m->inc.code.p, ph->part.p, u0, u1, ph->ncrowded.p);
+                       m->inc.code.p, ph->part.p, u0, u1, ph->counters + 3);
     PFEM_HIP(hipGetLastError());
 }
 
@@ -1304,11 +1303,9 @@ int pfem_particles_create(pfem_mesh2d m, int level, pfem_particles* out)
         ph->cell_start.alloc(m->nt + 1);
         ph->part.alloc(9 * (size_t)m->nt);
         ph->pst.alloc(8);
-        ph->ncrowded.alloc(1);
         PFEM_HIP(hipHostMalloc((void**)&ph->h_pst, 4 * sizeof(long), hipHostMallocDefault));
         PFEM_HIP(hipEventCreateWithFlags(&ph->pst_ev, hipEventDisableTiming));
         zero_async(c, ph->mask.p, ph->mask.bytes());
-        zero_async(c, ph->ncrowded.p, ph->ncrowded.bytes());
         alloc_state(ph.get(), 1024);
         put_device_state(c, ph.get());
         zero_async(c, ph->cell_start.p, ph->cell_start.bytes());   // no particles: every cell's range is empty
