@@ -179,8 +179,9 @@ __device__ __forceinline__ double res_sum(const ResArgs<T>& a, const ResSys& S, 
 // REL: reliable updates (batched PFEM_PRECISION_MIXED): the iterations run in FP64 like everything here, and
 // the true residual b - A x replaces the recursive one after every fall of gamma by `drop` and for the
 // stopping test.
-// WPS waves per SIMD: 4 is one workgroup to a CU; 8 holds two (with a few registers spilled: 10% slower
-// alone), so that in a batch of more workgroups than CUs one team's waits are another's work.
+// WPS waves per SIMD: 4 is one workgroup to a CU; 8 holds two (with 6 vector and up to 16 scalar registers spilled:
+// 10% slower alone), so that in a batch of more workgroups than CUs one team's waits are another's work. With REL
+// it is 24 to 31 and 26, and a mixed batch takes 13 to 18% longer than an FP64 one (15.1 and 17.0 ms for 64 systems).
 template <typename T, int W, bool JAC, bool REL, int WPS>
 __global__ __launch_bounds__(kResLanes, WPS) void k_resident_cg(ResArgs<T> a)
 {
@@ -532,7 +533,7 @@ bool ResidentWork::plan(Context* c, std::shared_ptr<Pattern> p, const std::vecto
     err.alloc(1);
     if (!single) {
         // A halo that does not fit ends a single system's first launch; in a batch the other systems would be solved
-        // in vain, so the halos are counted first (20 to 40 us; on the host 0.9 ms for 262144 rows).
+        // in vain, so the halos are counted first (0.28 ms for 14.8M rows; on the host 0.9 ms for 262144).
         zero_async(c, err.p, sizeof(int));
         hipLaunchKernelGGL(k_resident_halo, dim3(blocks), dim3(kResLanes), 0, c->stream, nsys, sys.p, P.rowptr.p, P.col.p,
                            err.p);

@@ -11,6 +11,9 @@
 // one sum over the workgroups: (y, y) = (r, M^-1 r) is published after the forward sweep and read after the
 // backward one, so only (p, A p) is waited for.
 //
+// Rows of 9 to 12 neighbours have a variant of their own that spills 25 of those registers: 16.0, 16.7, 18.0 and 19.1 us
+// an iteration at 5k, 13k, 65k and 256k rows, against 23.4, 22.9, 21.9 and 30.8 launch by launch.
+//
 // us per iteration at 13k, 65k, 132k and 256k rows: 26.0, 25.5, 26.7 and 31.4 launch by launch, 11.4, 12.5, 12.9 and
 // 13.5 here: 0.6 for the product, about 2.5 for (p, A p), 1.2 for each of the sweeps' eight steps (0.52 of it a
 // published value's way). Looking four times as often for a value came out slower (13.8), and so did halo places on

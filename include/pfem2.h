@@ -213,7 +213,7 @@ int pfem_precond_set_sweep(pfem_precond pc, int single_pass);
 /* Polls a single-pass wait makes before it is declared failed (no counterpart in the reference; default
  * 65536, about 0.1 s). A failed wait does not hang or fault: the launch completes, and the solve or apply
  * reports PFEM_ENUMERIC and re-arms the sweep buffers. 0 fails every wait that is not satisfied at once. (Natural
- * ordering with many small levels: polls come two to three times as often, and a wait's limit grows with the
+ * ordering with many small levels: polls come about three times as often, and a wait's limit grows with the
  * number of row blocks before it.) The waits of the single-launch PCG (PFEM_SOLVER_OPT_SINGLE_LAUNCH) scale with it
  * too: a quarter of it for a Jacobi or unpreconditioned system, about 18 ms at the default, and eight
  * times it, about 0.6 s, for a batch and for IC0. */
