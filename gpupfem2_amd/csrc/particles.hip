@@ -336,8 +336,10 @@ __global__ __launch_bounds__(kBlock) void k_advect(
 }
 
 // One wave per RANGES lists of k_advect: four make full waves where few particles leave, one gives a set of
-// a few million enough waves for the chip
-template <int RANGES>
+// a few million enough waves for the chip. SPLIT waves to a list: a small set, whose waves do not fill the chip, would
+// otherwise take a list in which all particles leave 64 at a time (12.8k particles, 20 substeps of half a cell:
+// 262 -> 130 us a step, where one kernel with a particle a lane took 208).
+template <int RANGES, int SPLIT>
 __global__ __launch_bounds__(kBlock) void k_relocate(
     const long* __restrict__ pst, int substeps, double dts, int* __restrict__ cell, double2* __restrict__ lam12,
     double* __restrict__ lam3, double2* __restrict__ pos, const int* __restrict__ tri, const double4* __restrict__ invJ,
@@ -347,7 +349,7 @@ __global__ __launch_bounds__(kBlock) void k_relocate(
     const int* __restrict__ left_n, int* __restrict__ dead)
 {
     const int lane = threadIdx.x & 63;
-    const long range = ((long)blockIdx.x * kWaves + (threadIdx.x >> 6)) * RANGES;
+    const long wave = (long)blockIdx.x * kWaves + (threadIdx.x >> 6), range = wave / SPLIT * RANGES;
     const long ranges = (pst[0] + kBlock - 1) / kBlock;
     if (range >= ranges) return;
     int end[RANGES], total = 0;
@@ -356,7 +358,7 @@ __global__ __launch_bounds__(kBlock) void k_relocate(
         total += range + r < ranges ? left_n[range + r] : 0;
         end[r] = total;
     }
-    for (int t0 = 0; t0 < total; t0 += 64) {
+    for (int t0 = 64 * (int)(wave % SPLIT); t0 < total; t0 += 64 * SPLIT) {
         const int t = t0 + lane;
         int c = -1;
         uint32_t bits = 0u;
@@ -1186,15 +1188,16 @@ void particles_advect_launch(pfem_particles_t* ph, int b, const double* u0, cons
     hipLaunchKernelGGL(k_advect, per_particle, bl, 0, c->stream, pst, substeps, dts, (const int*)ph->cell[b].p,
                        ph->lam12[b].p, ph->lam3[b].p, ph->pos[b].p, m->tri.p, (const double4*)m->invJ.p, m->v3.p, u0, u1,
                        ph->level, 1.0 / ph->level, ph->mask.p, ph->live, ph->order.p, ph->order2.p, ph->left_n.p);
-    auto relocate = [&](auto kernel, int ranges) {
-        hipLaunchKernelGGL(kernel, dim3(blocks_for(cap, kBlock * kWaves * ranges)), bl, 0, c->stream, pst, substeps, dts,
+    auto relocate = [&](auto kernel, int particles) {   // of a workgroup
+        hipLaunchKernelGGL(kernel, dim3(blocks_for(cap, particles)), bl, 0, c->stream, pst, substeps, dts,
                            ph->cell[b].p, ph->lam12[b].p, ph->lam3[b].p, ph->pos[b].p, m->tri.p,
                            (const double4*)m->invJ.p, m->v3.p, m->nbr_off.p, m->nbr_idx.p, u0, u1, ph->level,
                            1.0 / ph->level, ph->mask.p, ph->live, ph->order.p, ph->order2.p, ph->left_n.p, ph->counters);
     };
-    // (256 CUs x 32 waves x 1024 particles: below, four lists a wave leave wave slots empty)
-    if (cap >= (1L << 23)) relocate(k_relocate<4>, 4);
-    else relocate(k_relocate<1>, 1);
+    // (256 CUs x 32 waves x 1024 particles: below, four lists a wave leave wave slots empty; and x 64 particles)
+    if (cap >= (1L << 23)) relocate(k_relocate<4, 1>, 4 * kWaves * kBlock);
+    else if (cap >= (1L << 19)) relocate(k_relocate<1, 1>, kWaves * kBlock);
+    else relocate(k_relocate<1, kWaves>, kBlock);
     hipLaunchKernelGGL(k_cell_tiles, dim3(tiles), bl, 0, c->stream, nt, ph->ns, ph->mask.p, ph->live, ph->prefix.p,
                        ph->tile_sums.p);
     hipLaunchKernelGGL(k_cell_top, dim3(1), bl, 0, c->stream, tiles, ph->tile_sums.p, ph->counters, ph->pst.p);
